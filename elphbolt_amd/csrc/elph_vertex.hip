@@ -2201,6 +2201,8 @@ __global__ __launch_bounds__(256) void k_pair_q_fp64(PairQArgs a) {
     }
 }
 
+#include "axis_pair.h"
+
 // ---------------------------------------------------------------------------
 // Hamiltonian / dynamical matrix assembly and the batched eigensolver
 // ---------------------------------------------------------------------------
@@ -3706,6 +3708,253 @@ int elph_selftest_mfma(int device, double *max_err) {
 // ===========================================================================
 namespace {
 
+// Kernel variant of the axis-by-axis form: bounds on nb and nbr (registers of an
+// item's U_k' row and g), in-window ranks per item.
+struct AxisTier {
+    int id = -1, nbm = 0, ranks = 1;
+};
+AxisTier axis_tier(int64_t nb, int64_t nbr) {
+    if (nb <= 8 && nbr <= 6) return {0, 8, 2};
+    if (nb <= 8 && nbr <= 24) return {1, 8, 1};
+    if (nb <= 12 && nbr <= 12) return {2, 12, 1};
+    if (nb <= 16 && nbr <= 12) return {3, 16, 1};
+    if (nb <= 16 && nbr <= 24) return {4, 16, 1};
+    if (nb <= 32 && nbr <= 24) return {5, 32, 1};
+    return {};
+}
+AxisTier axis_tier_q(int64_t nb) {
+    if (nb <= 8) return {0, 8, 2};
+    if (nb <= 12) return {1, 12, 1};
+    if (nb <= 16) return {2, 16, 1};
+    return nb <= 32 ? AxisTier{3, 32, 1} : AxisTier{};
+}
+
+// The axis-by-axis form (axis_pair.h) of one driver: its tables on the device,
+// the column tiling and the kernel variant.
+struct AxisPlan {
+    bool on = false;
+    AxisTab t;
+    int tier = 0, ranks = 1, nbm = 8, vals = 0, nb = 0;  // kernel variant; results per rank
+    DBuf<int> pe, ecell, pl_k2, line_of, line_k, line_row, line_item;
+    DBuf<unsigned short> pidx;
+    DBuf<int4> items;
+    DBuf<double2> phA, T0, T1;
+    int64_t h_state() const { return (int64_t)t.ncell * t.CPs; }                   // elements of h per state
+    int64_t f2_state() const { return (int64_t)t.nl * (2 * t.rm + 1) * t.CPs; }    // elements of F2 per state
+    size_t lds_ab() const { return axis_ab_lds(t.np, t.ncell, t.rm, t.r1m, t.N1); }
+    size_t lds_c(bool items) const {  // 4 waves
+        return 4 * (axis_wave_bytes(t.N0, axis_ystride(t.CT, nbm, nb), 64 * ranks * vals) +
+                    (items ? axis_items_bytes(t.N0, nb, ranks) : 0));
+    }
+};
+
+// How many times cheaper (in multiply-adds) the axis sums must be than the direct
+// product: the axis kernels run at a smaller share of the FP64 rate than the fused FP64
+// product, and the int8 digit product does its multiply-adds several times faster than it.
+constexpr double kAxisMarginFp64 = 2.0, kAxisMarginMixed = 6.0;
+
+// Real multiply-adds per column and state: the direct product over `rows` rows
+// and Kp cell-pair rows against the three axis sums (B and C in tiles of 16 q
+// and 4 R on the matrix cores).
+double axis_direct_cost(int64_t rows, int64_t Kp) { return 2.0 * (double)rows * (double)Kp; }
+double axis_cost(int64_t npl, int64_t nl, int64_t ncell, int64_t rm, int64_t r1m, int64_t N0, int64_t N1) {
+    auto prod = [](int64_t N, int64_t r) { return 16.0 * (double)((N / 2 + 16) / 16) * (r > 7 ? 16.0 : 8.0) * 4.0; };
+    return 4.0 * npl * ncell + (double)(npl * (2 * rm + 1)) * prod(N1, r1m) + (double)nl * prod(N0, rm);
+}
+
+// Tables of the axis-by-axis form for `n` cells (column-major, leading dimension
+// ld) on the mesh N and the driver's rows (integer triplets).  nin / nout: inner and
+// outer column index counts; vals: results per in-window rank.  nwin, wband, offs
+// (ibzk): the rows' in-window bands and output offsets, for the list of work items; null
+// where the items depend on the state.  The form is taken (x.on) when its sums cost less
+// than 1 / `margin` of the direct product's, the rows are whole mesh lines in ascending
+// order and the sizes fit its kernels.
+void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const int64_t *N, const std::vector<int> &rows,
+                int64_t nin, int64_t nout, int64_t nrot, int nb, int vals, AxisTier tier, const std::vector<int> *nwin,
+                const std::vector<int> *wband, const std::vector<int64_t> *offs, int64_t Kp, double margin, int64_t lds_max,
+                hipStream_t s) {
+    x.on = false;
+    const int64_t nwv = (int64_t)rows.size() / 3;
+    if (tier.id < 0 || nrot > 32 || N[0] > kAxisMaxN || N[1] > kAxisMaxN || N[2] > 0x7fff || n == 0 || n > 0x7fff || nwv == 0) return;
+    AxisTab &t = x.t;
+    t = AxisTab{};
+    t.N0 = (int)N[0];
+    t.N1 = (int)N[1];
+    t.N2 = (int)N[2];
+    std::vector<int> order(n);
+    std::iota(order.begin(), order.end(), 0);
+    auto R = [&](int i, int d) { return cells[i + ld * d]; };
+    std::sort(order.begin(), order.end(), [&](int a, int b) {
+        for (int d = 0; d < 3; ++d)
+            if (R(a, d) != R(b, d)) return R(a, d) < R(b, d);
+        return a < b;
+    });
+    int64_t rm = 0, r1m = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        rm = std::max<int64_t>(rm, std::llabs(R((int)i, 0)));
+        r1m = std::max<int64_t>(r1m, std::llabs(R((int)i, 1)));
+    }
+    if (rm > kAxisMaxR || r1m > kAxisMaxR) return;
+    std::vector<int> pe;
+    std::vector<unsigned short> pidx((2 * rm + 1) * (2 * r1m + 1));
+    for (int64_t i = 0; i < n; ++i) {
+        const int c = order[i];
+        if (i == 0 || R(c, 0) != R(order[i - 1], 0) || R(c, 1) != R(order[i - 1], 1)) pe.push_back((int)i);
+    }
+    const int np = (int)pe.size();
+    std::fill(pidx.begin(), pidx.end(), (unsigned short)np);
+    for (int p = 0; p < np; ++p) {
+        const int c = order[pe[p]];
+        pidx[(R(c, 0) + rm) * (2 * r1m + 1) + R(c, 1) + r1m] = (unsigned short)p;
+    }
+    pe.push_back((int)n);
+    for (int p = 0; p < np; ++p)
+        if (pe[p + 1] - pe[p] > kAxisMaxCnt) return;
+    // lines and planes of the rows; ascending mesh order is what makes a line's rows consecutive
+    std::vector<int> pl_k2, line_k, line_row;
+    for (int64_t r = 0; r < nwv; ++r) {
+        const int *k = &rows[3 * r];
+        if (r > 0) {
+            const int *o = k - 3;
+            if (std::make_tuple(k[2], k[1], k[0]) <= std::make_tuple(o[2], o[1], o[0])) return;
+        }
+        if (r == 0 || k[2] != k[-1]) pl_k2.push_back(k[2]);
+        if (r == 0 || k[2] != k[-1] || k[1] != k[-2]) {
+            line_k.push_back(k[1] | (int)(pl_k2.size() - 1) << 16);
+            line_row.push_back((int)r);
+        }
+    }
+    line_row.push_back((int)nwv);
+    const int64_t npl = (int64_t)pl_k2.size(), nl = (int64_t)line_k.size();
+    if (axis_cost(npl, nl, n, rm, r1m, N[0], N[1]) * margin > axis_direct_cost(nwv, Kp)) return;
+    std::vector<int> line_of(npl * N[1], -1);
+    for (int64_t l = 0; l < nl; ++l) line_of[(line_k[l] >> 16) * N[1] + (line_k[l] & 0xffff)] = (int)l;
+    // column tiles: whole inner ranges, as many per 16 columns as fit
+    t.spt = nin >= 16 ? 1 : (int)std::min<int64_t>(16 / nin, nout);
+    t.CT = (int)(16 * ((t.spt * nin + 15) / 16));
+    t.CPs = (int)((nout + t.spt - 1) / t.spt) * t.CT;
+    t.np = np;
+    t.ncell = (int)n;
+    t.rm = (int)rm;
+    t.r1m = (int)r1m;
+    t.npl = (int)npl;
+    t.nl = (int)nl;
+    x.tier = tier.id;
+    x.ranks = tier.ranks;
+    x.nbm = tier.nbm;
+    x.vals = vals;
+    x.nb = nb;
+    if (lds_max > 0 && (int64_t)std::max(x.lds_ab(), x.lds_c(nwin == nullptr)) > lds_max) return;
+    std::vector<int> line_item;
+    std::vector<int4> items;
+    if (nwin) {
+        if (!offs->empty() && offs->back() + (int64_t)nb * vals > 0x7fffffff) return;
+        for (int64_t l = 0; l < nl; ++l) {
+            line_item.push_back((int)items.size());
+            for (int r = line_row[l]; r < line_row[l + 1]; ++r)
+                for (int j = 0; j < (*nwin)[r]; j += x.ranks) {
+                    const int nr = std::min(x.ranks, (*nwin)[r] - j), b0 = (*wband)[(int64_t)r * nb + j];
+                    const int b1 = nr > 1 ? (*wband)[(int64_t)r * nb + j + 1] : b0;
+                    items.push_back(make_int4(r, rows[3 * r] | nr << 8, b0 | b1 << 16, (int)((*offs)[r] + (int64_t)j * vals)));
+                }
+        }
+        line_item.push_back((int)items.size());
+    }
+    auto root = [](int64_t j, int64_t m) {
+        const double a = kTwoPi * (double)fmodulo(j, m) / (double)m;
+        return make_double2(std::cos(a), std::sin(a));
+    };
+    std::vector<double2> phA(N[2] * n), T0(N[0]), T1(N[1]), T2(N[2]);
+    for (int64_t j = 0; j < N[0]; ++j) T0[j] = root(j, N[0]);
+    for (int64_t j = 0; j < N[1]; ++j) T1[j] = root(j, N[1]);
+    for (int64_t j = 0; j < N[2]; ++j) T2[j] = root(j, N[2]);
+    for (int64_t q = 0; q < N[2]; ++q)
+        for (int64_t e = 0; e < n; ++e) phA[q * n + e] = T2[fmodulo(q * R(order[e], 2), N[2])];
+    x.pe.upload(pe, s);
+    x.ecell.upload(order, s);
+    x.pidx.upload(pidx, s);
+    x.pl_k2.upload(pl_k2, s);
+    x.line_of.upload(line_of, s);
+    x.line_k.upload(line_k, s);
+    x.line_row.upload(line_row, s);
+    if (nwin) {
+        x.line_item.upload(line_item, s);
+        x.items.upload(items, s);
+    }
+    x.phA.upload(phA, s);
+    x.T0.upload(T0, s);
+    x.T1.upload(T1, s);
+    HCHECK(hipStreamSynchronize(s));  // the host vectors may go out of scope
+    t.pe = x.pe.p;
+    t.ecell = x.ecell.p;
+    t.pidx = x.pidx.p;
+    t.pl_k2 = x.pl_k2.p;
+    t.line_of = x.line_of.p;
+    t.line_k = x.line_k.p;
+    t.line_row = x.line_row.p;
+    t.line_item = x.line_item.p;
+    t.items = x.items.p;
+    t.phA = x.phA.p;
+    t.T0 = x.T0.p;
+    t.T1 = x.T1.p;
+    x.on = true;
+}
+
+// States per chunk of the axis path for nst states: h and F2 of a chunk within `cap`
+// bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
+// of 1786 states at 617 cells, 24^3: 15.0 / 10.6 / 10.2 / 10.1 / 9.9 ms at 64 MiB / 128 MiB /
+// 512 MiB / 1 GiB / 3 GB; 251 states of 16 bands, 15 branches on 20^3: 14.4 / 9.3 / 7.8 / 7.2 / 7.1).
+constexpr int64_t kAxisChunkBytes = (int64_t)1 << 30;
+int64_t axis_chunk(const AxisPlan &x, int64_t nst, int64_t cap) {
+    const int64_t per_state = (x.h_state() + x.f2_state()) * (int64_t)sizeof(double2);
+    return std::max<int64_t>(1, std::min<int64_t>(nst, cap / per_state));
+}
+
+// Rotation and stages A and B of the states s0 .. s0 + ns - 1, of the k (or q) kb0 .. kb1 - 1.
+void axis_front(const AxisPlan &x, const AxisRotArgs &r, const int *st_shift, int s0, int ns, int kb0, int kb1, double2 *F2,
+                hipStream_t s) {
+    const AxisTab &t = x.t;
+    const dim3 rg((unsigned)((t.ncell + 3) / 4), (unsigned)(kb1 - kb0));
+    auto rot = [&](auto kern) { hipLaunchKernelGGL(kern, rg, dim3(256), 0, s, t, r, s0, ns, kb0); };
+    if (r.nrot <= 8) rot(k_axis_rot<8>);
+    else if (r.nrot <= 16) rot(k_axis_rot<16>);
+    else rot(k_axis_rot<32>);
+    const int64_t per = (int64_t)t.npl * (t.CPs / 16);
+    const dim3 ag((unsigned)((ns + 7) / 8 * 8 * per));
+    auto ab = [&](auto kern) { hipLaunchKernelGGL(kern, ag, dim3(256), x.lds_ab(), s, t, r.h, st_shift, s0, ns, F2); };
+    if (t.N1 > 31) ab(k_axis_ab<2, 4>);
+    else if (t.r1m > 7) ab(k_axis_ab<1, 4>);
+    else ab(k_axis_ab<1, 2>);
+    HCHECK(hipGetLastError());
+}
+
+// Launch shape of the C kernels for nk k (or q) of up to nm states: workgroups of
+// four lines (a multiple of the XCDs, so that the same lines of every k share an L2),
+// times the ways a k's states are split where that leaves the device idle.
+struct AxisGrid {
+    int nblk, msplit;
+};
+AxisGrid axis_grid(const AxisTab &t, int64_t nk, int64_t nm, int64_t ncu) {
+    AxisGrid g;
+    g.nblk = (t.nl + 31) / 32 * 8;
+    const int64_t have = nk * ((t.nl + 3) / 4), want = 16 * std::max<int64_t>(ncu, 1);
+    g.msplit = (int)std::max<int64_t>(1, std::min<int64_t>(nm, want / have));
+    return g;
+}
+// Calls f(tiles of 16 q, K steps of 4 R0) with the forms of stage C the kernels have.
+template <typename F>
+void axis_form(const AxisTab &t, F &&f) {
+    if (t.N0 > 31) f(axis_int<2>{}, axis_int<4>{});
+    else if (t.rm > 7) f(axis_int<1>{}, axis_int<4>{});
+    else f(axis_int<1>{}, axis_int<2>{});
+}
+// The k (or q) of the states s0 .. s0 + ns - 1 (the first and last maybe in part),
+// kst[i] the first state of k i.
+void axis_range(const std::vector<int> &kst, int64_t s0, int64_t ns, int &kb0, int &kb1) {
+    kb0 = (int)(std::upper_bound(kst.begin(), kst.end(), (int)s0) - kst.begin()) - 1;
+    kb1 = (int)(std::lower_bound(kst.begin(), kst.end(), (int)(s0 + ns)) - kst.begin());
+}
+
 // Device tables of one group of IBZ k of a run (up to the k of one launch of the
 // Re contraction: 64 in FP64, 128 in mixed runs) and of their in-window
 // states (built once; kernels then run from them without host work).
@@ -3715,12 +3964,14 @@ struct IbzkGroup {
     DBuf<double> kv;            // (nkb,3) column-major
     DBuf<double2> Ukb;          // [kb][m][mp]
     DBuf<int> st_kb, st_m, st_kint;
+    DBuf<int> kst;              // [nkb + 1] first state of each k
+    std::vector<int> kst_host;
     DBuf<int64_t> st_slot;
 };
 
 // Scratch of one stream running groups (sized by ibzk_reserve).
 struct IbzkScratch {
-    DBuf<double2> gk, h, phiT, Y;
+    DBuf<double2> gk, h, phiT, Y, F2;
     DBuf<v4i> bphi, bsl;
     DBuf<double> bscale, hmax;
 };
@@ -3758,7 +4009,13 @@ struct elph_ibzk_plan {
     // (FP64) 64*grb rows per block
     bool general = false;
     int gcb = 3, grb = 2;
-    int64_t y_bytes_cap = 0;  // general path: bytes of Y per chunk of states (0: 512 MiB)
+    // axis-by-axis form of the pair stage (either precision) where ax.on; `axis`
+    // says whether runs take it
+    AxisPlan ax;
+    bool axis = false;
+    DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
+    DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
+    int64_t y_bytes_cap = 0;  // general and axis paths: bytes of Y (or h and F2) per chunk of states (0: 512 MiB, axis kAxisChunkBytes)
     int64_t CPf = 0;  // column count of the fused layout (16-rounded nb*nbr)
     ConsumerScratch cons;
 };
@@ -3789,6 +4046,74 @@ int64_t general_chunk(const elph_ibzk_plan *p, int64_t nst) {
     const int64_t per_state = p->nwv * p->CP * (int64_t)sizeof(double2);
     const int64_t cap = p->y_bytes_cap > 0 ? p->y_bytes_cap : ((int64_t)1 << 29);
     return std::max<int64_t>(1, std::min<int64_t>(nst, cap / per_state));
+}
+
+int64_t axis_chunk(const elph_ibzk_plan *p, int64_t nst) {
+    return axis_chunk(p->ax, nst, p->y_bytes_cap > 0 ? p->y_bytes_cap : kAxisChunkBytes);
+}
+
+// Axis-by-axis path, a chunk of states at a time.
+void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, IbzkScratch &sc, hipStream_t s) {
+    const elph_ctx *c = p->ctx;
+    const int64_t chunk = axis_chunk(p, gr.nst);
+    const AxisTab &t = p->ax.t;
+    AxisRotArgs r{};
+    r.g = sc.gk.p;
+    r.g_kstride = p->nb * p->nb * p->nbr * c->nwsg;
+    r.cstride = p->nb * p->nb * p->nbr;
+    r.ostride = (int)(p->nb * p->nb);
+    r.rstride = r.nrot = r.nin = r.coef_rows = (int)p->nb;
+    r.nout = (int)p->nbr;
+    r.kst = gr.kst.p;
+    r.st_u = gr.st_m.p;
+    r.coef = gr.Ukb.p;
+    r.deg = c->degq.p;
+    r.h = sc.h.p;
+    AxisKArgs K{};
+    K.kst = gr.kst.p;
+    K.st_kint = gr.st_kint.p;
+    K.st_kb = gr.st_kb.p;
+    K.st_m = gr.st_m.p;
+    K.st_slot = gr.st_slot.p;
+    K.Vkp = a.Vkp;
+    K.uT = p->uT.p;
+    K.ufT = p->ufT.p;
+    K.wT = p->wT.p;
+    K.wfT = p->wfT.p;
+    K.lp = a.lp;
+    K.lpf = a.lpf;
+    K.Ukb = a.Ukb;
+    K.nb = a.nb;
+    K.nbr = a.nbr;
+    K.mesh_ref = a.mesh_ref;
+    K.Nph0 = a.Nph0;
+    K.Nph1 = a.Nph1;
+    K.out = a.out;
+    K.nprocs = a.nprocs;
+    const size_t lds = p->ax.lds_c(false);
+    for (int64_t s0 = 0; s0 < gr.nst; s0 += chunk) {
+        const int ns = (int)std::min(chunk, gr.nst - s0);
+        int kb0, kb1;
+        axis_range(gr.kst_host, s0, ns, kb0, kb1);
+        axis_front(p->ax, r, gr.st_kint.p, (int)s0, ns, kb0, kb1, sc.F2.p, s);
+        const AxisGrid g = axis_grid(t, kb1 - kb0, (ns + kb1 - kb0 - 1) / (kb1 - kb0), c->ncu);
+        const dim3 grid((unsigned)(g.nblk * g.msplit), (unsigned)(kb1 - kb0));
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, t, K, sc.F2.p, (int)s0, ns, kb0, g.nblk, g.msplit);
+        };
+        axis_form(t, [&](auto mt, auto ks) {
+            constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+            switch (p->ax.tier) {
+                case 0: go(k_axis_pair<8, 6, 2, MT, KS, true>); break;
+                case 1: go(k_axis_pair<8, 24, 1, MT, KS, true>); break;
+                case 2: go(k_axis_pair<12, 12, 1, MT, KS, true>); break;
+                case 3: go(k_axis_pair<16, 12, 1, MT, KS, true>); break;
+                case 4: go(k_axis_pair<16, 24, 1, MT, KS, true>); break;
+                default: go(k_axis_pair<32, 24, 1, MT, KS, false>); break;
+            }
+        });
+        HCHECK(hipGetLastError());
+    }
 }
 
 // General path: Y of a chunk of states into HBM, then the epilogue.
@@ -3901,7 +4226,9 @@ void pair_launch(elph_ibzk_plan *p, const IbzkGroup &gr, IbzkScratch &sc, hipStr
     const PairArgs a = pair_args(p, gr, sc, out);
     const int CB = (int)(p->CP / 16);
     if (timed) timed_begin(c, s);
-    if (p->general) {
+    if (p->axis) {
+        axis_launch(p, gr, a, sc, s);
+    } else if (p->general) {
         general_launch(p, a, nst_batch, sc, s);
     } else {
         fused_launch(p, a, nst_batch, sc, s, CB);
@@ -4043,7 +4370,7 @@ struct GroupHost {
     std::vector<int64_t> slot;
     std::vector<double> kv;
     std::vector<double2> Ukb;
-    std::vector<int> skb, sm, ski;
+    std::vector<int> skb, sm, ski, kst;
     std::vector<int64_t> sslot;
 };
 
@@ -4094,13 +4421,14 @@ std::vector<GroupHost> ibzk_group_hosts(const elph_ibzk_plan *p, int64_t first, 
         int64_t bidx = -1, prev = -1;
         for (int64_t j = 0; j < nst; ++j) {
             const St &a = act[i0 + j];
-            if (a.ik != prev) { ++bidx; prev = a.ik; }
+            if (a.ik != prev) { ++bidx; prev = a.ik; g.kst.push_back((int)j); }
             g.skb[j] = (int)bidx;
             g.sm[j] = (int)a.m;
             for (int d = 0; d < 3; ++d) g.ski[3 * j + d] = p->kint_irr[3 * a.ik + d];
             g.sslot[j] = on_device ? a.slot : j;
             g.slot.push_back(a.slot);
         }
+        g.kst.push_back((int)nst);
         out.push_back(std::move(g));
         i0 = i1;
     }
@@ -4118,6 +4446,8 @@ void ibzk_group_upload(const GroupHost &h, IbzkGroup &g, hipStream_t s) {
     g.st_kb.upload(h.skb, s);
     g.st_m.upload(h.sm, s);
     g.st_kint.upload(h.ski, s);
+    g.kst.upload(h.kst, s);
+    g.kst_host = h.kst;
     g.st_slot.upload(h.sslot, s);
     HCHECK(hipStreamSynchronize(s));  // the host vectors may go out of scope
 }
@@ -4140,10 +4470,15 @@ void ibzk_scratch(const elph_ibzk_plan *p, IbzkScratch &sc, int64_t nkb, int64_t
     elph_ctx *c = p->ctx;
     const int64_t nb2 = p->nb * p->nb, nslices = p->nbr * c->nwsg;
     get(sc.gk, nkb * nb2 * nslices);
-    if (p->precision != ELPH_MIXED) get(sc.h, nst * p->Kp * p->CP);  // mixed: digits straight from gk
     get(sc.phiT, gk_phi_count(c));
+    if (p->precision == ELPH_MIXED) get(sc.bphi, gk_bphi_count(c));
+    if (p->axis) {
+        get(sc.h, axis_chunk(p, nst) * p->ax.h_state());
+        get(sc.F2, axis_chunk(p, nst) * p->ax.f2_state());
+        return;
+    }
+    if (p->precision != ELPH_MIXED) get(sc.h, nst * p->Kp * p->CP);  // mixed: digits straight from gk
     if (p->precision == ELPH_MIXED) {
-        get(sc.bphi, gk_bphi_count(c));
         get(sc.bscale, nst * p->CP);
         get(sc.hmax, nst * rot_digits_nz(p) * p->CP);
         get(sc.bsl, nst * p->nkc * (p->CP / 16) * 2 * kNS * 64);
@@ -4165,7 +4500,8 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
     };
     IbzkScratch probe;
     ibzk_scratch(p, probe, nkb, nst, [&](auto &buf, int64_t n) {
-        if (with_y || (void *)&buf != (void *)&probe.Y) add(buf, n);
+        const void *b = &buf;
+        if (with_y || (b != &probe.Y && !(p->axis && (b == &probe.h || b == &probe.F2)))) add(buf, n);
     });
     IbzkGroup g;
     add(g.kv, 3 * nkb);
@@ -4173,6 +4509,7 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
     add(g.st_kb, nst);
     add(g.st_m, nst);
     add(g.st_kint, 3 * nst);
+    add(g.kst, nkb + 1);
     add(g.st_slot, nst);
     return total;
 }
@@ -4182,6 +4519,7 @@ void ibzk_prep(elph_ibzk_plan *p, const IbzkGroup &g, IbzkScratch &sc, hipStream
     elph_ctx *c = p->ctx;
     const int64_t nb = p->nb, nbr = p->nbr, nb2 = nb * nb, nslices = nbr * c->nwsg;
     launch_gkRp(c, s, g.nkb, g.kv.p, sc.gk.p, nb2 * nslices, p->precision == ELPH_MIXED, sc.phiT.p, sc.bphi.p);
+    if (p->axis) return;  // the rotation is part of the axis sums
     if (p->precision == ELPH_MIXED) {
         if (g.nst > 0) {
             const dim3 grid((unsigned)g.nkb, (unsigned)(p->CP / 16), (unsigned)rot_digits_nz(p));
@@ -4288,8 +4626,8 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         p->Vkp.upload(V, s);
         // phonons on the phonon mesh: u = e / sqrt(M), omega
         const int64_t nq = ph->nwv;
-        std::vector<double2> u(nq * nbr * nbr);
-        std::vector<double> om(nq * nbr);
+        std::vector<double2> u(nq * nbr * nbr), uf_host;
+        std::vector<double> om(nq * nbr), omf_host;
         for (int64_t q = 0; q < nq; ++q)
             for (int64_t sb = 0; sb < nbr; ++sb) {
                 om[q * nbr + sb] = ph->ens[q + nq * sb];
@@ -4324,8 +4662,10 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
             std::vector<double> en(nqf * nbr), ev(2 * nqf * nbr * nbr);
             int st = elph_ph_wann(ctx, nqf, qv.data(), en.data(), ev.data(), nullptr);
             if (st != ELPH_OK) throw Error{st, ctx->err};
-            std::vector<double2> uf(nqf * nbr * nbr);
-            std::vector<double> omf(nqf * nbr);
+            std::vector<double2> &uf = uf_host;
+            uf.resize(nqf * nbr * nbr);
+            std::vector<double> &omf = omf_host;
+            omf.resize(nqf * nbr);
             for (int64_t q = 0; q < nqf; ++q)
                 for (int64_t sb = 0; sb < nbr; ++sb) {
                     omf[q * nbr + sb] = en[q + nqf * sb];
@@ -4401,6 +4741,35 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         // the int8 digits of gwann, once per context, so that runs allocate no
         // context data
         if (precision == ELPH_MIXED) ensure_gwann_digits(ctx);
+        {
+            axis_build(p->ax, ctx->rcells_q.data(), ctx->nwsq, ctx->nwsg, p->Nel, kpi, nb, nbr, nb, (int)nb, (int)nbr,
+                       axis_tier(nb, nbr), &nw, &wb, &offs, p->Kp, precision == ELPH_MIXED ? kAxisMarginMixed : kAxisMarginFp64,
+                       ctx->lds_max, s);
+            p->axis = p->ax.on;
+            if (p->ax.on) {
+                auto transposed = [&](const std::vector<double2> &v, DBuf<double2> &dst) {
+                    std::vector<double2> w(v.size());
+                    const int64_t b2 = nbr * nbr;
+                    for (size_t q = 0; q < v.size() / b2; ++q)
+                        for (int64_t sb = 0; sb < nbr; ++sb)
+                            for (int64_t sp = 0; sp < nbr; ++sp) w[q * b2 + sp * nbr + sb] = v[q * b2 + sb * nbr + sp];
+                    dst.upload(w, s);
+                    HCHECK(hipStreamSynchronize(s));
+                };
+                auto weights = [&](const std::vector<double> &v, DBuf<double> &dst) {
+                    std::vector<double> w(v.size());
+                    for (size_t i = 0; i < v.size(); ++i) w[i] = v[i] != 0.0 ? 0.5 * kG2Unit / v[i] : 0.0;
+                    dst.upload(w, s);
+                    HCHECK(hipStreamSynchronize(s));
+                };
+                transposed(u, p->uT);
+                weights(om, p->wT);
+                if (mesh_ref > 1) {
+                    transposed(uf_host, p->ufT);
+                    weights(omf_host, p->wfT);
+                }
+            }
+        }
         // IBZ data
         p->kint_irr.resize(3 * p->nirr);
         p->ens_irred.assign(el->ens_irred, el->ens_irred + p->nirr * nb);
@@ -4478,6 +4847,7 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
     if (!p || !g2_device || !counts) return ELPH_EINVAL;
     elph_ctx *c = p->ctx;
     const int64_t y_cap = p->y_bytes_cap;
+    const bool axis = p->axis;
     try {
         HCHECK(hipSetDevice(c->device));
         if (first < 1 || last > p->nirr * p->nb || last < first - 1)
@@ -4489,16 +4859,21 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         // (a general-path plan also bounds its chunk of Y by what is left)
         const int64_t nb = p->nb;
         auto need = [&](int64_t nkb) {
-            if (p->general) {
+            if (p->general || p->axis) {
                 const size_t fixed = ibzk_noalloc_bytes(p, nkb, nkb * nb, false);
-                const int64_t per = p->nwv * p->CP * (int64_t)sizeof(double2);
-                if (fixed + per + 256 > cap) return cap + 1;
-                p->y_bytes_cap = ((int64_t)(cap - fixed) - 256) / per * per;
+                const int64_t per = (p->axis ? p->ax.h_state() + p->ax.f2_state() : p->nwv * p->CP) * (int64_t)sizeof(double2);
+                if (fixed + per + 512 > cap) return cap + 1;
+                p->y_bytes_cap = ((int64_t)(cap - fixed) - 512) / per * per;
             }
             return ibzk_noalloc_bytes(p, nkb, nkb * nb, true);
         };
         int64_t KB = 64;
         while (KB > 1 && need(KB) > cap) KB = (KB + 1) / 2;
+        if (need(KB) > cap && p->axis) {  // h and F2 of one state do not fit: the direct product
+            p->axis = false;
+            KB = 64;
+            while (KB > 1 && need(KB) > cap) KB = (KB + 1) / 2;
+        }
         if (need(KB) > cap)
             throw Error{ELPH_ENOMEM, "one IBZ k of this material needs more than the " + std::to_string(cap >> 20) +
                                          " MiB scratch of the allocation-free entry point"};
@@ -4521,6 +4896,7 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         cv.take(g.st_kb, nst);
         cv.take(g.st_m, nst);
         cv.take(g.st_kint, 3 * nst);
+        cv.take(g.kst, nkb + 1);
         cv.take(g.st_slot, nst);
         HCHECK(hipEventRecord(c->ev_c, s));
         for (const GroupHost &h : hosts) {
@@ -4535,10 +4911,12 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         timing_flush(c);
     } catch (const Error &e) {
         p->y_bytes_cap = y_cap;
+        p->axis = axis;
         c->tev_used = 0;
         return ret_error(c, e);
     }
     p->y_bytes_cap = y_cap;
+    p->axis = axis;
     return ELPH_OK;
 }
 
@@ -4629,6 +5007,7 @@ struct elph_batch {
         int cb = 0, kb = 0;  // size buckets of nb*nbr and Kp
         int64_t members = 0;
         elph_batch_class_t rep{};
+        bool axis = false;  // the first member takes the axis-by-axis form (no tile choice for the others)
     };
     int device = 0;
     std::vector<hipStream_t> streams;
@@ -4662,9 +5041,12 @@ int kp_bucket(int64_t kp) {
 struct TileCand {
     bool general;
     int gcb, grb;
+    bool axis = false;
 };
 
 void apply_cand(elph_ibzk_plan *p, const TileCand &t) {
+    p->axis = t.axis && p->ax.on;
+    if (t.axis) return;
     p->general = t.general;
     p->gcb = t.gcb;
     p->grb = t.grb;
@@ -4683,6 +5065,9 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
         for (int cb = 1; cb <= 4; ++cb)
             for (int rb = 1; rb <= 2; ++rb) cands.push_back({true, cb, rb});
     }
+    // the axis-by-axis form where the sizes take it: it is not timed against the
+    // direct product, whose operand preparation lies outside the pair stage
+    if (p->ax.on) cands.assign(1, TileCand{false, 0, 0, true});
     if (!tune) cands.resize(1);
     const IbzkGroup &g = *it.groups.front();
     IbzkScratch sc;
@@ -4690,7 +5075,7 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
     TileCand bc = cands.front();
     for (const TileCand &t : cands) {
         apply_cand(p, t);
-        if (p->ctx->lds_max > 0 && (int64_t)ibzk_pair_lds(p) > p->ctx->lds_max) continue;
+        if (!p->axis && p->ctx->lds_max > 0 && (int64_t)ibzk_pair_lds(p) > p->ctx->lds_max) continue;
         ibzk_reserve(p, sc, g.nkb, g.nst);
         ibzk_enqueue(p, g, sc, st, it.out, false);  // warm-up (also builds h for this layout)
         float tmin = 1e30f;
@@ -4711,9 +5096,15 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
     apply_cand(p, bc);
     elph_batch_class_t r{};
     r.precision = p->precision;
-    r.path = bc.general ? 1 : 0;
-    r.cb = bc.general ? bc.gcb : (int)(p->CPf / 16);
-    r.rb = bc.general ? bc.grb : (mixed ? 1 : 2);
+    if (bc.axis) {
+        r.path = p->general ? 1 : 0;
+        r.cb = p->ax.t.CPs / 16;
+        r.rb = 1;
+    } else {
+        r.path = bc.general ? 1 : 0;
+        r.cb = bc.general ? bc.gcb : (int)(p->CPf / 16);
+        r.rb = bc.general ? bc.grb : (mixed ? 1 : 2);
+    }
     r.candidates = (int32_t)cands.size();
     r.cols = p->nb * p->nbr;
     r.kp = p->Kp;
@@ -4800,12 +5191,15 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
                 c.cb = std::get<1>(key);
                 c.kb = std::get<2>(key);
                 c.rep = autotune(b, it, b->streams[0], autotune_tiles != 0);
+                c.axis = it.p->axis;
                 key2cls[key] = (int)b->classes.size();
                 b->classes.push_back(c);
                 f = key2cls.find(key);
             } else {
+                // plans of the axis-by-axis form keep it; the others take the class's
+                // tile shape where one was timed, else the plan's own
                 const elph_batch_class_t &r = b->classes[f->second].rep;
-                apply_cand(it.p, {r.path == 1, r.cb, r.rb});
+                if (!it.p->ax.on && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
             }
             it.cls = f->second;
             b->classes[f->second].members += 1;
@@ -4829,7 +5223,7 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
         b->lists.clear();
         for (auto &it : b->items) {
             it.ops.clear();
-            if (it.p->general) continue;
+            if (it.p->general || it.p->axis) continue;
             elph_ibzk_plan *p = it.p;
             const FusedShape f = fused_shape(p);
             auto fl = shape2list.find(f);
@@ -4883,13 +5277,13 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
         HCHECK(hipStreamWaitEvent(b->lstream, b->fork, 0));
         std::vector<const elph_batch::Item *> order2;
         for (const auto &it : b->items)
-            if (!it.p->general) order2.push_back(&it);
+            if (!it.p->general && !it.p->axis) order2.push_back(&it);
         for (const auto &it : b->items)
-            if (it.p->general) order2.push_back(&it);
+            if (it.p->general || it.p->axis) order2.push_back(&it);
         bool general_phase = false;
         for (const elph_batch::Item *itp : order2) {
             const elph_batch::Item &it = *itp;
-            if (it.p->general && !general_phase) {
+            if ((it.p->general || it.p->axis) && !general_phase) {
                 general_phase = true;
                 for (size_t i = 0; i < b->streams.size(); ++i) HCHECK(hipEventRecord(b->prepped[i], b->streams[i]));
             }
@@ -4897,7 +5291,7 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
             IbzkScratch &ss = *b->scr[it.stream];
             for (size_t gi = 0; gi < it.groups.size(); ++gi) {
                 const IbzkGroup &g = *it.groups[gi];
-                if (it.p->general) {
+                if (it.p->general || it.p->axis) {
                     ibzk_enqueue(it.p, g, ss, st, it.out, false);
                     continue;
                 }
@@ -5050,6 +5444,9 @@ struct elph_ibzq_plan {
     DBuf<double> g2stage;
     bool general = false;  // nb^2 beyond the fused kernel: Y tiles in HBM, then the epilogue
     DBuf<double2> Y;
+    AxisPlan ax;           // axis-by-axis form where ax.on
+    DBuf<double2> F2;
+    DBuf<int> qst;         // [q of the batch + 1] first state of each
 };
 
 extern "C" {
@@ -5148,6 +5545,8 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
             T[j] = make_double2(std::cos(x), std::sin(x));
         }
         p->T.upload(T, s);
+        axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb,
+                   axis_tier_q(nb), nullptr, nullptr, nullptr, p->Kp, kAxisMarginFp64, ctx->lds_max, s);
         p->nirr_q = ph->nwv_irred;
         p->nq = ph->nwv;
         p->q_irr.assign(ph->indexlist_irred, ph->indexlist_irred + ph->nwv_irred);
@@ -5206,7 +5605,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             p->qv.upload(qv, s);
             p->gq.alloc(nqb * gblk);
             gReq_device(c, nqb, p->qv.p, p->gq.p, gblk);
-            std::vector<int> sqb(nst), sqe(3 * nst);
+            std::vector<int> sqb(nst), sqe(3 * nst), qst;
             std::vector<double2> su(nst * nbr);
             std::vector<double> som(nst);
             std::vector<int64_t> sslot(nst);
@@ -5214,7 +5613,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             for (int64_t t = 0; t < nst; ++t) {
                 int64_t sb, iq;
                 demux_state(sts[t], nbr, &sb, &iq);
-                if (iq - 1 != prev) { ++bidx; prev = iq - 1; }
+                if (iq - 1 != prev) { ++bidx; prev = iq - 1; qst.push_back((int)t); }
                 sqb[t] = (int)bidx;
                 const int64_t iqf = p->q_irr[iq - 1];  // muxed, phonon mesh
                 int64_t v[3];
@@ -5228,6 +5627,8 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 }
                 sslot[t] = on_device ? (sts[t] - first) : t;
             }
+            qst.push_back((int)nst);
+            p->qst.upload(qst, s);
             p->st_qb.upload(sqb, s);
             p->st_qe.upload(sqe, s);
             p->st_u.upload(su, s);
@@ -5240,9 +5641,9 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 hipLaunchKernelGGL(k_polar_lp, dim3((unsigned)((nst + 255) / 256)), dim3(256), 0, s, (int)nst,
                                    (int)nbr, 1, p->st_qb.p, p->Lq.p, p->st_u.p, p->st_lp.p);
             }
-            p->h.alloc(nst * p->Kp * p->CP);
+            if (!p->ax.on) p->h.alloc(nst * p->Kp * p->CP);
             const int64_t tot = nst * p->Kp * p->CP;
-            hipLaunchKernelGGL(k_rotate_hq, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, (int)nst, (int)nb,
+            if (!p->ax.on) hipLaunchKernelGGL(k_rotate_hq, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, (int)nst, (int)nb,
                                (int)nbr, (int)c->npairk, (int)p->Kp, (int)p->CP, p->gq.p, gblk, p->st_qb.p, p->st_u.p,
                                c->gpair.p, c->ginvdeg.p, p->h.p);
             p->rowmap.alloc(nst * p->nwv);
@@ -5291,6 +5692,46 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             a.Nel2 = (int)p->Nel[2];
             a.Lmul = phase_lmul(p->L);
             const bool packed = p->L <= 255 && p->Nel[0] <= 255 && p->Nel[1] <= 255 && p->Nel[2] <= 255;
+            auto axis = [&]() {
+                const AxisTab &t = p->ax.t;
+                const int64_t chunk = axis_chunk(p->ax, nst, kAxisChunkBytes);
+                p->h.alloc(chunk * p->ax.h_state());
+                p->F2.alloc(chunk * p->ax.f2_state());
+                AxisRotArgs r{};
+                r.g = p->gq.p;
+                r.g_kstride = gblk;
+                r.cstride = nb2 * nbr;
+                r.ostride = (int)nb;
+                r.rstride = (int)nb2;
+                r.nrot = (int)nbr;
+                r.kst = p->qst.p;
+                r.coef = p->st_u.p;
+                r.deg = c->degk.p;
+                r.nin = r.nout = (int)nb;
+                r.h = p->h.p;
+                for (int64_t t0 = 0; t0 < nst; t0 += chunk) {
+                    const int nc = (int)std::min(chunk, nst - t0);
+                    int qb0, qb1;
+                    axis_range(qst, t0, nc, qb0, qb1);
+                    axis_front(p->ax, r, nullptr, (int)t0, nc, qb0, qb1, p->F2.p, s);
+                    const AxisGrid ag = axis_grid(t, qb1 - qb0, (nc + qb1 - qb0 - 1) / (qb1 - qb0), c->ncu);
+                    const dim3 g((unsigned)(ag.nblk * ag.msplit), (unsigned)(qb1 - qb0));
+                    auto go = [&](auto kern) {
+                        hipLaunchKernelGGL(kern, g, dim3(256), p->ax.lds_c(true), s, t, a, p->F2.p, (int)t0, nc, qb0,
+                                           p->qst.p, ag.nblk, ag.msplit);
+                    };
+                    axis_form(t, [&](auto mt, auto ks) {
+                        constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+                        switch (p->ax.tier) {
+                            case 0: go(k_axis_pair_q<8, 2, MT, KS>); break;
+                            case 1: go(k_axis_pair_q<12, 1, MT, KS>); break;
+                            case 2: go(k_axis_pair_q<16, 1, MT, KS>); break;
+                            default: go(k_axis_pair_q<32, 1, MT, KS>); break;
+                        }
+                    });
+                    HCHECK(hipGetLastError());
+                }
+            };
             auto launch = [&](auto pk) {
                 constexpr bool PK = decltype(pk)::value;
                 if (p->general) {
@@ -5320,7 +5761,8 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                     default: throw Error{ELPH_EINVAL, "unsupported column count"};
                 }
             };
-            if (packed) launch(std::true_type{});
+            if (p->ax.on) axis();
+            else if (packed) launch(std::true_type{});
             else launch(std::false_type{});
             HCHECK(hipGetLastError());
             HCHECK(hipEventRecord(c->ev_b, s));

@@ -1,0 +1,180 @@
+"""The axis-by-axis form of the phase contraction (k_axis_rot, k_axis_ab,
+k_axis_pair, k_axis_pair_q) against the oracle where its tiles and rules can go
+wrong: every kernel variant (bands, branches), meshes with three different
+lengths, odd ones and ones beyond 31 points (two row tiles), cells beyond 7 along an
+axis (four K steps), windows that leave lines short or empty, more than one round of
+work items, polar terms, mesh_ref 2, states of a k split over calls.  Counts exact, exact zeros
+equal, |g|^2 relative above 1e-6 * max within 1e-12 (FP64: sums of at most 1e3
+terms of one sign pattern, a few hundred units of 1.1e-16 after the cancellation
+the floor allows) and 1e-5 (mixed)."""
+import types
+
+import numpy as np
+import pytest
+
+from elphbolt_amd import interactions, synth
+from elphbolt_amd.wannier import Wannier
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+FLOOR = 1e-6
+
+
+def _rel(x, ref):
+    x, ref = np.asarray(x).ravel(), np.asarray(ref).ravel()
+    sel = np.abs(ref) > FLOOR * np.abs(ref).max()
+    return float(np.max(np.abs(x[sel] - ref[sel]) / np.abs(ref[sel]))) if sel.any() else 0.0
+
+
+def _material(nb, nat, ws, mesh, biw, polar=None, mesh_ref=1, seed=5):
+    masses = [28.0855, 12.0107, 15.999, 24.305, 69.723, 74.92, 10.81, 30.97][:nat]
+    mat = synth.make_material(f"axis_nb{nb}_na{nat}", 4.36, masses, nb, ws, mesh, seed, mesh_ref=mesh_ref,
+                              bands_in_window=biw)
+    return synth.with_polar(mat, polar, seed=3) if polar else mat
+
+
+def _state(mat):
+    o = O.Wannier(mat)
+    eye = np.eye(3).ravel()  # one operation: meshes with different lengths keep no rotation
+    el = O.Electrons(o, eye, 1, mat.wvmesh, mat.enref, mat.fsthick)
+    ph = O.Phonons(o, eye, 1, mat.phmesh)
+    return o, el, ph
+
+
+def _rows(el):
+    m = np.asarray(el.wvmesh)
+    i = np.asarray(el.indexlist) - 1
+    return np.stack([i % m[0], (i // m[0]) % m[1], i // (m[0] * m[1])], 1)
+
+
+def _takes_axis(cells, el, mixed):
+    """The dispatch's rule (axis_cost, axis_direct_cost) for these sizes."""
+    m, k = np.asarray(el.wvmesh), _rows(el)
+    npl, nl = len(set(k[:, 2])), len({(a, b) for a, b in k[:, 1:]})
+    c = np.asarray(cells)
+    rm, r1m = np.abs(c[:, 0]).max(), np.abs(c[:, 1]).max()
+    npair = (len(c) + 1) // 2  # symmetric sets pair up except R = 0
+    kp = -(-2 * npair // 64) * 64
+
+    def prod(n, r):
+        return 16.0 * ((n // 2 + 16) // 16) * (16.0 if r > 7 else 8.0) * 4.0
+    cost = 4.0 * npl * len(c) + npl * (2 * rm + 1) * prod(m[1], r1m) + nl * prod(m[0], rm)
+    return cost * (6.0 if mixed else 2.0) <= 2.0 * len(k) * kp
+
+
+# name, nb, nat, ws, mesh, bands in window, polar, precision
+CASES = [
+    ("nb8_na2", 8, 2, [5, 5, 5], [14, 16, 9], 3.0, None, "fp64"),
+    ("nb8_na2_mixed", 8, 2, [5, 5, 5], [14, 16, 8], 3.0, None, "mixed"),
+    ("nb8_na2_wide", 8, 2, [4, 4, 4], [24, 7, 8], 7.5, None, "fp64"),    # more than 64 items on a line
+    ("nb7_na2_narrow", 7, 2, [5, 5, 5], [14, 16, 9], 0.4, None, "fp64"),  # short and missing lines
+    ("nb3_na1", 3, 1, [4, 4, 4], [11, 13, 10], 1.5, None, "fp64"),
+    ("nb8_na2_polar", 8, 2, [5, 5, 5], [13, 12, 9], 3.0, "sic", "fp64"),
+    ("nb5_na3", 5, 3, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
+    ("nb5_na3_polar_mixed", 5, 3, [5, 5, 5], [15, 20, 12], 2.0, "random", "mixed"),
+    ("nb11_na3", 11, 3, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
+    ("nb13_na4", 13, 4, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
+    ("nb16_na5_polar", 16, 5, [4, 4, 4], [12, 11, 8], 2.0, "random", "fp64"),
+    ("nb19_na2", 19, 2, [4, 4, 4], [12, 11, 8], 2.0, None, "fp64"),
+    ("nb26_na8", 26, 8, [4, 4, 4], [12, 11, 8], 1.0, None, "fp64"),
+    ("n0_34", 4, 2, [4, 4, 4], [34, 6, 6], 2.0, None, "fp64"),
+    ("n1_33", 4, 2, [4, 4, 4], [12, 33, 4], 2.0, None, "fp64"),
+    ("n0_62_n1_61", 2, 1, [5, 5, 5], [62, 61, 2], 1.0, None, "fp64"),
+    ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None, "fp64"),
+    ("r1_beyond_7", 4, 1, [3, 15, 3], [13, 24, 8], 2.0, None, "fp64"),
+    ("r2_long", 4, 1, [3, 3, 15], [12, 13, 24], 2.0, None, "fp64"),
+]
+
+
+@pytest.mark.parametrize("name,nb,nat,ws,mesh,biw,polar,precision", CASES, ids=[c[0] for c in CASES])
+def test_ibzk_axis(name, nb, nat, ws, mesh, biw, polar, precision):
+    mat = _material(nb, nat, ws, mesh, biw, polar)
+    o, el, ph = _state(mat)
+    assert _takes_axis(mat.rcells_q, el, precision == "mixed")
+    plan = interactions.IbzkPlan(Wannier(mat), el, ph, precision=precision)
+    # the in-window states of the first, a middle and the last k, over the first and last rows
+    act = np.abs(el.ens_irred - el.enref) <= el.fsthick
+    ks = np.nonzero(act.any(1))[0]
+    nwin = (np.abs(el.ens - el.enref) <= el.fsthick).sum(1)
+    offs = np.concatenate([[0], np.cumsum(nwin)]) * mat.nbr
+    span = min(el.nwv, 48 if nb <= 8 else 20)
+    err = 0.0
+    for ik in sorted({int(ks[0]), int(ks[len(ks) // 2]), int(ks[-1])}):
+        first, last = ik * nb + 1, (ik + 1) * nb
+        print(f"axis ibzk {name} {precision}: k {ik + 1}, {el.nwv} rows", flush=True)
+        c_g, g_g = plan.run(first, last)
+        for r0 in (0, el.nwv - span):
+            c_o, g_o, _ = O.ibzk_g2_window(o, el, ph, first, last, r0 + 1, span)
+            got = g_g[:, offs[r0]:offs[r0 + span]]
+            sel = c_o >= 0
+            assert np.array_equal(sel, c_g >= 0) and sel.any()
+            assert np.all(c_g[sel] == plan.nprocs)
+            ref = g_o[sel][:, :got.shape[1]]
+            assert np.array_equal(ref == 0.0, got[sel] == 0.0)
+            err = max(err, _rel(got[sel], ref))
+    print(f"  max rel {err:.2e}", flush=True)
+    assert err < (1e-12 if precision == "fp64" else 1e-5)
+    # the same bits whatever states share a call
+    one = plan.run(int(ks[0]) * nb + 1, int(ks[-1]) * nb + nb) if len(ks) < 40 else None
+    if one is not None:
+        assert np.array_equal(one[1][-nb:], g_g)
+
+
+def test_ibzk_axis_mesh_ref2():
+    """The oracle takes, as the phonons of the electron mesh, the given ones on
+    the phonon mesh and the library's own ph_wann off it (the phonons the plan
+    interpolates), so both sides rotate with the same eigenvectors."""
+    mat = _material(4, 2, [4, 4, 4], [14, 12, 10], 2.0, mesh_ref=2)
+    o, el, ph = _state(mat)
+    assert _takes_axis(mat.rcells_q, el, False)
+    w = Wannier(mat)
+    mesh = np.asarray(mat.wvmesh)
+    i = np.arange(int(np.prod(mesh)))
+    pts = np.stack([i % mesh[0], (i // mesh[0]) % mesh[1], i // (mesh[0] * mesh[1])], 1)
+    ens, evecs, _ = w.ph_wann(pts / mesh)
+    on = np.all(pts % 2 == 0, axis=1)
+    half, cm = pts[on] // 2, mesh // 2
+    coarse = (half[:, 2] * cm[1] + half[:, 1]) * cm[0] + half[:, 0]
+    ens[on], evecs[on] = ph.ens[coarse], ph.evecs[coarse]
+    fine = types.SimpleNamespace(wvmesh=mesh, nwv=len(pts), ens=ens, evecs=evecs, nwv_irred=len(pts),
+                                 indexlist_irred=np.arange(1, len(pts) + 1))
+    last = 8
+    c_o, g_o = O.ibzk_g2(o, el, fine, 1, 1, last)
+    c_g, g_g = interactions.IbzkPlan(w, el, ph, mesh_ref=2, precision="fp64").run(1, last)
+    assert np.array_equal(c_o, c_g) and (c_o >= 0).any()
+    act = c_o >= 0
+    assert np.array_equal(g_o[act] == 0.0, g_g[act] == 0.0)
+    assert _rel(g_g[act], g_o[act]) < 1e-12
+
+
+# name, nb, nat, ws, mesh, bands in window, polar
+CASES_Q = [
+    ("nb6_na2", 6, 2, [4, 4, 4], [12, 11, 9], 2.5, None),
+    ("nb8_na1_narrow", 8, 1, [5, 5, 5], [14, 13, 9], 0.6, None),
+    ("nb8_na1_wide", 8, 1, [4, 4, 4], [24, 7, 8], 7.5, None),
+    ("nb11_na2_polar", 11, 2, [4, 4, 4], [12, 11, 9], 2.0, "sic"),
+    ("nb14_na1", 14, 1, [4, 4, 4], [12, 11, 9], 2.0, None),
+    ("nb19_na1", 19, 1, [4, 4, 4], [12, 11, 8], 2.0, None),
+    ("n0_35_n1_33", 4, 1, [4, 4, 4], [35, 33, 2], 1.5, None),
+    ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None),
+]
+
+
+@pytest.mark.parametrize("name,nb,nat,ws,mesh,biw,polar", CASES_Q, ids=[c[0] for c in CASES_Q])
+def test_ibzq_axis(name, nb, nat, ws, mesh, biw, polar):
+    mat = _material(nb, nat, ws, mesh, biw, polar, seed=6)
+    o, el, ph = _state(mat)
+    assert _takes_axis(mat.rcells_k, el, False)
+    first = 3 * mat.nbr + 1  # past q = 0
+    last = first + (mat.nbr if nb > 8 else 2 * mat.nbr) - 1
+    print(f"axis ibzq {name}: states {first}..{last}, {el.nwv} rows", flush=True)
+    c_o, g_o = O.ibzq_g2(o, el, ph, first, last)
+    c_g, g_g = interactions.IbzqPlan(Wannier(mat), el, ph).run(first, last)
+    assert np.array_equal(c_o, c_g) and c_o.max() > 0
+    err = 0.0
+    for t, n in enumerate(c_o):
+        assert np.array_equal(g_o[t, :n] == 0.0, g_g[t, :n] == 0.0)
+        err = max(err, _rel(g_g[t, :n], g_o[t, :n]))
+    print(f"  max rel {err:.2e}", flush=True)
+    assert err < 1e-12
