@@ -579,8 +579,8 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
     unsigned short *items = reinterpret_cast<unsigned short *>(wbase + wb);
     AxisC<MT, KS> sc;
     sc.init(x, lane);
-    const int *rowmap = a.rowmap + (size_t)s_lo * a.nwv;
-    const int64_t *rowoff = a.rowoff + (size_t)s_lo * a.nwv;
+    const int *rowmap = a.rowmap + (size_t)qb * a.nwv;  // (one row set per q)
+    const int64_t *rowoff = a.rowoff + (size_t)qb * a.nwv;
     const int row0 = x.line_row[line], nrow = x.line_row[line + 1] - row0;
     int mine = 0;
     if (lane < nrow) {
@@ -687,5 +687,171 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
             for (int i = lane; i < n; i += 64) __builtin_nontemporal_store(stage[i], outrow + i);
             wave_lds_sync();
         }
+    }
+}
+
+// The same three sums at a list of mesh points, for the mixed representations
+// g(k, Rp) (cells Re) and g(Re, q) (cells Rp):
+//   out[point][column] = sum_R e^{i 2 pi k.R} gwann(R, column) / deg(R).
+// Irreducible points lie in few planes and lines (413 of 24^3: 7 planes, 49 lines),
+// so the sums over R2 and R1 are shared by many points: 5.9e4 multiply-adds per
+// column instead of 5.1e5 of the cell-pair product, which leaves the reads of gwann and the
+// writes as the larger part.  A workgroup takes 4 columns (64 bytes of a cell) of one outer
+// index: A for up to 8 planes at once (each cell is loaded once for all of them) into
+// LDS, then a lane takes one line and column, F2 of all R0 in registers (rows R0 = r - RM,
+// RM >= rm), and sums its line's points in the symmetric form.
+// Measured for 413 points, 617 cells, 237e3 columns (2.3 GB read, 1.6 GB written): 2.6 ms against
+// 10.0 ms in 7 passes of k_gkRp and 6.9 ms in 4 of k_gReq.  Its LDS reads and FP64 operations
+// bound it (without the stores 2.4 ms, without the reads beyond L2 2.5); A's phases as scalar
+// operands instead of from LDS were slower where few planes are taken (0.54 against 0.23 ms at
+// 48 points, 279 cells): every scalar load waits for all of a wave's.
+constexpr int kPtsPlanes = 8;
+struct AxisCellTab {
+    int N0 = 1, N1 = 1, N2 = 1;
+    int np = 0, ncell = 0, rm = 0, r1m = 0, r2n = 0;  // pairs, entries, largest |R0|, |R1|, distinct R2
+    const int *pe = nullptr;       // [np + 1] first entry of a pair (R0, R1)
+    const int *ent = nullptr;      // [ncell] cell | index of its R2 << 16
+    const double *dinv = nullptr;  // [ncell] 1 / degeneracy
+    const int *poff = nullptr;     // [2 r1m + 1][2 RM + 2] pair of (R0 = r - RM, R1), np where there is none
+    const double2 *T0 = nullptr, *T1 = nullptr;  // roots of unity
+};
+struct AxisPtsArgs {
+    const double2 *g;
+    int64_t cstride, ostride;  // elements between cells, and between outer indices
+    int no, nb2;               // outer indices, contiguous inner columns
+    int od;                    // output offset of outer index o: nb2 ((o / od) om + (o % od) on)
+    int64_t om, on;
+    double2 *out;
+    int64_t kstride;           // elements between points
+    int npl, nk;
+    const int *pl_line;        // [npl + 1] first line of a plane
+    const double2 *phA;        // [planes / 8][r2n][8] e^{i 2 pi k2 R2 / N2}
+    const int4 *lines;         // k1, first point, points, plane
+    const int *ks;             // [nk] points by line: k0 | position in the output << 8
+};
+__host__ __device__ inline size_t axis_pts_lds(int np, int ncell, int r2n, int N0, int N1, int npl, int nk) {
+    const int pl = npl < kPtsPlanes ? npl : kPtsPlanes;
+    return ((size_t)pl * (np + 1) * 4 + (size_t)r2n * kPtsPlanes + N0 + N1) * 16 + (size_t)ncell * 12 + (size_t)nk * 4 + 16;
+}
+template <int RM>
+__global__ __launch_bounds__(256, 2) void k_axis_pts(AxisCellTab c, AxisPtsArgs a, int nq) {
+    extern __shared__ double2 smem[];
+    // nq workgroups share the column tiles of an outer index, all on one XCD; at any time
+    // they are at neighbouring tiles, which share cache lines
+    const int nt = (a.nb2 + 3) >> 2, id = blockIdx.x, seq = id >> 3;
+    const int o = seq / nq * 8 + (id & 7), t0 = seq % nq, t1 = nt;
+    if (o >= a.no || t0 >= t1) return;
+    const int tid = threadIdx.x, col = tid & 3, slot = tid >> 2;
+    const int npl8 = min(a.npl, kPtsPlanes), prow = (c.np + 1) * 4;
+    double2 *F1 = smem, *ph2 = F1 + npl8 * prow, *T0s = ph2 + c.r2n * kPtsPlanes, *T1s = T0s + c.N0;
+    double *dinv = reinterpret_cast<double *>(T1s + c.N1);
+    int *ent = reinterpret_cast<int *>(dinv + c.ncell), *ks = ent + c.ncell;
+    for (int i = tid; i < c.N0; i += 256) T0s[i] = c.T0[i];
+    for (int i = tid; i < c.N1; i += 256) T1s[i] = c.T1[i];
+    for (int i = tid; i < c.ncell; i += 256) {
+        ent[i] = c.ent[i];
+        dinv[i] = c.dinv[i];
+    }
+    for (int i = tid; i < a.nk; i += 256) ks[i] = a.ks[i];
+    for (int i = tid; i < npl8 * 4; i += 256) F1[(i >> 2) * prow + c.np * 4 + (i & 3)] = make_double2(0.0, 0.0);
+    const dv2 *go = reinterpret_cast<const dv2 *>(a.g) + (size_t)o * a.ostride;
+    double2 *out = a.out + (size_t)a.nb2 * ((size_t)(o / a.od) * a.om + (size_t)(o % a.od) * a.on);
+    const int w1 = 2 * c.r1m + 1;
+    for (int p0 = 0; p0 < a.npl; p0 += kPtsPlanes) {
+        const int npl = min(kPtsPlanes, a.npl - p0);
+        const double2 *ph = a.phA + (size_t)(p0 / kPtsPlanes) * c.r2n * kPtsPlanes;
+        for (int i = tid; i < c.r2n * kPtsPlanes; i += 256) ph2[i] = ph[i];
+        const int l0 = a.pl_line[p0], l1 = a.pl_line[p0 + npl];
+        for (int tile = t0; tile < t1; tile += nq) {
+            __syncthreads();  // the tables are there; every wave has read the last tile's F1
+            const dv2 *gs = go + min(tile * 4 + col, a.nb2 - 1);
+            for (int P = slot; P < c.np; P += 64) {
+                const int e0 = c.pe[P], e1 = c.pe[P + 1];
+                double sx[kPtsPlanes], sy[kPtsPlanes];
+#pragma unroll
+                for (int j = 0; j < kPtsPlanes; ++j) sx[j] = sy[j] = 0.0;
+                for (int e = e0; e < e1; e += 8) {
+                    dv2 v[8];
+                    int w[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        w[i] = ent[min(e + i, e1 - 1)];
+                        v[i] = gs[(size_t)(w[i] & 0xffff) * a.cstride];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (e + i < e1) {
+                            const double d = dinv[e + i], x = v[i].x * d, y = v[i].y * d;
+                            const double2 *t = ph2 + (w[i] >> 16) * kPtsPlanes;
+#pragma unroll
+                            for (int j = 0; j < kPtsPlanes; ++j) {
+                                const double2 u = t[j];
+                                sx[j] = fma(u.x, x, sx[j]);
+                                sy[j] = fma(u.x, y, sy[j]);
+                                sx[j] = fma(-u.y, y, sx[j]);
+                                sy[j] = fma(u.y, x, sy[j]);
+                            }
+                        }
+                }
+#pragma unroll
+                for (int j = 0; j < kPtsPlanes; ++j)
+                    if (j < npl) F1[j * prow + P * 4 + col] = make_double2(sx[j], sy[j]);
+            }
+            __syncthreads();
+            const bool colok = tile * 4 + col < a.nb2;
+            for (int l = l0 + slot; l < l1; l += 64) {
+                const int4 ln = a.lines[l];
+                const double2 *f = F1 + (ln.w - p0) * prow + col;
+                double ax[2 * RM + 1], ay[2 * RM + 1];
+#pragma unroll
+                for (int r = 0; r <= 2 * RM; ++r) ax[r] = ay[r] = 0.0;
+                int x1 = c.N1 - (c.r1m * ln.x) % c.N1;  // (k1 R1) mod N1 from R1 = -r1m
+                x1 = x1 == c.N1 ? 0 : x1;
+                for (int i1 = 0; i1 < w1; ++i1) {
+                    const double2 w = T1s[x1];
+                    x1 += ln.x;
+                    x1 -= x1 >= c.N1 ? c.N1 : 0;
+                    const sc_int po = as_scalar(c.poff) + i1 * (2 * RM + 2);
+#pragma unroll
+                    for (int r = 0; r <= 2 * RM; ++r) {
+                        const double2 u = f[po[r] * 4];
+                        ax[r] = fma(w.x, u.x, ax[r]);
+                        ay[r] = fma(w.x, u.y, ay[r]);
+                        ax[r] = fma(-w.y, u.y, ax[r]);
+                        ay[r] = fma(w.y, u.x, ay[r]);
+                    }
+                }
+                // the symmetric form over R0: sums and i times the differences of +-R0
+                double px[RM + 1], py[RM + 1], mx[RM + 1], my[RM + 1];
+                px[0] = ax[RM];
+                py[0] = ay[RM];
+                mx[0] = my[0] = 0.0;
+#pragma unroll
+                for (int R = 1; R <= RM; ++R) {
+                    px[R] = ax[RM + R] + ax[RM - R];
+                    py[R] = ay[RM + R] + ay[RM - R];
+                    mx[R] = ay[RM - R] - ay[RM + R];
+                    my[R] = ax[RM + R] - ax[RM - R];
+                }
+                double2 *ol = out + tile * 4 + col;
+                for (int j = 0; j < ln.z; ++j) {
+                    const int k = ks[ln.y + j], k0 = k & 0xff;
+                    int x0 = 0;
+                    double sx = 0.0, sy = 0.0;
+#pragma unroll
+                    for (int R = 0; R <= RM; ++R) {
+                        const double2 w = T0s[x0];
+                        x0 += k0;
+                        x0 -= x0 >= c.N0 ? c.N0 : 0;
+                        sx = fma(w.x, px[R], sx);
+                        sy = fma(w.x, py[R], sy);
+                        sx = fma(w.y, mx[R], sx);
+                        sy = fma(w.y, my[R], sy);
+                    }
+                    if (colok) ol[(size_t)(k >> 8) * a.kstride] = make_double2(sx, sy);
+                }
+            }
+        }
+        __syncthreads();  // F1 is written again
     }
 }

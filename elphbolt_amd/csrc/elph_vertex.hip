@@ -3955,6 +3955,185 @@ void axis_range(const std::vector<int> &kst, int64_t s0, int64_t ns, int &kb0, i
     kb1 = (int)(std::lower_bound(kst.begin(), kst.end(), (int)(s0 + ns)) - kst.begin());
 }
 
+// One cell list on one mesh for k_axis_pts.
+struct AxisCells {
+    bool on = false;
+    int RM = 15;
+    AxisCellTab t;
+    std::vector<int> r2;  // the R2
+    DBuf<int> pe, ent, poff;
+    DBuf<double> dinv;
+    DBuf<double2> T0, T1;
+};
+double2 axis_root(int64_t j, int64_t n) {
+    const double a = kTwoPi * (double)fmodulo(j, n) / (double)n;
+    return make_double2(std::cos(a), std::sin(a));
+}
+void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n, const std::vector<int64_t> &deg,
+                      const int64_t *N, hipStream_t s) {
+    x.on = false;
+    if (n == 0 || n > 0x7fff || N[0] > 255 || N[1] > 0x7fff || N[2] > 0x7fff) return;
+    std::vector<int> order(n);
+    std::iota(order.begin(), order.end(), 0);
+    auto R = [&](int i, int d) { return cells[i + ld * d]; };
+    std::sort(order.begin(), order.end(), [&](int a, int b) {
+        for (int d = 0; d < 3; ++d)
+            if (R(a, d) != R(b, d)) return R(a, d) < R(b, d);
+        return a < b;
+    });
+    int64_t rm = 0, r1m = 0;
+    std::vector<int> r2;
+    for (int64_t i = 0; i < n; ++i) {
+        rm = std::max<int64_t>(rm, std::llabs(R((int)i, 0)));
+        r1m = std::max<int64_t>(r1m, std::llabs(R((int)i, 1)));
+        r2.push_back((int)R((int)i, 2));
+    }
+    std::sort(r2.begin(), r2.end());
+    r2.erase(std::unique(r2.begin(), r2.end()), r2.end());
+    if (rm > kAxisMaxR || r1m > kAxisMaxR || r2.size() > 128) return;
+    x.RM = rm <= 3 ? 3 : (rm <= 7 ? (int)rm : 15);
+    std::vector<int> poff((2 * r1m + 1) * (2 * x.RM + 2), -1);
+    int np = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        const int c = order[i];
+        if (i > 0 && R(c, 0) == R(order[i - 1], 0) && R(c, 1) == R(order[i - 1], 1)) {
+            if (R(c, 2) == R(order[i - 1], 2)) return;  // a cell twice
+            continue;
+        }
+        poff[(R(c, 1) + r1m) * (2 * x.RM + 2) + R(c, 0) + x.RM] = np++;
+    }
+    for (int &v : poff)
+        if (v < 0) v = np;
+    const int64_t r2n = (int64_t)r2.size();
+    std::vector<int> pe, ent(n);
+    std::vector<double> dinv(n);
+    for (int64_t i = 0; i < n; ++i) {
+        const int c = order[i];
+        if (i == 0 || R(c, 0) != R(order[i - 1], 0) || R(c, 1) != R(order[i - 1], 1)) pe.push_back((int)i);
+        ent[i] = c | (int)(std::lower_bound(r2.begin(), r2.end(), (int)R(c, 2)) - r2.begin()) << 16;
+        dinv[i] = 1.0 / (double)deg[c];
+    }
+    pe.push_back((int)n);
+    AxisCellTab &t = x.t;
+    t.N0 = (int)N[0];
+    t.N1 = (int)N[1];
+    t.N2 = (int)N[2];
+    t.np = np;
+    t.ncell = (int)n;
+    t.rm = (int)rm;
+    t.r1m = (int)r1m;
+    t.r2n = (int)r2n;
+    DBuf<double2> *T[2] = {&x.T0, &x.T1};
+    for (int d = 0; d < 2; ++d) {
+        std::vector<double2> v(N[d]);
+        for (int64_t j = 0; j < N[d]; ++j) v[j] = axis_root(j, N[d]);
+        T[d]->upload(v, s);
+        HCHECK(hipStreamSynchronize(s));
+    }
+    x.pe.upload(pe, s);
+    x.ent.upload(ent, s);
+    x.dinv.upload(dinv, s);
+    x.poff.upload(poff, s);
+    HCHECK(hipStreamSynchronize(s));
+    t.pe = x.pe.p;
+    t.ent = x.ent.p;
+    t.dinv = x.dinv.p;
+    t.poff = x.poff.p;
+    t.T0 = x.T0.p;
+    t.T1 = x.T1.p;
+    x.r2 = r2;
+    x.on = true;
+}
+
+// A list of mesh points (integer triplets) by planes and lines, for k_axis_pts.
+struct AxisPtsHost {
+    std::vector<int> pl_k2, pl_line, ks;
+    std::vector<int4> lines;
+    std::vector<double2> phA;
+};
+int64_t axis_pts_phases(const AxisCells &x, int64_t npl) { return (npl + kPtsPlanes - 1) / kPtsPlanes * kPtsPlanes * x.t.r2n; }
+AxisPtsHost axis_pts_host(const AxisCells &x, const std::vector<int> &k) {
+    AxisPtsHost h;
+    const int n = (int)k.size() / 3;
+    std::vector<int> o(n);
+    std::iota(o.begin(), o.end(), 0);
+    std::sort(o.begin(), o.end(), [&](int a, int b) {
+        return std::make_tuple(k[3 * a + 2], k[3 * a + 1], k[3 * a], a) < std::make_tuple(k[3 * b + 2], k[3 * b + 1], k[3 * b], b);
+    });
+    for (int i = 0; i < n; ++i) {
+        const int *p = &k[3 * o[i]], *q = i ? &k[3 * o[i - 1]] : nullptr;
+        const bool plane = !q || p[2] != q[2];
+        if (plane) {
+            h.pl_k2.push_back(p[2]);
+            h.pl_line.push_back((int)h.lines.size());
+        }
+        if (plane || p[1] != q[1]) h.lines.push_back(make_int4(p[1], i, 0, (int)h.pl_k2.size() - 1));
+        h.lines.back().z += 1;
+        h.ks.push_back(p[0] | o[i] << 8);
+    }
+    h.pl_line.push_back((int)h.lines.size());
+    // the lines of the planes taken together, longest first: a wave's lanes then
+    // have about as many points each
+    for (size_t p = 0; p + 1 < h.pl_line.size(); p += kPtsPlanes)
+        std::stable_sort(h.lines.begin() + h.pl_line[p],
+                         h.lines.begin() + h.pl_line[std::min(p + kPtsPlanes, h.pl_line.size() - 1)],
+                         [](const int4 &a, const int4 &b) { return a.z > b.z; });
+    h.phA.resize(axis_pts_phases(x, (int64_t)h.pl_k2.size()), make_double2(0.0, 0.0));
+    for (size_t p = 0; p < h.pl_k2.size(); ++p)
+        for (int j = 0; j < x.t.r2n; ++j)
+            h.phA[((p / kPtsPlanes) * x.t.r2n + j) * kPtsPlanes + p % kPtsPlanes] =
+                axis_root((int64_t)x.r2[j] * h.pl_k2[p], x.t.N2);
+    return h;
+}
+struct AxisPts {
+    int npl = 0, nk = 0;
+    DBuf<int> pl_line, ks;
+    DBuf<int4> lines;
+    DBuf<double2> phA;
+    void upload(const AxisPtsHost &h, hipStream_t s) {
+        npl = (int)h.pl_k2.size();
+        nk = (int)h.ks.size();
+        pl_line.upload(h.pl_line, s);
+        ks.upload(h.ks, s);
+        lines.upload(h.lines, s);
+        phA.upload(h.phA, s);
+    }
+};
+// Points of one k_axis_pts launch: their results within 2 GiB (one pass over gwann
+// serves them all), at most what the LDS list holds.
+int64_t axis_pts_max(int64_t bytes_per_point) {
+    return std::max<int64_t>(64, std::min<int64_t>(1024, ((int64_t)2 << 30) / std::max<int64_t>(1, bytes_per_point)));
+}
+size_t axis_pts_lds(const AxisCells &x, int npl, int nk) {
+    return axis_pts_lds(x.t.np, x.t.ncell, x.t.r2n, x.t.N0, x.t.N1, npl, nk);
+}
+void axis_pts_launch(const AxisCells &x, const AxisPts &p, AxisPtsArgs a, int64_t ncu, hipStream_t s) {
+    a.npl = p.npl;
+    a.nk = p.nk;
+    a.phA = p.phA.p;
+    a.pl_line = p.pl_line.p;
+    a.lines = p.lines.p;
+    a.ks = p.ks.p;
+    // workgroups per outer index: the tables a workgroup loads first serve all its
+    // column tiles, as long as the launch keeps several rounds of two workgroups per CU
+    // (48 points, 279 cells, nb 8: 4 workgroups per outer index 0.23 ms, 16 workgroups
+    // 0.25; 413 points, 617 cells: 2.6 ms with either)
+    const int64_t nt = (a.nb2 + 3) / 4;
+    const int64_t tpb = std::max<int64_t>(1, std::min<int64_t>((nt + 1) / 2, a.no * nt / (16 * std::max<int64_t>(ncu, 1))));
+    const int nq = (int)((nt + tpb - 1) / tpb);
+    const dim3 grid((unsigned)((a.no + 7) / 8 * 8 * nq));
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), axis_pts_lds(x, p.npl, p.nk), s, x.t, a, nq); };
+    switch (x.RM) {
+        case 3: go(k_axis_pts<3>); break;
+        case 4: go(k_axis_pts<4>); break;
+        case 5: go(k_axis_pts<5>); break;
+        case 6: go(k_axis_pts<6>); break;
+        case 7: go(k_axis_pts<7>); break;
+        default: go(k_axis_pts<15>); break;
+    }
+    HCHECK(hipGetLastError());
+}
+
 // Device tables of one group of IBZ k of a run (up to the k of one launch of the
 // Re contraction: 64 in FP64, 128 in mixed runs) and of their in-window
 // states (built once; kernels then run from them without host work).
@@ -3966,6 +4145,7 @@ struct IbzkGroup {
     DBuf<int> st_kb, st_m, st_kint;
     DBuf<int> kst;              // [nkb + 1] first state of each k
     std::vector<int> kst_host;
+    AxisPts pts;                // the k by planes and lines (axis form of the Re sum)
     DBuf<int64_t> st_slot;
 };
 
@@ -4014,6 +4194,7 @@ struct elph_ibzk_plan {
     AxisPlan ax;
     bool axis = false;
     DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
+    AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 runs) where kcells.on
     DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
     int64_t y_bytes_cap = 0;  // general and axis paths: bytes of Y (or h and F2) per chunk of states (0: 512 MiB, axis kAxisChunkBytes)
     int64_t CPf = 0;  // column count of the fused layout (16-rounded nb*nbr)
@@ -4370,7 +4551,7 @@ struct GroupHost {
     std::vector<int64_t> slot;
     std::vector<double> kv;
     std::vector<double2> Ukb;
-    std::vector<int> skb, sm, ski, kst;
+    std::vector<int> skb, sm, ski, kst, kint;  // kint: the k, integer triplets
     std::vector<int64_t> sslot;
 };
 
@@ -4411,6 +4592,7 @@ std::vector<GroupHost> ibzk_group_hosts(const elph_ibzk_plan *p, int64_t first, 
         g.kv.resize(3 * nkb);
         g.Ukb.resize(nkb * nb2);
         for (int64_t b = 0; b < nkb; ++b) {
+            for (int d = 0; d < 3; ++d) g.kint.push_back(p->kint_irr[3 * ks[b] + d]);
             for (int d = 0; d < 3; ++d) g.kv[b + nkb * d] = (double)p->kint_irr[3 * ks[b] + d] / (double)p->Nel[d];
             std::memcpy(&g.Ukb[b * nb2], &p->Uk_host[ks[b] * nb2], nb2 * sizeof(double2));
         }
@@ -4437,7 +4619,7 @@ std::vector<GroupHost> ibzk_group_hosts(const elph_ibzk_plan *p, int64_t first, 
 
 // Device tables of a group (buffers of `g` that are borrowed and large enough
 // are written in place); returns after the copies.
-void ibzk_group_upload(const GroupHost &h, IbzkGroup &g, hipStream_t s) {
+void ibzk_group_upload(const GroupHost &h, const AxisCells &cells, IbzkGroup &g, hipStream_t s) {
     g.nkb = h.nkb;
     g.nst = h.nst;
     g.slot = h.slot;
@@ -4448,6 +4630,8 @@ void ibzk_group_upload(const GroupHost &h, IbzkGroup &g, hipStream_t s) {
     g.st_kint.upload(h.ski, s);
     g.kst.upload(h.kst, s);
     g.kst_host = h.kst;
+    const AxisPtsHost pts = cells.on ? axis_pts_host(cells, h.kint) : AxisPtsHost{};
+    if (cells.on) g.pts.upload(pts, s);
     g.st_slot.upload(h.sslot, s);
     HCHECK(hipStreamSynchronize(s));  // the host vectors may go out of scope
 }
@@ -4455,10 +4639,13 @@ void ibzk_group_upload(const GroupHost &h, IbzkGroup &g, hipStream_t s) {
 void ibzk_groups(elph_ibzk_plan *p, int64_t first, int64_t last, bool on_device, int64_t *counts, hipStream_t s,
                  std::vector<std::unique_ptr<IbzkGroup>> &groups, bool compact = false) {
     // IBZ k per group: the k of one launch of the Re contraction
-    const int64_t KB = p->precision == ELPH_MIXED ? kGkKTMixed : kGkKT;
+    // (rows staged for the host, and the direct product's operand, bound a group at the smaller size)
+    const int64_t KB = p->kcells.on && p->axis && on_device
+                           ? axis_pts_max(p->nb * p->nb * p->nbr * p->ctx->nwsg * (int64_t)sizeof(double2))
+                           : (p->precision == ELPH_MIXED ? kGkKTMixed : kGkKT);
     for (const GroupHost &h : ibzk_group_hosts(p, first, last, on_device, counts, compact, KB)) {
         auto g = std::make_unique<IbzkGroup>();
-        ibzk_group_upload(h, *g, s);
+        ibzk_group_upload(h, p->kcells, *g, s);
         groups.push_back(std::move(g));
     }
 }
@@ -4510,6 +4697,12 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
     add(g.st_m, nst);
     add(g.st_kint, 3 * nst);
     add(g.kst, nkb + 1);
+    if (p->kcells.on) {
+        add(g.pts.pl_line, nkb + 1);
+        add(g.pts.ks, nkb);
+        add(g.pts.lines, nkb);
+        add(g.pts.phA, axis_pts_phases(p->kcells, nkb));
+    }
     add(g.st_slot, nst);
     return total;
 }
@@ -4518,7 +4711,21 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
 void ibzk_prep(elph_ibzk_plan *p, const IbzkGroup &g, IbzkScratch &sc, hipStream_t s) {
     elph_ctx *c = p->ctx;
     const int64_t nb = p->nb, nbr = p->nbr, nb2 = nb * nb, nslices = nbr * c->nwsg;
-    launch_gkRp(c, s, g.nkb, g.kv.p, sc.gk.p, nb2 * nslices, p->precision == ELPH_MIXED, sc.phiT.p, sc.bphi.p);
+    if (p->kcells.on && p->precision != ELPH_MIXED) {
+        AxisPtsArgs a{};
+        a.g = c->gwann.p;
+        a.cstride = nb2;
+        a.ostride = nb2 * c->nwsk;
+        a.no = (int)nslices;
+        a.nb2 = (int)nb2;
+        a.od = a.no;
+        a.on = 1;
+        a.out = sc.gk.p;
+        a.kstride = nb2 * nslices;
+        axis_pts_launch(p->kcells, g.pts, a, c->ncu, s);
+    } else {
+        launch_gkRp(c, s, g.nkb, g.kv.p, sc.gk.p, nb2 * nslices, p->precision == ELPH_MIXED, sc.phiT.p, sc.bphi.p);
+    }
     if (p->axis) return;  // the rotation is part of the axis sums
     if (p->precision == ELPH_MIXED) {
         if (g.nst > 0) {
@@ -4746,6 +4953,11 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
                        axis_tier(nb, nbr), &nw, &wb, &offs, p->Kp, precision == ELPH_MIXED ? kAxisMarginMixed : kAxisMarginFp64,
                        ctx->lds_max, s);
             p->axis = p->ax.on;
+            if (precision != ELPH_MIXED)
+                axis_cells_build(p->kcells, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, ctx->elwsdeg, p->Nel, s);
+            if (p->kcells.on && ctx->lds_max > 0 &&
+                (int64_t)axis_pts_lds(p->kcells, kPtsPlanes, 1024) > ctx->lds_max)
+                p->kcells.on = false;
             if (p->ax.on) {
                 auto transposed = [&](const std::vector<double2> &v, DBuf<double2> &dst) {
                     std::vector<double2> w(v.size());
@@ -4897,10 +5109,16 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         cv.take(g.st_m, nst);
         cv.take(g.st_kint, 3 * nst);
         cv.take(g.kst, nkb + 1);
+        if (p->kcells.on) {
+            cv.take(g.pts.pl_line, nkb + 1);
+            cv.take(g.pts.ks, nkb);
+            cv.take(g.pts.lines, nkb);
+            cv.take(g.pts.phA, axis_pts_phases(p->kcells, nkb));
+        }
         cv.take(g.st_slot, nst);
         HCHECK(hipEventRecord(c->ev_c, s));
         for (const GroupHost &h : hosts) {
-            ibzk_group_upload(h, g, s);  // stream-ordered after the previous group's kernels
+            ibzk_group_upload(h, p->kcells, g, s);  // stream-ordered after the previous group's kernels
             ibzk_enqueue(p, g, sc, s, g2_device, true);
         }
         HCHECK(hipEventRecord(c->ev_d, s));
@@ -5446,6 +5664,8 @@ struct elph_ibzq_plan {
     DBuf<double2> Y;
     AxisPlan ax;           // axis-by-axis form where ax.on
     DBuf<double2> F2;
+    AxisCells rcells;      // axis-by-axis form of the Rp sum where rcells.on
+    AxisPts pts;
     DBuf<int> qst;         // [q of the batch + 1] first state of each
 };
 
@@ -5547,6 +5767,9 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         p->T.upload(T, s);
         axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb,
                    axis_tier_q(nb), nullptr, nullptr, nullptr, p->Kp, kAxisMarginFp64, ctx->lds_max, s);
+        axis_cells_build(p->rcells, ctx->rcells_g.data(), ctx->nwsg, ctx->nwsg, ctx->gwsdeg, p->Nel, s);
+        if (p->rcells.on && ctx->lds_max > 0 && (int64_t)axis_pts_lds(p->rcells, kPtsPlanes, 1024) > ctx->lds_max)
+            p->rcells.on = false;
         p->nirr_q = ph->nwv_irred;
         p->nq = ph->nwv;
         p->q_irr.assign(ph->indexlist_irred, ph->indexlist_irred + ph->nwv_irred);
@@ -5579,8 +5802,9 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
         c->t_dominant_ms = 0;
         c->n_dominant = 0;
         HCHECK(hipEventRecord(c->ev_c, s));
-        const int64_t QB = 16 * kGReqNCB;  // IBZ q per gReq pass (one pass over gwann)
         const int64_t gblk = nb2 * nbr * c->nwsk;
+        // IBZ q per pass over gwann
+        const int64_t QB = p->rcells.on && p->ax.on && on_device ? axis_pts_max(gblk * (int64_t)sizeof(double2)) : 16 * kGReqNCB;
         int64_t istate = first;
         while (istate <= last) {
             // states of up to QB distinct IBZ q
@@ -5604,7 +5828,31 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             }
             p->qv.upload(qv, s);
             p->gq.alloc(nqb * gblk);
-            gReq_device(c, nqb, p->qv.p, p->gq.p, gblk);
+            if (p->rcells.on) {
+                std::vector<int> qint(3 * nqb);
+                for (int64_t b = 0; b < nqb; ++b) {
+                    int64_t v[3];
+                    demux_vector0(p->q_irr[qs[b]], v, p->Nph);
+                    for (int d = 0; d < 3; ++d) qint[3 * b + d] = (int)(v[d] * p->mesh_ref);
+                }
+                const AxisPtsHost ph = axis_pts_host(p->rcells, qint);
+                p->pts.upload(ph, s);
+                HCHECK(hipStreamSynchronize(s));  // ph goes out of scope
+                AxisPtsArgs pa{};
+                pa.g = c->gwann.p;
+                pa.cstride = nb2 * c->nwsk * nbr;
+                pa.ostride = nb2;
+                pa.no = (int)(nbr * c->nwsk);
+                pa.nb2 = (int)nb2;
+                pa.od = (int)c->nwsk;
+                pa.om = 1;
+                pa.on = nbr;
+                pa.out = p->gq.p;
+                pa.kstride = gblk;
+                axis_pts_launch(p->rcells, p->pts, pa, c->ncu, s);
+            } else {
+                gReq_device(c, nqb, p->qv.p, p->gq.p, gblk);
+            }
             std::vector<int> sqb(nst), sqe(3 * nst), qst;
             std::vector<double2> su(nst * nbr);
             std::vector<double> som(nst);
@@ -5630,6 +5878,9 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             qst.push_back((int)nst);
             p->qst.upload(qst, s);
             p->st_qb.upload(sqb, s);
+            if (p->ax.on)
+                for (int64_t b = 0; b < nqb; ++b)  // one row set per q
+                    for (int d = 0; d < 3; ++d) sqe[3 * b + d] = sqe[3 * qst[b] + d];
             p->st_qe.upload(sqe, s);
             p->st_u.upload(su, s);
             p->st_om.upload(som, s);
@@ -5646,13 +5897,15 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             if (!p->ax.on) hipLaunchKernelGGL(k_rotate_hq, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, (int)nst, (int)nb,
                                (int)nbr, (int)c->npairk, (int)p->Kp, (int)p->CP, p->gq.p, gblk, p->st_qb.p, p->st_u.p,
                                c->gpair.p, c->ginvdeg.p, p->h.p);
-            p->rowmap.alloc(nst * p->nwv);
-            p->rowoff.alloc(nst * p->nwv);
-            p->st_tot.alloc(nst);
-            hipLaunchKernelGGL(k_ibzq_rows, dim3((unsigned)((p->nwv + 255) / 256), (unsigned)nst), dim3(256), 0, s,
-                               (int)nst, (int)p->nwv, p->st_qe.p, p->kint.p, (int)p->Nel[0], (int)p->Nel[1],
+            // rows of the states (axis form: of the q, which its states share)
+            const int64_t nrm = p->ax.on ? nqb : nst;
+            p->rowmap.alloc(nrm * p->nwv);
+            p->rowoff.alloc(nrm * p->nwv);
+            p->st_tot.alloc(nrm);
+            hipLaunchKernelGGL(k_ibzq_rows, dim3((unsigned)((p->nwv + 255) / 256), (unsigned)nrm), dim3(256), 0, s,
+                               (int)nrm, (int)p->nwv, p->st_qe.p, p->kint.p, (int)p->Nel[0], (int)p->Nel[1],
                                (int)p->Nel[2], p->lut.p, p->nwin.p, p->rowmap.p, p->rowoff.p);
-            hipLaunchKernelGGL(k_scan_rows, dim3((unsigned)nst), dim3(1024), 0, s, (int)p->nwv, p->rowoff.p, p->st_tot.p);
+            hipLaunchKernelGGL(k_scan_rows, dim3((unsigned)nrm), dim3(1024), 0, s, (int)p->nwv, p->rowoff.p, p->st_tot.p);
             HCHECK(hipGetLastError());
             double *dst = g2;
             if (!on_device) {
@@ -5766,13 +6019,18 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             else launch(std::false_type{});
             HCHECK(hipGetLastError());
             HCHECK(hipEventRecord(c->ev_b, s));
-            std::vector<int64_t> tot_h(nst);
-            HCHECK(hipMemcpyAsync(tot_h.data(), p->st_tot.p, nst * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+            std::vector<int64_t> tot_h(nrm);
+            HCHECK(hipMemcpyAsync(tot_h.data(), p->st_tot.p, nrm * sizeof(int64_t), hipMemcpyDeviceToHost, s));
             HCHECK(hipStreamSynchronize(s));
             float ms = 0;
             HCHECK(hipEventElapsedTime(&ms, c->ev_a, c->ev_b));
             c->t_dominant_ms += ms;
             c->n_dominant += 1;
+            if (p->ax.on) {
+                std::vector<int64_t> per_state(nst);
+                for (int64_t t = 0; t < nst; ++t) per_state[t] = tot_h[sqb[t]];
+                tot_h.swap(per_state);
+            }
             for (int64_t t = 0; t < nst; ++t) {
                 counts[sts[t] - first] = tot_h[t];
                 if (tot_h[t] > p->stride) throw Error{ELPH_EINVAL, "ibzq count exceeds the row stride"};

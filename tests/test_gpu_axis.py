@@ -178,3 +178,30 @@ def test_ibzq_axis(name, nb, nat, ws, mesh, biw, polar):
         err = max(err, _rel(g_g[t, :n], g_o[t, :n]))
     print(f"  max rel {err:.2e}", flush=True)
     assert err < 1e-12
+
+
+@pytest.mark.parametrize("kind", ["ibzk", "ibzq"])
+def test_many_points_per_pass(kind):
+    """More IBZ points than one pass of the mesh-point sum takes (1024), more than its
+    8 planes and 64 lines at a time: a run into device rows, which takes the large
+    groups, gives the bits of runs into host rows, which take groups of 64."""
+    import torch
+    mat = _material(3, 1, [4, 4, 4], [14, 16, 9], 1.5)
+    _, el, ph = _state(mat)
+    w = Wannier(mat)
+    plan = (interactions.IbzkPlan if kind == "ibzk" else interactions.IbzqPlan)(w, el, ph)
+    assert (el.nwv_irred if kind == "ibzk" else ph.nwv_irred) > 1024
+    nst = (el if kind == "ibzk" else ph).nwv_irred * 3
+    width = plan.nprocs if kind == "ibzk" else plan.stride
+    print(f"axis {kind}: {nst} states in one call", flush=True)
+    dev = torch.zeros((nst, width), dtype=torch.float64, device="cuda")
+    counts, _ = plan.run(1, nst, out=dev)
+    for first, last in [(1, 60), (3 * 1000 + 2, 3 * 1060), (nst - 40, nst)]:
+        c, g = plan.run(first, last)
+        assert np.array_equal(c, counts[first - 1:last]) and c.max() > 0
+        got = dev[first - 1:last].cpu().numpy()
+        if kind == "ibzk":
+            assert np.array_equal(got[c >= 0], g[c >= 0])
+        else:
+            for t, n in enumerate(c):
+                assert np.array_equal(got[t, :n], g[t, :n])
