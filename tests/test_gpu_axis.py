@@ -185,7 +185,6 @@ def test_many_points_per_pass(kind):
     """More IBZ points than one pass of the mesh-point sum takes (1024), more than its
     8 planes and 64 lines at a time: a run into device rows, which takes the large
     groups, gives the bits of runs into host rows, which take groups of 64."""
-    import torch
     mat = _material(3, 1, [4, 4, 4], [14, 16, 9], 1.5)
     _, el, ph = _state(mat)
     w = Wannier(mat)
@@ -194,12 +193,13 @@ def test_many_points_per_pass(kind):
     nst = (el if kind == "ibzk" else ph).nwv_irred * 3
     width = plan.nprocs if kind == "ibzk" else plan.stride
     print(f"axis {kind}: {nst} states in one call", flush=True)
-    dev = torch.zeros((nst, width), dtype=torch.float64, device="cuda")
+    dev = w.device_buffer((nst, width))
     counts, _ = plan.run(1, nst, out=dev)
+    rows = dev.numpy()
     for first, last in [(1, 60), (3 * 1000 + 2, 3 * 1060), (nst - 40, nst)]:
         c, g = plan.run(first, last)
         assert np.array_equal(c, counts[first - 1:last]) and c.max() > 0
-        got = dev[first - 1:last].cpu().numpy()
+        got = rows[first - 1:last]
         if kind == "ibzk":
             assert np.array_equal(got[c >= 0], g[c >= 0])
         else:
