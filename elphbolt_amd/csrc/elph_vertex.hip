@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
 #include <array>
 #include <cmath>
 #include <cstdio>
@@ -4045,6 +4046,69 @@ void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n,
     x.on = true;
 }
 
+// Pinned host memory that a plan keeps for its calls.
+struct HostBuf {
+    char *p = nullptr;
+    size_t n = 0;
+    HostBuf() = default;
+    HostBuf(const HostBuf &) = delete;
+    HostBuf &operator=(const HostBuf &) = delete;
+    ~HostBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    char *get(size_t count) {
+        if (count > n) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+            n = 0;
+            if (hipHostMalloc((void **)&p, count, hipHostMallocDefault) != hipSuccess) {
+                p = nullptr;
+                throw Error{ELPH_ENOMEM, "hipHostMalloc of " + std::to_string(count) + " bytes failed"};
+            }
+            n = count;
+        }
+        return p;
+    }
+};
+
+// The small host tables of a call, packed so that one buffer and one copy carry them
+// all: a buffer and a copy of its own for each of a dozen tables took 0.08 ms of a call
+// (one k, 24^3 mesh, mixed: 0.39 -> 0.32 ms; 48 k, 12^3 mesh: 0.53 -> 0.41).  The parts become
+// views of `dev` at 256-byte offsets.
+struct TablePack {
+    DBuf<char> dev;
+    struct Part { const void *src; size_t off, bytes; };
+    std::vector<Part> parts;
+    std::vector<std::function<void(char *)>> bind;
+    size_t used = 0;
+    static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 255) & ~(size_t)255; }
+    void clear() {
+        parts.clear();
+        bind.clear();
+        used = 0;
+    }
+    template <typename T> void add(const std::vector<T> &v, DBuf<T> &dst) {
+        const size_t off = used, n = v.size();
+        parts.push_back({v.data(), off, n * sizeof(T)});
+        bind.push_back([&dst, off, n](char *p) { dst.borrow((T *)(p + off), n); });
+        used += round(n * sizeof(T));
+    }
+    // Copies the parts, whose vectors are still there, and empties the list.  With `pinned`
+    // the copy may be in flight on return: the memory is the plan's, whose calls
+    // all end with the stream drained.
+    void upload(hipStream_t s, HostBuf *pinned) {
+        std::vector<char> pageable(pinned ? 0 : used);
+        char *h = pinned ? pinned->get(used) : pageable.data();
+        for (const Part &x : parts)
+            if (x.bytes) std::memcpy(h + x.off, x.src, x.bytes);
+        dev.alloc(used);
+        HCHECK(hipMemcpyAsync(dev.p, h, used, hipMemcpyHostToDevice, s));
+        if (!pinned) HCHECK(hipStreamSynchronize(s));
+        for (auto &b : bind) b(dev.p);
+        clear();
+    }
+};
+
 // A list of mesh points (integer triplets) by planes and lines, for k_axis_pts.
 struct AxisPtsHost {
     std::vector<int> pl_k2, pl_line, ks;
@@ -4090,13 +4154,13 @@ struct AxisPts {
     DBuf<int> pl_line, ks;
     DBuf<int4> lines;
     DBuf<double2> phA;
-    void upload(const AxisPtsHost &h, hipStream_t s) {
+    void pack(const AxisPtsHost &h, TablePack &t) {
         npl = (int)h.pl_k2.size();
         nk = (int)h.ks.size();
-        pl_line.upload(h.pl_line, s);
-        ks.upload(h.ks, s);
-        lines.upload(h.lines, s);
-        phA.upload(h.phA, s);
+        t.add(h.pl_line, pl_line);
+        t.add(h.ks, ks);
+        t.add(h.lines, lines);
+        t.add(h.phA, phA);
     }
 };
 // Points of one k_axis_pts launch: their results within 2 GiB (one pass over gwann
@@ -4195,6 +4259,8 @@ struct elph_ibzk_plan {
     bool axis = false;
     DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
     AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 runs) where kcells.on
+    TablePack tables;       // the groups' tables of the running call
+    HostBuf tables_host;
     DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
     int64_t y_bytes_cap = 0;  // general and axis paths: bytes of Y (or h and F2) per chunk of states (0: 512 MiB, axis kAxisChunkBytes)
     int64_t CPf = 0;  // column count of the fused layout (16-rounded nb*nbr)
@@ -4553,6 +4619,7 @@ struct GroupHost {
     std::vector<double2> Ukb;
     std::vector<int> skb, sm, ski, kst, kint;  // kint: the k, integer triplets
     std::vector<int64_t> sslot;
+    AxisPtsHost pts;
 };
 
 // Active states of first..last (counts -1 for out-of-window states) grouped by
@@ -4617,37 +4684,50 @@ std::vector<GroupHost> ibzk_group_hosts(const elph_ibzk_plan *p, int64_t first, 
     return out;
 }
 
-// Device tables of a group (buffers of `g` that are borrowed and large enough
-// are written in place); returns after the copies.
-void ibzk_group_upload(const GroupHost &h, const AxisCells &cells, IbzkGroup &g, hipStream_t s) {
+// Adds the tables of a group to `t` (`h` must live until t.upload).
+void ibzk_group_pack(GroupHost &h, const AxisCells &cells, IbzkGroup &g, TablePack &t) {
     g.nkb = h.nkb;
     g.nst = h.nst;
     g.slot = h.slot;
-    g.kv.upload(h.kv, s);
-    g.Ukb.upload(h.Ukb, s);
-    g.st_kb.upload(h.skb, s);
-    g.st_m.upload(h.sm, s);
-    g.st_kint.upload(h.ski, s);
-    g.kst.upload(h.kst, s);
+    t.add(h.kv, g.kv);
+    t.add(h.Ukb, g.Ukb);
+    t.add(h.skb, g.st_kb);
+    t.add(h.sm, g.st_m);
+    t.add(h.ski, g.st_kint);
+    t.add(h.kst, g.kst);
     g.kst_host = h.kst;
-    const AxisPtsHost pts = cells.on ? axis_pts_host(cells, h.kint) : AxisPtsHost{};
-    if (cells.on) g.pts.upload(pts, s);
-    g.st_slot.upload(h.sslot, s);
-    HCHECK(hipStreamSynchronize(s));  // the host vectors may go out of scope
+    if (cells.on) {
+        h.pts = axis_pts_host(cells, h.kint);
+        g.pts.pack(h.pts, t);
+    }
+    t.add(h.sslot, g.st_slot);
+}
+
+// Bytes of the tables of a group of nkb IBZ k and nst states.
+size_t ibzk_group_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst) {
+    auto b = [](int64_t n, size_t size) { return TablePack::round((size_t)n * size); };
+    size_t total = b(3 * nkb, sizeof(double)) + b(nkb * p->nb * p->nb, sizeof(double2)) + 2 * b(nst, sizeof(int)) +
+                   b(3 * nst, sizeof(int)) + b(nkb + 1, sizeof(int)) + b(nst, sizeof(int64_t));
+    if (p->kcells.on)
+        total += b(nkb + 1, sizeof(int)) + b(nkb, sizeof(int)) + b(nkb, sizeof(int4)) +
+                 b(axis_pts_phases(p->kcells, nkb), sizeof(double2));
+    return total;
 }
 
 void ibzk_groups(elph_ibzk_plan *p, int64_t first, int64_t last, bool on_device, int64_t *counts, hipStream_t s,
-                 std::vector<std::unique_ptr<IbzkGroup>> &groups, bool compact = false) {
+                 std::vector<std::unique_ptr<IbzkGroup>> &groups, TablePack &tables, HostBuf *pinned, bool compact = false) {
     // IBZ k per group: the k of one launch of the Re contraction
     // (rows staged for the host, and the direct product's operand, bound a group at the smaller size)
     const int64_t KB = p->kcells.on && p->axis && on_device
                            ? axis_pts_max(p->nb * p->nb * p->nbr * p->ctx->nwsg * (int64_t)sizeof(double2))
                            : (p->precision == ELPH_MIXED ? kGkKTMixed : kGkKT);
-    for (const GroupHost &h : ibzk_group_hosts(p, first, last, on_device, counts, compact, KB)) {
-        auto g = std::make_unique<IbzkGroup>();
-        ibzk_group_upload(h, p->kcells, *g, s);
-        groups.push_back(std::move(g));
+    std::vector<GroupHost> hosts = ibzk_group_hosts(p, first, last, on_device, counts, compact, KB);
+    tables.clear();
+    for (GroupHost &h : hosts) {
+        groups.push_back(std::make_unique<IbzkGroup>());
+        ibzk_group_pack(h, p->kcells, *groups.back(), tables);
     }
+    if (!hosts.empty()) tables.upload(s, pinned);
 }
 
 // Scratch for groups of up to nkb IBZ k and nst states; get(buffer, count)
@@ -4690,20 +4770,7 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
         const void *b = &buf;
         if (with_y || (b != &probe.Y && !(p->axis && (b == &probe.h || b == &probe.F2)))) add(buf, n);
     });
-    IbzkGroup g;
-    add(g.kv, 3 * nkb);
-    add(g.Ukb, nkb * p->nb * p->nb);
-    add(g.st_kb, nst);
-    add(g.st_m, nst);
-    add(g.st_kint, 3 * nst);
-    add(g.kst, nkb + 1);
-    if (p->kcells.on) {
-        add(g.pts.pl_line, nkb + 1);
-        add(g.pts.ks, nkb);
-        add(g.pts.lines, nkb);
-        add(g.pts.phA, axis_pts_phases(p->kcells, nkb));
-    }
-    add(g.st_slot, nst);
+    total += ibzk_group_bytes(p, nkb, nst);
     return total;
 }
 
@@ -5023,7 +5090,7 @@ int elph_ibzk_plan_run(elph_ibzk_plan *p, int64_t first, int64_t last, int64_t *
         c->n_dominant = 0;
         c->tev_used = 0;
         std::vector<std::unique_ptr<IbzkGroup>> groups;
-        ibzk_groups(p, first, last, on_device != 0, counts, s, groups);
+        ibzk_groups(p, first, last, on_device != 0, counts, s, groups, p->tables, &p->tables_host);
         int64_t nkb = 1, nst = 1;
         for (auto &g : groups) {
             nkb = std::max(nkb, g->nkb);
@@ -5049,6 +5116,7 @@ int elph_ibzk_plan_run(elph_ibzk_plan *p, int64_t first, int64_t last, int64_t *
         c->t_all_ms = ms;
         timing_flush(c);
     } catch (const Error &e) {
+        (void)hipStreamSynchronize(c->stream);
         c->tev_used = 0;
         return ret_error(c, e);
     }
@@ -5093,7 +5161,7 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         c->t_dominant_ms = 0;
         c->n_dominant = 0;
         c->tev_used = 0;
-        const std::vector<GroupHost> hosts = ibzk_group_hosts(p, first, last, true, counts, false, KB);
+        std::vector<GroupHost> hosts = ibzk_group_hosts(p, first, last, true, counts, false, KB);
         int64_t nkb = 1, nst = 1;
         for (const GroupHost &h : hosts) {
             nkb = std::max(nkb, h.nkb);
@@ -5103,22 +5171,12 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         IbzkScratch sc;
         ibzk_scratch(p, sc, nkb, nst, [&cv](auto &buf, int64_t n) { cv.take(buf, (size_t)n); });
         IbzkGroup g;
-        cv.take(g.kv, 3 * nkb);
-        cv.take(g.Ukb, nkb * nb * nb);
-        cv.take(g.st_kb, nst);
-        cv.take(g.st_m, nst);
-        cv.take(g.st_kint, 3 * nst);
-        cv.take(g.kst, nkb + 1);
-        if (p->kcells.on) {
-            cv.take(g.pts.pl_line, nkb + 1);
-            cv.take(g.pts.ks, nkb);
-            cv.take(g.pts.lines, nkb);
-            cv.take(g.pts.phA, axis_pts_phases(p->kcells, nkb));
-        }
-        cv.take(g.st_slot, nst);
+        TablePack tables;
+        cv.take(tables.dev, ibzk_group_bytes(p, nkb, nst));
         HCHECK(hipEventRecord(c->ev_c, s));
-        for (const GroupHost &h : hosts) {
-            ibzk_group_upload(h, p->kcells, g, s);  // stream-ordered after the previous group's kernels
+        for (GroupHost &h : hosts) {
+            ibzk_group_pack(h, p->kcells, g, tables);
+            tables.upload(s, nullptr);  // stream-ordered after the previous group's kernels
             ibzk_enqueue(p, g, sc, s, g2_device, true);
         }
         HCHECK(hipEventRecord(c->ev_d, s));
@@ -5200,6 +5258,7 @@ struct elph_batch {
         int64_t first = 0, last = 0;
         double *out = nullptr;
         std::vector<std::unique_ptr<IbzkGroup>> groups;
+        std::unique_ptr<TablePack> tables;  // of the groups
         int stream = 0, cls = -1;
         double work = 0;
         // fused path: each group's pair operands (B digits and column scales,
@@ -5380,7 +5439,8 @@ int elph_batch_add(elph_batch *b, elph_ibzk_plan *plan, int64_t first, int64_t l
         it.first = first;
         it.last = last;
         it.out = g2_device;
-        ibzk_groups(plan, first, last, true, counts, b->streams[0], it.groups, true);
+        it.tables = std::make_unique<TablePack>();
+        ibzk_groups(plan, first, last, true, counts, b->streams[0], it.groups, *it.tables, nullptr, true);
         int64_t nst = 0;
         for (auto &g : it.groups) nst += g->nst;
         it.work = (double)nst * plan->nwv * plan->Kp * plan->nb * plan->nbr;
@@ -5666,6 +5726,8 @@ struct elph_ibzq_plan {
     DBuf<double2> F2;
     AxisCells rcells;      // axis-by-axis form of the Rp sum where rcells.on
     AxisPts pts;
+    TablePack tables;      // the tables of the running batch of q
+    HostBuf tables_host;
     DBuf<int> qst;         // [q of the batch + 1] first state of each
 };
 
@@ -5826,33 +5888,6 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 demux_vector0(p->q_irr[qs[b]], v, p->Nph);
                 for (int d = 0; d < 3; ++d) qv[b + nqb * d] = (double)v[d] / (double)p->Nph[d];
             }
-            p->qv.upload(qv, s);
-            p->gq.alloc(nqb * gblk);
-            if (p->rcells.on) {
-                std::vector<int> qint(3 * nqb);
-                for (int64_t b = 0; b < nqb; ++b) {
-                    int64_t v[3];
-                    demux_vector0(p->q_irr[qs[b]], v, p->Nph);
-                    for (int d = 0; d < 3; ++d) qint[3 * b + d] = (int)(v[d] * p->mesh_ref);
-                }
-                const AxisPtsHost ph = axis_pts_host(p->rcells, qint);
-                p->pts.upload(ph, s);
-                HCHECK(hipStreamSynchronize(s));  // ph goes out of scope
-                AxisPtsArgs pa{};
-                pa.g = c->gwann.p;
-                pa.cstride = nb2 * c->nwsk * nbr;
-                pa.ostride = nb2;
-                pa.no = (int)(nbr * c->nwsk);
-                pa.nb2 = (int)nb2;
-                pa.od = (int)c->nwsk;
-                pa.om = 1;
-                pa.on = nbr;
-                pa.out = p->gq.p;
-                pa.kstride = gblk;
-                axis_pts_launch(p->rcells, p->pts, pa, c->ncu, s);
-            } else {
-                gReq_device(c, nqb, p->qv.p, p->gq.p, gblk);
-            }
             std::vector<int> sqb(nst), sqe(3 * nst), qst;
             std::vector<double2> su(nst * nbr);
             std::vector<double> som(nst);
@@ -5876,15 +5911,47 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 sslot[t] = on_device ? (sts[t] - first) : t;
             }
             qst.push_back((int)nst);
-            p->qst.upload(qst, s);
-            p->st_qb.upload(sqb, s);
             if (p->ax.on)
                 for (int64_t b = 0; b < nqb; ++b)  // one row set per q
                     for (int d = 0; d < 3; ++d) sqe[3 * b + d] = sqe[3 * qst[b] + d];
-            p->st_qe.upload(sqe, s);
-            p->st_u.upload(su, s);
-            p->st_om.upload(som, s);
-            p->st_slot.upload(sslot, s);
+            AxisPtsHost ph;
+            if (p->rcells.on) {
+                std::vector<int> qint(3 * nqb);
+                for (int64_t b = 0; b < nqb; ++b) {
+                    int64_t v[3];
+                    demux_vector0(p->q_irr[qs[b]], v, p->Nph);
+                    for (int d = 0; d < 3; ++d) qint[3 * b + d] = (int)(v[d] * p->mesh_ref);
+                }
+                ph = axis_pts_host(p->rcells, qint);
+            }
+            TablePack &tp = p->tables;
+            tp.clear();
+            tp.add(qv, p->qv);
+            if (p->rcells.on) p->pts.pack(ph, tp);
+            tp.add(qst, p->qst);
+            tp.add(sqb, p->st_qb);
+            tp.add(sqe, p->st_qe);
+            tp.add(su, p->st_u);
+            tp.add(som, p->st_om);
+            tp.add(sslot, p->st_slot);
+            tp.upload(s, &p->tables_host);
+            p->gq.alloc(nqb * gblk);
+            if (p->rcells.on) {
+                AxisPtsArgs pa{};
+                pa.g = c->gwann.p;
+                pa.cstride = nb2 * c->nwsk * nbr;
+                pa.ostride = nb2;
+                pa.no = (int)(nbr * c->nwsk);
+                pa.nb2 = (int)nb2;
+                pa.od = (int)c->nwsk;
+                pa.om = 1;
+                pa.on = nbr;
+                pa.out = p->gq.p;
+                pa.kstride = gblk;
+                axis_pts_launch(p->rcells, p->pts, pa, c->ncu, s);
+            } else {
+                gReq_device(c, nqb, p->qv.p, p->gq.p, gblk);
+            }
             if (c->polar) {
                 p->Lq.alloc(nqb * nbr);
                 p->st_lp.alloc(nst);
@@ -6049,6 +6116,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
         HCHECK(hipEventElapsedTime(&ms, c->ev_c, c->ev_d));
         c->t_all_ms = ms;
     } catch (const Error &e) {
+        (void)hipStreamSynchronize(c->stream);
         return ret_error(c, e);
     }
     return ELPH_OK;
