@@ -348,7 +348,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Y(np, sp), g(s) += u_q(s, sp) z(sp), so nothing per sp is held.  Bands run to
 // NBM (U_k' rows padded with zeros): a guard per band would put every LDS
 // read of Y in a block of its own and expose its latency.
-// VREG: an item's U_k' rows stay in registers.
+// VREG: an item's U_k' rows stay in registers.  ULDS (nbr = NBRM): u_q of the line's q
+// is copied to LDS once for all states of the k, [sp][q0][s].  Loads from memory
+// return in order, so a wait for u loaded by the lanes themselves is a wait for the F2 of the
+// next tile, issued before it.
 struct AxisKArgs {
     const int *kst;            // [nkb + 1] first state of each k
     const int *st_kint, *st_kb, *st_m;
@@ -361,7 +364,8 @@ struct AxisKArgs {
     double *out;
     int64_t nprocs;
 };
-template <int NBM, int NBRM, int RANKS, int MT, int KS, bool VREG>
+__host__ __device__ inline size_t axis_u_bytes(int N0, int nbr) { return (size_t)N0 * nbr * nbr * 16; }
+template <int NBM, int NBRM, int RANKS, int MT, int KS, bool VREG, bool ULDS>
 __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, const double2 *__restrict__ F2, int st0, int ns,
                                                       int kb0, int nblk, int msplit) {
     extern __shared__ double2 smem[];
@@ -371,21 +375,37 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
     const int kb = kb0 + blockIdx.y;
     const int s_lo = max(a.kst[kb], st0) + (int)blockIdx.x / nblk, s_hi = min(a.kst[kb + 1], st0 + ns);
     if (s_lo >= s_hi) return;
-    const int nb = a.nb, nbr = a.nbr, N0 = x.N0;
+    const int nb = a.nb, nbr = ULDS ? NBRM : a.nbr, N0 = x.N0;
     const int k0 = a.st_kint[3 * s_lo];
     const int lk12 = x.line_k[line];
     int q1 = (lk12 & 0xffff) - a.st_kint[3 * s_lo + 1], q2 = x.pl_k2[lk12 >> 16] - a.st_kint[3 * s_lo + 2];
     q1 += q1 < 0 ? x.N1 : 0;
     q2 += q2 < 0 ? x.N2 : 0;
     const int ys = axis_ystride(x.CT, NBM, nb), npad = ys - x.CT;
-    double2 *Yw = reinterpret_cast<double2 *>(reinterpret_cast<char *>(smem) +
-                                              wave * axis_wave_bytes(N0, ys, 64 * RANKS * nbr));
+    const size_t wb = axis_wave_bytes(N0, ys, 64 * RANKS * nbr);
+    char *wbase = reinterpret_cast<char *>(smem) + wave * (wb + (ULDS ? axis_u_bytes(N0, nbr) : 0));
+    double2 *Yw = reinterpret_cast<double2 *>(wbase);
+    dv2 *Uw = reinterpret_cast<dv2 *>(wbase + wb);
+    auto phonon = [&](int q0) {  // phonon row of q, as phonon_code
+        if (q0 % a.mesh_ref == 0 && q1 % a.mesh_ref == 0 && q2 % a.mesh_ref == 0)
+            return ((q2 / a.mesh_ref) * a.Nph1 + q1 / a.mesh_ref) * a.Nph0 + q0 / a.mesh_ref;
+        return -((q2 * x.N1 + q1) * N0 + q0) - 1;
+    };
+    auto u_of = [&](int code) {
+        return reinterpret_cast<const dv2 *>(code >= 0 ? a.uT : a.ufT) + (size_t)(code >= 0 ? code : -code - 1) * nbr * nbr;
+    };
+    if constexpr (ULDS) {
+        for (int i = lane; i < N0 * NBRM * NBRM; i += 64) {
+            const int q0 = i / (NBRM * NBRM), j = i - q0 * (NBRM * NBRM), sp = j / NBRM;
+            Uw[(sp * N0 + q0) * NBRM + j - sp * NBRM] = u_of(phonon(q0))[j];
+        }
+    }
     AxisC<MT, KS> sc;
     sc.init(x, lane);
     const int it0 = x.line_item[line], nit = x.line_item[line + 1] - it0;
     const size_t lsz = (size_t)(2 * x.rm + 1) * x.CPs, ssz = (size_t)x.nl * lsz;
     const double2 *F2l = F2 + (size_t)line * lsz;
-    constexpr bool PF = NBRM <= 12;  // u of the next sp loaded ahead
+    constexpr bool PF = !ULDS && NBRM <= 12;  // u of the next sp loaded ahead
     constexpr int UM = PF ? NBRM : 3, VM = VREG ? NBM : 1;
     for (int i0 = 0; i0 < nit; i0 += 64) {
         // the lane's item
@@ -394,13 +414,8 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
         const int nr = has ? it.y >> 8 : 0;
         int q0 = (it.y & 0xff) - k0;
         q0 += q0 < 0 ? N0 : 0;
-        int code;  // phonon row of q, as phonon_code
-        if (q0 % a.mesh_ref == 0 && q1 % a.mesh_ref == 0 && q2 % a.mesh_ref == 0)
-            code = ((q2 / a.mesh_ref) * a.Nph1 + q1 / a.mesh_ref) * a.Nph0 + q0 / a.mesh_ref;
-        else
-            code = -((q2 * x.N1 + q1) * N0 + q0) - 1;
-        const dv2 *uq = reinterpret_cast<const dv2 *>(code >= 0 ? a.uT : a.ufT) +
-                        (size_t)(code >= 0 ? code : -code - 1) * nbr * nbr;
+        const int code = phonon(q0);
+        const dv2 *uq = ULDS ? Uw + q0 * NBRM : u_of(code);
         const dv2 *V0 = reinterpret_cast<const dv2 *>(a.Vkp) + ((size_t)it.x * nb + (it.z & 0xffff)) * nb;
         const dv2 *V1 = reinterpret_cast<const dv2 *>(a.Vkp) + ((size_t)it.x * nb + (it.z >> 16)) * nb;
         dv2 v[RANKS][VM];
@@ -411,6 +426,11 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
                 if constexpr (RANKS > 1) v[1][i] = i < nb ? V1[i] : dv2{0.0, 0.0};
             }
         }
+        const double *w = (code >= 0 ? a.wT : a.wfT) + (size_t)(code >= 0 ? code : -code - 1) * nbr;
+        double wr[NBRM];  // (as u: not loaded behind the next F2)
+        if constexpr (ULDS)
+#pragma unroll
+            for (int s = 0; s < NBRM; ++s) wr[s] = w[s];
         const int first = __shfl(it.w, 0), off = it.w - first;
         const int n = __shfl(off + nr * nbr, min(63, nit - i0 - 1));
         sc.load(F2l + (size_t)(s_lo - st0) * ssz);
@@ -479,7 +499,7 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
                                 add(s + 1, un[s + 1]);
                                 add(s + 2, un[s + 2]);
                             } else {
-                                const dv2 *up = uq + sp * nbr + s;
+                                const dv2 *up = uq + sp * (ULDS ? N0 * NBRM : nbr) + s;
                                 const dv2 u0 = up[0], u1 = up[1], u2 = up[2];
                                 add(s, u0);
                                 add(s + 1, u1);
@@ -521,12 +541,13 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
             }
             // |g|^2 staged over the wave's Y tile (the items' results are one
             // contiguous range of the output), then written by consecutive lanes
-            const double *w = (code >= 0 ? a.wT : a.wfT) + (size_t)(code >= 0 ? code : -code - 1) * nbr;
             double *stage = reinterpret_cast<double *>(Yw), *o = stage + off;
 #pragma unroll
             for (int s = 0; s < NBRM; s += 3)
                 if (s < nbr) {
-                    const double f[3] = {w[s], w[s + 1], w[s + 2]};
+                    double f[3];
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) f[j] = ULDS ? wr[s + j] : w[s + j];
 #pragma unroll
                     for (int k = 0; k < RANKS; ++k)
                         if (k < nr)

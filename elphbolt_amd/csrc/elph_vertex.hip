@@ -3905,6 +3905,7 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
 // bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
 // of 1786 states at 617 cells, 24^3: 15.0 / 10.6 / 10.2 / 10.1 / 9.9 ms at 64 MiB / 128 MiB /
 // 512 MiB / 1 GiB / 3 GB; 251 states of 16 bands, 15 branches on 20^3: 14.4 / 9.3 / 7.8 / 7.2 / 7.1).
+constexpr size_t kAxisUldsMax = 80 << 10;
 constexpr int64_t kAxisChunkBytes = (int64_t)1 << 30;
 int64_t axis_chunk(const AxisPlan &x, int64_t nst, int64_t cap) {
     const int64_t per_state = (x.h_state() + x.f2_state()) * (int64_t)sizeof(double2);
@@ -4337,7 +4338,11 @@ void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, Ibzk
     K.Nph1 = a.Nph1;
     K.out = a.out;
     K.nprocs = a.nprocs;
-    const size_t lds = p->ax.lds_c(false);
+    // u_q in LDS where that leaves room for two workgroups per CU
+    const size_t lds_u = p->ax.lds_c(false) + 4 * axis_u_bytes(t.N0, (int)p->nbr);
+    const bool ulds = p->ax.tier == 0 && (p->nbr == 3 || p->nbr == 6) &&
+                      lds_u <= std::min<size_t>(kAxisUldsMax, c->lds_max > 0 ? (size_t)c->lds_max : kAxisUldsMax);
+    const size_t lds = ulds ? lds_u : p->ax.lds_c(false);
     for (int64_t s0 = 0; s0 < gr.nst; s0 += chunk) {
         const int ns = (int)std::min(chunk, gr.nst - s0);
         int kb0, kb1;
@@ -4350,13 +4355,18 @@ void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, Ibzk
         };
         axis_form(t, [&](auto mt, auto ks) {
             constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+            if (ulds) {
+                if (p->nbr == 3) go(k_axis_pair<8, 3, 2, MT, KS, true, true>);
+                else go(k_axis_pair<8, 6, 2, MT, KS, true, true>);
+                return;
+            }
             switch (p->ax.tier) {
-                case 0: go(k_axis_pair<8, 6, 2, MT, KS, true>); break;
-                case 1: go(k_axis_pair<8, 24, 1, MT, KS, true>); break;
-                case 2: go(k_axis_pair<12, 12, 1, MT, KS, true>); break;
-                case 3: go(k_axis_pair<16, 12, 1, MT, KS, true>); break;
-                case 4: go(k_axis_pair<16, 24, 1, MT, KS, true>); break;
-                default: go(k_axis_pair<32, 24, 1, MT, KS, false>); break;
+                case 0: go(k_axis_pair<8, 6, 2, MT, KS, true, false>); break;
+                case 1: go(k_axis_pair<8, 24, 1, MT, KS, true, false>); break;
+                case 2: go(k_axis_pair<12, 12, 1, MT, KS, true, false>); break;
+                case 3: go(k_axis_pair<16, 12, 1, MT, KS, true, false>); break;
+                case 4: go(k_axis_pair<16, 24, 1, MT, KS, true, false>); break;
+                default: go(k_axis_pair<32, 24, 1, MT, KS, false, false>); break;
             }
         });
         HCHECK(hipGetLastError());
