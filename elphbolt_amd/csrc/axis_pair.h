@@ -32,15 +32,15 @@ __device__ __forceinline__ sc_int as_scalar(const int *p) { return (sc_int)(uint
 template <int I>
 using axis_int = std::integral_constant<int, I>;
 
-// One cell list on one mesh, its cells sorted by (R0, R1, R2) ("entries"), and the
+// One cell list on one mesh, its cells by pairs (R0, R1) and R2 ("entries"), and the
 // driver's rows by lines and planes.
 struct AxisTab {
     int N0 = 1, N1 = 1, N2 = 1;
     int np = 0;                // pairs (R0, R1)
-    int ncell = 0;             // entries
+    int ncell = 0;             // entries (a multiple of 4 per pair: entries past a pair's cells are zero)
     int rm = 0, r1m = 0;       // largest |R0|, |R1|
-    const int *pe = nullptr;           // [np + 1] first entry of a pair
-    const int *ecell = nullptr;        // [ncell] cell of an entry
+    const int *pe = nullptr;           // [np + 1] first entry of a pair, most cells first
+    const int *ecell = nullptr;        // [ncell] cell of an entry, -1 past a pair's cells
     const unsigned short *pidx = nullptr;  // [2 rm + 1][2 r1m + 1] pair of (R0, R1), np if there is none
     const double2 *phA = nullptr;      // [N2][ncell] e^{i 2 pi q2 R2 / N2}
     const double2 *T0 = nullptr, *T1 = nullptr;  // e^{i 2 pi j / N0}, e^{i 2 pi j / N1}
@@ -86,6 +86,11 @@ __global__ __launch_bounds__(256) void k_axis_rot(AxisTab x, AxisRotArgs a, int 
     const sc_int kst = as_scalar(a.kst);
     const int s_lo = max(kst[kb], st0), s_hi = min(kst[kb + 1], st0 + ns);
     const int cell = as_scalar(x.ecell)[e];
+    if (cell < 0) {
+        for (int st = s_lo; st < s_hi; ++st)
+            for (int c = lane; c < x.CPs; c += 64) a.h[((size_t)(st - st0) * x.ncell + e) * x.CPs + c] = make_double2(0.0, 0.0);
+        return;
+    }
     const double d = 1.0 / (double)as_scalar(a.deg)[cell];
     for (int c = lane; c < x.CPs; c += 64) {
         const int t = c / x.CT, jc = c - t * x.CT, j = jc / a.nin, in = jc - j * a.nin;
@@ -115,20 +120,25 @@ __global__ __launch_bounds__(256) void k_axis_rot(AxisTab x, AxisRotArgs a, int 
 }
 
 // LDS of k_axis_ab (bytes): F1 of 16 columns (and a zero row), the plane's A
-// phases, the pair table and the lines of q1.
+// phases, the pair table, the lines of q1 and the pairs' first entries.
 __host__ __device__ inline size_t axis_ab_lds(int np, int ncell, int rm, int r1m, int N1) {
     return ((size_t)(np + 1) * 16 + ncell) * 16 + (((size_t)(2 * rm + 1) * (2 * r1m + 1) * 2 + 15) & ~(size_t)15) +
-           (size_t)N1 * 4;
+           (size_t)(N1 + np + 1) * 4;
 }
 
 // A and B for 16 columns (tile ct) of one state and plane.  A: a thread sums the
-// cells of one (R0, R1) of one column, 8 loads in flight; F1 stays in LDS.  B: a wave takes
+// cells of one (R0, R1) of one column, four at a time, the next four (of this pair or its next
+// one) already in flight; pairs with as many cells share a wave, and the zero entries that
+// fill up the fours spare it every check.  F1 stays in LDS.  B: a wave takes
 // +-R0; with E and D the sum and i times the difference of the rows of R0 and -R0, their
 // sums and differences over +-R1 are the operands of the four products that give the
-// rows F+ and F- of stage C (row R0 and rm + R0 of F2, lines q1 and N1 - q1).  MT: tiles of 16 q1,
-// 4 KS > r1m.
+// rows F+ and F- of stage C (row R0 and rm + R0 of F2, lines q1 and N1 - q1).  F2 goes past the
+// L2, which keeps the states' h for their planes and tiles.  MT: tiles of 16 q1, 4 KS > r1m.
+// The write of F2 bounds it (617 cells, 24^3, 1786 states: 10.3 GB in 2.15 ms, the rate of a
+// large copy); with F2 through the L2 3.4 ms, with a check per entry instead of the zero entries 3.3
+// and 3.6.
 template <int MT, int KS>
-__global__ __launch_bounds__(256) void k_axis_ab(AxisTab x, const double2 *__restrict__ h, const int *__restrict__ st_shift,
+__global__ __launch_bounds__(256, MT * KS > 2 ? 1 : 3) void k_axis_ab(AxisTab x, const double2 *__restrict__ h, const int *__restrict__ st_shift,
                                                  int st0, int ns, double2 *__restrict__ F2) {
     extern __shared__ double2 smem[];
     // the states' workgroups by XCD (workgroups go to the XCDs in turn), so that an
@@ -142,7 +152,7 @@ __global__ __launch_bounds__(256) void k_axis_ab(AxisTab x, const double2 *__res
     double2 *F1 = smem, *ph = smem + (x.np + 1) * 16;
     unsigned short *pidx = reinterpret_cast<unsigned short *>(ph + x.ncell);
     const int w1 = 2 * x.r1m + 1, npx = (2 * x.rm + 1) * w1;
-    int *lineq = reinterpret_cast<int *>(pidx + ((npx + 7) & ~7));
+    int *lineq = reinterpret_cast<int *>(pidx + ((npx + 7) & ~7)), *pe = lineq + x.N1;
     int k1 = 0, k2 = 0;
     if (st_shift) {
         k1 = st_shift[3 * st + 1];
@@ -153,6 +163,7 @@ __global__ __launch_bounds__(256) void k_axis_ab(AxisTab x, const double2 *__res
     const double2 *pa = x.phA + (size_t)q2 * x.ncell;
     for (int i = tid; i < x.ncell; i += 256) ph[i] = pa[i];
     for (int i = tid; i < npx; i += 256) pidx[i] = x.pidx[i];
+    for (int i = tid; i <= x.np; i += 256) pe[i] = x.pe[i];
     for (int i = tid; i < x.N1; i += 256) {
         const int k = i + k1;
         lineq[i] = x.line_of[pl * x.N1 + (k >= x.N1 ? k - x.N1 : k)];
@@ -170,31 +181,53 @@ __global__ __launch_bounds__(256) void k_axis_ab(AxisTab x, const double2 *__res
         }
     __syncthreads();
     {
-        const dv2 *hs = reinterpret_cast<const dv2 *>(h) + (size_t)stl * x.ncell * x.CPs + ct * 16;
         const int col = tid & 15;
-        for (int P = tid >> 4; P < x.np; P += 16) {
-            const int e0 = x.pe[P], e1 = x.pe[P + 1];
+        const dv2 *hs = reinterpret_cast<const dv2 *>(h) + (size_t)stl * x.ncell * x.CPs + ct * 16 + col;
+        auto load = [&](int e, dv2 (&v)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = hs[(unsigned)((e + i) * x.CPs)];
+        };
+        int P = tid >> 4;
+        if (P < x.np) {
+            int e = pe[P], e1 = pe[P + 1];
+            dv2 v[4];
+            load(e, v);
             double sx = 0.0, sy = 0.0;
-            for (int e = e0; e < e1; e += 8) {
-                dv2 v[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = hs[(unsigned)(min(e + i, e1 - 1) * x.CPs + col)];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const double2 w = ph[min(e + i, e1 - 1)];
-                    const double wx = e + i < e1 ? w.x : 0.0, wy = e + i < e1 ? w.y : 0.0;
-                    sx = fma(wx, v[i].x, sx);
-                    sy = fma(wx, v[i].y, sy);
-                    sx = fma(-wy, v[i].y, sx);
-                    sy = fma(wy, v[i].x, sy);
+            while (true) {
+                const int Pn = e + 4 < e1 ? P : P + 16;
+                int en = e + 4, en1 = e1;
+                if (Pn != P) {
+                    const int Pc = min(Pn, x.np - 1);
+                    en = pe[Pc];
+                    en1 = pe[Pc + 1];
                 }
+                dv2 vn[4];
+                load(en, vn);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const double2 w = ph[e + i];
+                    sx = fma(w.x, v[i].x, sx);
+                    sy = fma(w.x, v[i].y, sy);
+                    sx = fma(-w.y, v[i].y, sx);
+                    sy = fma(w.y, v[i].x, sy);
+                }
+                if (Pn != P) {
+                    F1[P * 16 + col] = make_double2(sx, sy);
+                    sx = sy = 0.0;
+                    if (Pn >= x.np) break;
+                }
+                P = Pn;
+                e = en;
+                e1 = en1;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = vn[i];
             }
-            F1[P * 16 + col] = make_double2(sx, sy);
         }
     }
     __syncthreads();
     double2 *F2s = F2 + (size_t)stl * x.nl * (2 * x.rm + 1) * x.CPs + ct * 16 + li;
     const size_t lstride = (size_t)(2 * x.rm + 1) * x.CPs;
+    auto put = [](double2 *o, dv2 v) { __builtin_nontemporal_store(v, reinterpret_cast<dv2 *>(o)); };
     for (int R = wave; R <= x.rm; R += 4) {
         d4 ecr[MT], eci[MT], esr[MT], esi[MT], dcr[MT], dci[MT], dsr[MT], dsi[MT];
 #pragma unroll
@@ -245,13 +278,13 @@ __global__ __launch_bounds__(256) void k_axis_ab(AxisTab x, const double2 *__res
                 const int la = lineq[q], lb = q > 0 && 2 * q < x.N1 ? lineq[x.N1 - q] : -1;
                 if (la >= 0) {
                     double2 *o = F2s + la * lstride;
-                    o[R * x.CPs] = make_double2(ecr[mt][r] + esr[mt][r], eci[mt][r] + esi[mt][r]);
-                    if (R > 0) o[(x.rm + R) * x.CPs] = make_double2(dcr[mt][r] + dsr[mt][r], dci[mt][r] + dsi[mt][r]);
+                    put(o + R * x.CPs, dv2{ecr[mt][r] + esr[mt][r], eci[mt][r] + esi[mt][r]});
+                    if (R > 0) put(o + (x.rm + R) * x.CPs, dv2{dcr[mt][r] + dsr[mt][r], dci[mt][r] + dsi[mt][r]});
                 }
                 if (lb >= 0) {
                     double2 *o = F2s + lb * lstride;
-                    o[R * x.CPs] = make_double2(ecr[mt][r] - esr[mt][r], eci[mt][r] - esi[mt][r]);
-                    if (R > 0) o[(x.rm + R) * x.CPs] = make_double2(dcr[mt][r] - dsr[mt][r], dci[mt][r] - dsi[mt][r]);
+                    put(o + R * x.CPs, dv2{ecr[mt][r] - esr[mt][r], eci[mt][r] - esi[mt][r]});
+                    if (R > 0) put(o + (x.rm + R) * x.CPs, dv2{dcr[mt][r] - dsr[mt][r], dci[mt][r] - dsi[mt][r]});
                 }
             }
     }
@@ -298,8 +331,8 @@ struct AxisC {
         const dv2 *p = reinterpret_cast<const dv2 *>(F2l);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            bc[ks] = p[oc[ks]];
-            bs[ks] = p[os[ks]];
+            bc[ks] = __builtin_nontemporal_load(p + oc[ks]);
+            bs[ks] = __builtin_nontemporal_load(p + os[ks]);
         }
     }
     // forms the tile from the loaded operands, then loads those of `next`

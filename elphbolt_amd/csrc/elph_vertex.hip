@@ -3782,35 +3782,34 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     t.N0 = (int)N[0];
     t.N1 = (int)N[1];
     t.N2 = (int)N[2];
-    std::vector<int> order(n);
-    std::iota(order.begin(), order.end(), 0);
     auto R = [&](int i, int d) { return cells[i + ld * d]; };
-    std::sort(order.begin(), order.end(), [&](int a, int b) {
-        for (int d = 0; d < 3; ++d)
-            if (R(a, d) != R(b, d)) return R(a, d) < R(b, d);
-        return a < b;
-    });
     int64_t rm = 0, r1m = 0;
     for (int64_t i = 0; i < n; ++i) {
         rm = std::max<int64_t>(rm, std::llabs(R((int)i, 0)));
         r1m = std::max<int64_t>(r1m, std::llabs(R((int)i, 1)));
     }
     if (rm > kAxisMaxR || r1m > kAxisMaxR) return;
-    std::vector<int> pe;
-    std::vector<unsigned short> pidx((2 * rm + 1) * (2 * r1m + 1));
-    for (int64_t i = 0; i < n; ++i) {
-        const int c = order[i];
-        if (i == 0 || R(c, 0) != R(order[i - 1], 0) || R(c, 1) != R(order[i - 1], 1)) pe.push_back((int)i);
-    }
-    const int np = (int)pe.size();
-    std::fill(pidx.begin(), pidx.end(), (unsigned short)np);
+    // the cells by pairs (R0, R1), those with most cells first (the pairs that share a wave of
+    // stage A then have about as many), each in the order of R2 and filled up to a multiple of 4
+    std::map<std::pair<int64_t, int64_t>, std::vector<int>> by_pair;
+    for (int64_t i = 0; i < n; ++i) by_pair[{R((int)i, 0), R((int)i, 1)}].push_back((int)i);
+    std::vector<std::vector<int>> pairs;
+    for (auto &c : by_pair) pairs.push_back(std::move(c.second));
+    std::stable_sort(pairs.begin(), pairs.end(), [](const auto &a, const auto &b) { return a.size() > b.size(); });
+    const int np = (int)pairs.size();
+    if (pairs[0].size() > kAxisMaxCnt) return;
+    std::vector<int> pe, order;
+    std::vector<unsigned short> pidx((2 * rm + 1) * (2 * r1m + 1), (unsigned short)np);
     for (int p = 0; p < np; ++p) {
-        const int c = order[pe[p]];
-        pidx[(R(c, 0) + rm) * (2 * r1m + 1) + R(c, 1) + r1m] = (unsigned short)p;
+        std::vector<int> &c = pairs[p];
+        std::stable_sort(c.begin(), c.end(), [&](int a, int b) { return R(a, 2) < R(b, 2); });
+        pidx[(R(c[0], 0) + rm) * (2 * r1m + 1) + R(c[0], 1) + r1m] = (unsigned short)p;
+        pe.push_back((int)order.size());
+        order.insert(order.end(), c.begin(), c.end());
+        while (order.size() % 4) order.push_back(-1);
     }
-    pe.push_back((int)n);
-    for (int p = 0; p < np; ++p)
-        if (pe[p + 1] - pe[p] > kAxisMaxCnt) return;
+    pe.push_back((int)order.size());
+    const int64_t ne = (int64_t)order.size();
     // lines and planes of the rows; ascending mesh order is what makes a line's rows consecutive
     std::vector<int> pl_k2, line_k, line_row;
     for (int64_t r = 0; r < nwv; ++r) {
@@ -3835,7 +3834,7 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     t.CT = (int)(16 * ((t.spt * nin + 15) / 16));
     t.CPs = (int)((nout + t.spt - 1) / t.spt) * t.CT;
     t.np = np;
-    t.ncell = (int)n;
+    t.ncell = (int)ne;
     t.rm = (int)rm;
     t.r1m = (int)r1m;
     t.npl = (int)npl;
@@ -3865,12 +3864,13 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
         const double a = kTwoPi * (double)fmodulo(j, m) / (double)m;
         return make_double2(std::cos(a), std::sin(a));
     };
-    std::vector<double2> phA(N[2] * n), T0(N[0]), T1(N[1]), T2(N[2]);
+    std::vector<double2> phA(N[2] * ne, make_double2(0.0, 0.0)), T0(N[0]), T1(N[1]), T2(N[2]);
     for (int64_t j = 0; j < N[0]; ++j) T0[j] = root(j, N[0]);
     for (int64_t j = 0; j < N[1]; ++j) T1[j] = root(j, N[1]);
     for (int64_t j = 0; j < N[2]; ++j) T2[j] = root(j, N[2]);
     for (int64_t q = 0; q < N[2]; ++q)
-        for (int64_t e = 0; e < n; ++e) phA[q * n + e] = T2[fmodulo(q * R(order[e], 2), N[2])];
+        for (int64_t e = 0; e < ne; ++e)
+            if (order[e] >= 0) phA[q * ne + e] = T2[fmodulo(q * R(order[e], 2), N[2])];
     x.pe.upload(pe, s);
     x.ecell.upload(order, s);
     x.pidx.upload(pidx, s);
