@@ -614,7 +614,9 @@ __device__ __forceinline__ int axis_items(int mine, int lane, unsigned short *it
 // The same for ibzq (rows k, no shift), the states of one IBZ q in turn: items
 // (row, RANKS in-window ranks m); W(np) += U_k(m, mp) Y(np, mp) per column tile
 // of mp, then for every in-window n of k' = k + q, g = sum_np conj(U_k'(n, np)) W(np)
-// and |g|^2 as in ibzq_row.
+// and |g|^2 as in ibzq_row.  Loads return in order: those of U_k for a tile are issued
+// ahead of the F2 of the next one, the first U_k'(n) ahead of the next state's, and a lane
+// keeps the bands of its k' so that no load waits for another.
 template <int NBM, int RANKS, int MT, int KS>
 __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, const double2 *__restrict__ F2, int st0, int ns,
                                                         int qb0, const int *__restrict__ qst, int nblk, int msplit) {
@@ -657,6 +659,20 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
         const dv2 *U[RANKS];
 #pragma unroll
         for (int k = 0; k < RANKS; ++k) U[k] = Vk + ((size_t)row * nb + a.wband[row * nb + rank + (k < nr ? k : 0)]) * nb;
+        unsigned long long bands = 0;  // in-window bands of k'
+        if constexpr (NBM <= 16)
+            for (int j = 0; j < nn; ++j) bands |= (unsigned long long)a.wband[kp * nb + j] << (4 * j);
+        auto kprow = [&](int nj) {
+            return Vk + ((size_t)kp * nb + (NBM <= 16 ? (int)(bands >> (4 * nj)) & 15 : a.wband[kp * nb + nj])) * nb;
+        };
+        constexpr bool PV = NBM <= 12 && MT * KS <= 2;  // the next n's U_k' loaded ahead (registers)
+        dv2 vn[PV ? NBM : 1];
+        auto load_v = [&](int nj) {
+            const dv2 *v = kprow(nj);
+            if constexpr (PV)
+#pragma unroll
+                for (int i = 0; i < NBM; ++i) vn[i] = i < nb ? v[i] : dv2{0.0, 0.0};
+        };
         sc.load(F2l + (size_t)(s_lo - st0) * ssz);
         for (int st = s_lo; st < s_hi; st += msplit) {
             const double2 *F2c = F2l + (size_t)(st - st0) * ssz;
@@ -667,45 +683,56 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
             for (int k = 0; k < RANKS; ++k)
 #pragma unroll
                 for (int i = 0; i < NBM; ++i) Wx[k][i] = Wy[k][i] = 0.0;
-            dv2 un[RANKS];
+            dv2 u[2][RANKS];
+            auto load_u = [&](int mp) {
 #pragma unroll
-            for (int k = 0; k < RANKS; ++k) un[k] = U[k][0];
+                for (int k = 0; k < RANKS; ++k) {
+                    u[0][k] = U[k][min(mp, nb - 1)];
+                    u[1][k] = U[k][min(mp + 1, nb - 1)];
+                }
+            };
             for (int i = lane; i < N0 * npad; i += 64) Yw[i / npad * ys + x.CT + i % npad] = make_double2(0.0, 0.0);
             for (int t0 = 0, mp = 0; t0 < x.CPs; t0 += x.CT) {
+                load_u(mp);
+                if (t0 + x.CT >= x.CPs) load_v(0);
                 for (int cb = 0; cb < x.CT; cb += 16)
                     sc.tile(t0 + cb + 16 < x.CPs ? F2c + t0 + cb + 16 : F2n, ys, N0, lane, Yw + cb);
                 wave_lds_sync();
                 const double2 *Yr = Yw + yrow * ys;
-                for (int j = 0; j < x.spt && mp < nb; ++j, ++mp, Yr += nb) {
-                    dv2 u[RANKS];
-#pragma unroll
-                    for (int k = 0; k < RANKS; ++k) {
-                        u[k] = un[k];
-                        un[k] = U[k][min(mp + 1, nb - 1)];
-                    }
+                auto mac = [&](int h) {
 #pragma unroll
                     for (int i = 0; i < NBM; ++i) {
                         const double2 y = Yr[i];
 #pragma unroll
                         for (int k = 0; k < RANKS; ++k) {
-                            Wx[k][i] = fma(u[k].x, y.x, Wx[k][i]);
-                            Wy[k][i] = fma(u[k].x, y.y, Wy[k][i]);
-                            Wx[k][i] = fma(-u[k].y, y.y, Wx[k][i]);
-                            Wy[k][i] = fma(u[k].y, y.x, Wy[k][i]);
+                            Wx[k][i] = fma(u[h][k].x, y.x, Wx[k][i]);
+                            Wy[k][i] = fma(u[h][k].x, y.y, Wy[k][i]);
+                            Wx[k][i] = fma(-u[h][k].y, y.y, Wx[k][i]);
+                            Wy[k][i] = fma(u[h][k].y, y.x, Wy[k][i]);
                         }
                     }
+                    ++mp;
+                    Yr += nb;
+                };
+                for (const int m1 = min(mp + x.spt, nb); mp < m1;) {
+                    mac(0);
+                    if (mp < m1) mac(1);
+                    if (mp < m1) load_u(mp);
                 }
                 wave_lds_sync();
             }
             double *stage = reinterpret_cast<double *>(Yw), *o = stage + off;
             for (int nj = 0; nj < nn; ++nj) {
-                const dv2 *Ukp = Vk + ((size_t)kp * nb + a.wband[kp * nb + nj]) * nb;
+                const dv2 *Ukp = kprow(nj);
                 double2 g[RANKS];
 #pragma unroll
                 for (int k = 0; k < RANKS; ++k) g[k] = make_double2(0.0, 0.0);
                 dv2 v[NBM];
 #pragma unroll
-                for (int i = 0; i < NBM; ++i) v[i] = i < nb ? Ukp[i] : dv2{0.0, 0.0};
+                for (int i = 0; i < NBM; ++i)
+                    if constexpr (PV) v[i] = vn[i];
+                    else v[i] = i < nb ? Ukp[i] : dv2{0.0, 0.0};
+                if constexpr (PV) load_v(min(nj + 1, nn - 1));
 #pragma unroll
                 for (int i = 0; i < NBM; ++i)
 #pragma unroll
