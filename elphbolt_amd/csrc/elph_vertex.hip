@@ -2209,20 +2209,26 @@ __global__ __launch_bounds__(256) void k_pair_q_fp64(PairQArgs a) {
 // ---------------------------------------------------------------------------
 
 // H[k][ij] = sum_R phi[k][R] Hw[R][ij]; dH[k][p][ij] = sum_R i rcart_p(R) phi Hw
-// (src/wannier.f90:462-478).
-__global__ void k_build_H(int nk, int nb2, int nws, const double2 *__restrict__ phi, const double2 *__restrict__ HwT,
-                          const double *__restrict__ rcart, double2 *__restrict__ H, double2 *__restrict__ dH) {
+// (src/wannier.f90:462-478).  A wave forms 64 elements of one k; the phases are wave-uniform,
+// scalar operands four R at a time (3100 k, 423 cells, 8 bands: 141 -> 78 us).  The reads of Hw
+// from L2 bound it.  Several k per wave read it less often, but every one adds scalar loads
+// that the wave waits for: 8 k 292 us, 4 k 106 us.
+template <bool VEL>
+__global__ __launch_bounds__(64) void k_build_H(int nk, int nb2, int nws, const double2 *__restrict__ phi,
+                                                const double2 *__restrict__ HwT, const double *__restrict__ rcart,
+                                                double2 *__restrict__ H, double2 *__restrict__ dH) {
     const int k = blockIdx.y;
-    const int ij = blockIdx.x * blockDim.x + threadIdx.x;
+    const int ij = blockIdx.x * 64 + threadIdx.x;
     if (ij >= nb2 || k >= nk) return;
-    double2 acc = make_double2(0.0, 0.0);
-    double2 d0 = acc, d1 = acc, d2 = acc;
-    const double2 *ph = phi + (size_t)k * nws;
+    double2 acc = make_double2(0.0, 0.0), d0 = acc, d1 = acc, d2 = acc;
+    const sc_dv2 ph = as_scalar(phi) + (size_t)k * nws;
+#pragma unroll 4
     for (int r = 0; r < nws; ++r) {
-        const double2 t = cmul(ph[r], HwT[(size_t)r * nb2 + ij]);
+        const dv2 w = ph[r];
+        const double2 t = cmul(make_double2(w.x, w.y), HwT[(size_t)r * nb2 + ij]);
         acc.x += t.x;
         acc.y += t.y;
-        if (dH) {
+        if constexpr (VEL) {
             const double x = rcart[3 * r], y = rcart[3 * r + 1], z = rcart[3 * r + 2];
             d0.x -= x * t.y; d0.y += x * t.x;
             d1.x -= y * t.y; d1.y += y * t.x;
@@ -2230,56 +2236,88 @@ __global__ void k_build_H(int nk, int nb2, int nws, const double2 *__restrict__ 
         }
     }
     H[(size_t)k * nb2 + ij] = acc;
-    if (dH) {
+    if constexpr (VEL) {
         dH[((size_t)k * 3 + 0) * nb2 + ij] = d0;
         dH[((size_t)k * 3 + 1) * nb2 + ij] = d1;
         dH[((size_t)k * 3 + 2) * nb2 + ij] = d2;
     }
 }
+void build_H(const elph_ctx *c, hipStream_t s, int64_t nk, const double2 *phi, double2 *H, double2 *dH) {
+    const int64_t nb2 = c->nb * c->nb;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((nb2 + 63) / 64), (unsigned)nk), dim3(64), 0, s, (int)nk, (int)nb2,
+                           (int)c->nwsk, phi, c->HwT.p, c->rcart_k.p, H, dH);
+    };
+    if (dH) go(k_build_H<true>);
+    else go(k_build_H<false>);
+}
 
 // D(q) of src/wannier.f90:631-665: for each cell, the WS-wrapped images of the
-// atom pair, weighted 1 / (phwsdeg * num_wrap), times Dphwann.
-__global__ void k_build_D(int nq, int nbr, int nat, const double *__restrict__ qv, const int *__restrict__ toff,
-                          const int *__restrict__ tiuc, const int *__restrict__ tT, const int *__restrict__ tdiv,
-                          const double2 *__restrict__ DphT, const double *__restrict__ rcart, double2 *__restrict__ D,
-                          double2 *__restrict__ dD) {
-    const int q = blockIdx.y;
-    const int nbr2 = nbr * nbr;
-    const int ij = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ij >= nbr2 || q >= nq) return;
-    const int i = ij % nbr, j = ij / nbr;
-    const int ia = i / 3, ja = j / 3;
+// atom pair, weighted 1 / (phwsdeg * num_wrap), times Dphwann.  One wave per q and atom
+// pair: the lanes take an image each for its phase, 64 at a time into LDS, then seven
+// groups of nine lanes (the pair's 3 x 3 block) sum every seventh image.  With a thread per
+// element each phase's sine and cosine were formed nine times and by 36 of 64 lanes at six
+// branches (3000 q, 279 cells, 2 atoms, with velocities: 0.515 ms, now 0.116).
+__global__ __launch_bounds__(64) void k_build_D(int nq, int nbr, int nat, const double *__restrict__ qv,
+                                                const int *__restrict__ toff, const int *__restrict__ tiuc,
+                                                const int *__restrict__ tT, const int *__restrict__ tdiv,
+                                                const double2 *__restrict__ DphT, const double *__restrict__ rcart,
+                                                double2 *__restrict__ D, double2 *__restrict__ dD) {
+    __shared__ double2 cm[64];
+    __shared__ int cell[64];
+    __shared__ double red[8][64];
+    const int q = blockIdx.y, pair = blockIdx.x, lane = threadIdx.x;
+    const int ia = pair % nat, ja = pair / nat, nbr2 = nbr * nbr;
+    const int g = lane / 9, e = lane - 9 * g;
+    const int ij = 3 * ia + e % 3 + nbr * (3 * ja + e / 3);
     const double qx = qv[q], qy = qv[q + nq], qz = qv[q + 2 * nq];
     double2 acc = make_double2(0.0, 0.0), d0 = acc, d1 = acc, d2 = acc;
-    const int pair = ia + nat * ja;
-    int t = toff[pair];
     const int tend = toff[pair + 1];
-    while (t < tend) {
-        const int iuc = tiuc[t];
-        double2 cm = make_double2(0.0, 0.0);
-        for (; t < tend && tiuc[t] == iuc; ++t) {
+    for (int t0 = toff[pair]; t0 < tend; t0 += 64) {
+        const int t = t0 + lane, n = min(64, tend - t0);
+        if (t < tend) {
             const double dot = qx * (double)tT[3 * t] + qy * (double)tT[3 * t + 1] + qz * (double)tT[3 * t + 2];
             double s, c;
             sincos(kTwoPi * dot, &s, &c);
             const double dv = (double)tdiv[t];
-            cm.x += c / dv;
-            cm.y += s / dv;
+            cm[lane] = make_double2(c / dv, s / dv);
+            cell[lane] = tiuc[t];
         }
-        const double2 v = cmul(cm, DphT[(size_t)iuc * nbr2 + ij]);
-        acc.x += v.x;
-        acc.y += v.y;
-        if (dD) {
-            const double x = rcart[3 * iuc], y = rcart[3 * iuc + 1], z = rcart[3 * iuc + 2];
-            d0.x -= x * v.y; d0.y += x * v.x;
-            d1.x -= y * v.y; d1.y += y * v.x;
-            d2.x -= z * v.y; d2.y += z * v.x;
+        __syncthreads();
+        if (g < 7) {
+#pragma unroll 3
+            for (int i = g; i < n; i += 7) {
+                const int iuc = cell[i];
+                const double2 v = cmul(cm[i], DphT[(size_t)iuc * nbr2 + ij]);
+                acc.x += v.x;
+                acc.y += v.y;
+                if (dD) {
+                    const double x = rcart[3 * iuc], y = rcart[3 * iuc + 1], z = rcart[3 * iuc + 2];
+                    d0.x -= x * v.y; d0.y += x * v.x;
+                    d1.x -= y * v.y; d1.y += y * v.x;
+                    d2.x -= z * v.y; d2.y += z * v.x;
+                }
+            }
         }
+        __syncthreads();
     }
-    D[(size_t)q * nbr2 + ij] = acc;
+    red[0][lane] = acc.x;
+    red[1][lane] = acc.y;
     if (dD) {
-        dD[((size_t)q * 3 + 0) * nbr2 + ij] = d0;
-        dD[((size_t)q * 3 + 1) * nbr2 + ij] = d1;
-        dD[((size_t)q * 3 + 2) * nbr2 + ij] = d2;
+        red[2][lane] = d0.x; red[3][lane] = d0.y;
+        red[4][lane] = d1.x; red[5][lane] = d1.y;
+        red[6][lane] = d2.x; red[7][lane] = d2.y;
+    }
+    __syncthreads();
+    // lane 9 m + e: value m (0: D, 1 .. 3: dD) of element e
+    if (lane < (dD ? 36 : 9)) {
+        double2 sum = make_double2(0.0, 0.0);
+        for (int j = 0; j < 7; ++j) {
+            sum.x += red[2 * g][9 * j + e];
+            sum.y += red[2 * g + 1][9 * j + e];
+        }
+        if (g == 0) D[(size_t)q * nbr2 + ij] = sum;
+        else dD[((size_t)q * 3 + g - 1) * nbr2 + ij] = sum;
     }
 }
 
@@ -3042,19 +3080,15 @@ void elph::launch_jacobi(hipStream_t st, int64_t nmat, int n, const double2 *A, 
 
 void elph::launch_build_H(elph_ctx *c, hipStream_t st, int64_t n, const double *d_kvecs, int64_t vstride, double2 *phi,
                           double2 *H) {
-    const int64_t nb2 = c->nb * c->nb;
     dim3 gp((unsigned)((c->nwsk + 127) / 128), (unsigned)n);
     hipLaunchKernelGGL(k_phase_list, gp, dim3(128), 0, st, (int)n, (int)c->nwsk, d_kvecs, vstride, c->rk.p, c->degk.p,
                        phi, c->nwsk, (int64_t)1);
-    dim3 grid((unsigned)((nb2 + 63) / 64), (unsigned)n);
-    hipLaunchKernelGGL(k_build_H, grid, dim3(64), 0, st, (int)n, (int)nb2, (int)c->nwsk, phi, c->HwT.p, c->rcart_k.p,
-                       H, (double2 *)nullptr);
+    build_H(c, st, n, phi, H, nullptr);
     HCHECK(hipGetLastError());
 }
 
 void elph::launch_dynmat(elph_ctx *c, hipStream_t st, int64_t nq, const double *d_qvecs, double2 *D) {
-    const int64_t nbr2 = c->nbr * c->nbr;
-    dim3 grid((unsigned)((nbr2 + 63) / 64), (unsigned)nq);
+    const dim3 grid((unsigned)(c->natoms * c->natoms), (unsigned)nq);
     hipLaunchKernelGGL(k_build_D, grid, dim3(64), 0, st, (int)nq, (int)c->nbr, (int)c->natoms, d_qvecs,
                        c->term_off.p, c->term_iuc.p, c->term_T.p, c->term_div.p, c->DphT.p, c->rcart_q.p, D,
                        (double2 *)nullptr);
@@ -3121,9 +3155,7 @@ void el_wann_device(elph_ctx *c, int64_t nk, const double *d_kvecs, DBuf<double>
     phase_list(c, nk, d_kvecs, c->rk, c->degk, c->nwsk, phi);
     H.alloc(nk * nb2);
     if (vel) dH.alloc(nk * 3 * nb2);
-    dim3 grid((unsigned)((nb2 + 63) / 64), (unsigned)nk);
-    hipLaunchKernelGGL(k_build_H, grid, dim3(64), 0, c->stream, (int)nk, (int)nb2, (int)c->nwsk, phi.p, c->HwT.p,
-                       c->rcart_k.p, H.p, vel ? dH.p : (double2 *)nullptr);
+    build_H(c, c->stream, nk, phi.p, H.p, vel ? dH.p : (double2 *)nullptr);
     W.alloc(nk * nb);
     V.alloc(nk * nb2);
     launch_jacobi(c->stream, nk, (int)nb, H.p, nullptr, W.p, V.p);
@@ -3142,7 +3174,7 @@ void ph_wann_device(elph_ctx *c, int64_t nq, const double *d_qvecs, DBuf<double>
     DBuf<double2> D, dD;
     D.alloc(nq * nbr2);
     if (vel) dD.alloc(nq * 3 * nbr2);
-    dim3 grid((unsigned)((nbr2 + 63) / 64), (unsigned)nq);
+    const dim3 grid((unsigned)(c->natoms * c->natoms), (unsigned)nq);
     hipLaunchKernelGGL(k_build_D, grid, dim3(64), 0, c->stream, (int)nq, (int)nbr, (int)c->natoms, d_qvecs,
                        c->term_off.p, c->term_iuc.p, c->term_T.p, c->term_div.p, c->DphT.p, c->rcart_q.p, D.p,
                        vel ? dD.p : (double2 *)nullptr);
