@@ -3933,11 +3933,14 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     x.on = true;
 }
 
+// LDS of a k_axis_pair workgroup up to which u_q is kept there: half a CU's, so that two
+// workgroups share it (24^3, 6 branches: 79.5 KB, 6.08 -> 5.21 ms; one workgroup per CU would halve the
+// waves that hide each other's latency).
+constexpr size_t kAxisUldsMax = 80 << 10;
 // States per chunk of the axis path for nst states: h and F2 of a chunk within `cap`
 // bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
 // of 1786 states at 617 cells, 24^3: 15.0 / 10.6 / 10.2 / 10.1 / 9.9 ms at 64 MiB / 128 MiB /
 // 512 MiB / 1 GiB / 3 GB; 251 states of 16 bands, 15 branches on 20^3: 14.4 / 9.3 / 7.8 / 7.2 / 7.1).
-constexpr size_t kAxisUldsMax = 80 << 10;
 constexpr int64_t kAxisChunkBytes = (int64_t)1 << 30;
 int64_t axis_chunk(const AxisPlan &x, int64_t nst, int64_t cap) {
     const int64_t per_state = (x.h_state() + x.f2_state()) * (int64_t)sizeof(double2);
