@@ -87,6 +87,7 @@ PROTOTYPES = {
     "elph_el_transport_destroy": (ct.c_int, [ct.c_void_p]),
     "elph_ibzk_plan_X": (ct.c_int, [ct.c_void_p, ct.c_void_p, ct.c_double, ct.c_double, ct.c_int64, ct.c_int64,
                                     ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p]),
+    "elph_ibzk_plan_form": (ct.c_int, [ct.c_void_p, ct.c_int32, ct.POINTER(ct.c_int32)]),
     "elph_ibzk_plan_destroy": (ct.c_int, [ct.c_void_p]),
     "elph_ibzk_g2": (ct.c_int, [ct.c_void_p, ct.POINTER(ElphElectrons), ct.POINTER(ElphPhonons), ct.c_int64, ct.c_int32,
                                 ct.c_int64, ct.c_int64, c_i64p, c_dblp]),
@@ -94,6 +95,7 @@ PROTOTYPES = {
                                          ct.POINTER(ct.c_void_p)]),
     "elph_ibzq_plan_run": (ct.c_int, [ct.c_void_p, ct.c_int64, ct.c_int64, c_i64p, ct.c_void_p, ct.c_int32]),
     "elph_ibzq_plan_stride": (ct.c_int64, [ct.c_void_p]),
+    "elph_ibzq_plan_form": (ct.c_int, [ct.c_void_p, ct.c_int32, ct.POINTER(ct.c_int32)]),
     "elph_ibzq_plan_destroy": (ct.c_int, [ct.c_void_p]),
     "elph_write_X_files": (ct.c_int, [ct.c_char_p, ct.c_int64, ct.c_int64, c_i64p, c_dblp, c_dblp, c_i64p, c_i64p,
                                       ct.c_int64]),

@@ -3937,6 +3937,17 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
 // workgroups share it (24^3, 6 branches: 79.5 KB, 6.08 -> 5.21 ms; one workgroup per CU would halve the
 // waves that hide each other's latency).
 constexpr size_t kAxisUldsMax = 80 << 10;
+// The forms that a plan has (pair, pts) and takes (axis, axis_pts): elph_ibzk_plan_form.
+int axis_choice(int32_t want, bool pair, bool pts, bool &axis, bool &axis_pts, int32_t *form) {
+    if (want >= 0) {
+        if (want > 3 || ((want & ELPH_FORM_AXIS_PAIR) && !pair) || ((want & ELPH_FORM_AXIS_POINTS) && !pts)) return ELPH_EINVAL;
+        axis = (want & ELPH_FORM_AXIS_PAIR) != 0;
+        axis_pts = (want & ELPH_FORM_AXIS_POINTS) != 0;
+    }
+    if (form) *form = (axis ? ELPH_FORM_AXIS_PAIR : 0) | (axis_pts ? ELPH_FORM_AXIS_POINTS : 0);
+    return ELPH_OK;
+}
+
 // States per chunk of the axis path for nst states: h and F2 of a chunk within `cap`
 // bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
 // of 1786 states at 617 cells, 24^3: 15.0 / 10.6 / 10.2 / 10.1 / 9.9 ms at 64 MiB / 128 MiB /
@@ -4294,7 +4305,8 @@ struct elph_ibzk_plan {
     AxisPlan ax;
     bool axis = false;
     DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
-    AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 runs) where kcells.on
+    AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 plans) where kcells.on; `axis_pts`
+    bool axis_pts = false;  // says whether runs take it
     TablePack tables;       // the groups' tables of the running call
     HostBuf tables_host;
     DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
@@ -4730,7 +4742,7 @@ std::vector<GroupHost> ibzk_group_hosts(const elph_ibzk_plan *p, int64_t first, 
 }
 
 // Adds the tables of a group to `t` (`h` must live until t.upload).
-void ibzk_group_pack(GroupHost &h, const AxisCells &cells, IbzkGroup &g, TablePack &t) {
+void ibzk_group_pack(const elph_ibzk_plan *p, GroupHost &h, IbzkGroup &g, TablePack &t) {
     g.nkb = h.nkb;
     g.nst = h.nst;
     g.slot = h.slot;
@@ -4741,8 +4753,8 @@ void ibzk_group_pack(GroupHost &h, const AxisCells &cells, IbzkGroup &g, TablePa
     t.add(h.ski, g.st_kint);
     t.add(h.kst, g.kst);
     g.kst_host = h.kst;
-    if (cells.on) {
-        h.pts = axis_pts_host(cells, h.kint);
+    if (p->axis_pts) {
+        h.pts = axis_pts_host(p->kcells, h.kint);
         g.pts.pack(h.pts, t);
     }
     t.add(h.sslot, g.st_slot);
@@ -4753,7 +4765,7 @@ size_t ibzk_group_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst) {
     auto b = [](int64_t n, size_t size) { return TablePack::round((size_t)n * size); };
     size_t total = b(3 * nkb, sizeof(double)) + b(nkb * p->nb * p->nb, sizeof(double2)) + 2 * b(nst, sizeof(int)) +
                    b(3 * nst, sizeof(int)) + b(nkb + 1, sizeof(int)) + b(nst, sizeof(int64_t));
-    if (p->kcells.on)
+    if (p->axis_pts)
         total += b(nkb + 1, sizeof(int)) + b(nkb, sizeof(int)) + b(nkb, sizeof(int4)) +
                  b(axis_pts_phases(p->kcells, nkb), sizeof(double2));
     return total;
@@ -4763,14 +4775,14 @@ void ibzk_groups(elph_ibzk_plan *p, int64_t first, int64_t last, bool on_device,
                  std::vector<std::unique_ptr<IbzkGroup>> &groups, TablePack &tables, HostBuf *pinned, bool compact = false) {
     // IBZ k per group: the k of one launch of the Re contraction
     // (rows staged for the host, and the direct product's operand, bound a group at the smaller size)
-    const int64_t KB = p->kcells.on && p->axis && on_device
+    const int64_t KB = p->axis_pts && p->axis && on_device
                            ? axis_pts_max(p->nb * p->nb * p->nbr * p->ctx->nwsg * (int64_t)sizeof(double2))
                            : (p->precision == ELPH_MIXED ? kGkKTMixed : kGkKT);
     std::vector<GroupHost> hosts = ibzk_group_hosts(p, first, last, on_device, counts, compact, KB);
     tables.clear();
     for (GroupHost &h : hosts) {
         groups.push_back(std::make_unique<IbzkGroup>());
-        ibzk_group_pack(h, p->kcells, *groups.back(), tables);
+        ibzk_group_pack(p, h, *groups.back(), tables);
     }
     if (!hosts.empty()) tables.upload(s, pinned);
 }
@@ -4823,7 +4835,7 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
 void ibzk_prep(elph_ibzk_plan *p, const IbzkGroup &g, IbzkScratch &sc, hipStream_t s) {
     elph_ctx *c = p->ctx;
     const int64_t nb = p->nb, nbr = p->nbr, nb2 = nb * nb, nslices = nbr * c->nwsg;
-    if (p->kcells.on && p->precision != ELPH_MIXED) {
+    if (p->axis_pts) {
         AxisPtsArgs a{};
         a.g = c->gwann.p;
         a.cstride = nb2;
@@ -5070,6 +5082,7 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
             if (p->kcells.on && ctx->lds_max > 0 &&
                 (int64_t)axis_pts_lds(p->kcells, kPtsPlanes, 1024) > ctx->lds_max)
                 p->kcells.on = false;
+            p->axis_pts = p->kcells.on;
             if (p->ax.on) {
                 auto transposed = [&](const std::vector<double2> &v, DBuf<double2> &dst) {
                     std::vector<double2> w(v.size());
@@ -5117,6 +5130,11 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
 }
 
 int64_t elph_ibzk_plan_nprocs(const elph_ibzk_plan *p) { return p ? p->nprocs : -1; }
+
+int elph_ibzk_plan_form(elph_ibzk_plan *p, int32_t want, int32_t *form) {
+    if (!p) return ELPH_EINVAL;
+    return axis_choice(want, p->ax.on, p->kcells.on, p->axis, p->axis_pts, form);
+}
 
 int elph_ibzk_plan_destroy(elph_ibzk_plan *p) {
     delete p;
@@ -5220,7 +5238,7 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         cv.take(tables.dev, ibzk_group_bytes(p, nkb, nst));
         HCHECK(hipEventRecord(c->ev_c, s));
         for (GroupHost &h : hosts) {
-            ibzk_group_pack(h, p->kcells, g, tables);
+            ibzk_group_pack(p, h, g, tables);
             tables.upload(s, nullptr);  // stream-ordered after the previous group's kernels
             ibzk_enqueue(p, g, sc, s, g2_device, true);
         }
@@ -5389,7 +5407,7 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
     }
     // the axis-by-axis form where the sizes take it: it is not timed against the
     // direct product, whose operand preparation lies outside the pair stage
-    if (p->ax.on) cands.assign(1, TileCand{false, 0, 0, true});
+    if (p->axis) cands.assign(1, TileCand{false, 0, 0, true});
     if (!tune) cands.resize(1);
     const IbzkGroup &g = *it.groups.front();
     IbzkScratch sc;
@@ -5522,7 +5540,7 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
                 // plans of the axis-by-axis form keep it; the others take the class's
                 // tile shape where one was timed, else the plan's own
                 const elph_batch_class_t &r = b->classes[f->second].rep;
-                if (!it.p->ax.on && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
+                if (!it.p->axis && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
             }
             it.cls = f->second;
             b->classes[f->second].members += 1;
@@ -5767,9 +5785,12 @@ struct elph_ibzq_plan {
     DBuf<double> g2stage;
     bool general = false;  // nb^2 beyond the fused kernel: Y tiles in HBM, then the epilogue
     DBuf<double2> Y;
-    AxisPlan ax;           // axis-by-axis form where ax.on
+    // axis-by-axis form of the pair stage where ax.on and of the Rp sum where rcells.on;
+    // `axis` and `axis_pts` say whether runs take them
+    AxisPlan ax;
     DBuf<double2> F2;
-    AxisCells rcells;      // axis-by-axis form of the Rp sum where rcells.on
+    AxisCells rcells;
+    bool axis = false, axis_pts = false;
     AxisPts pts;
     TablePack tables;      // the tables of the running batch of q
     HostBuf tables_host;
@@ -5877,6 +5898,8 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         axis_cells_build(p->rcells, ctx->rcells_g.data(), ctx->nwsg, ctx->nwsg, ctx->gwsdeg, p->Nel, s);
         if (p->rcells.on && ctx->lds_max > 0 && (int64_t)axis_pts_lds(p->rcells, kPtsPlanes, 1024) > ctx->lds_max)
             p->rcells.on = false;
+        p->axis = p->ax.on;
+        p->axis_pts = p->rcells.on;
         p->nirr_q = ph->nwv_irred;
         p->nq = ph->nwv;
         p->q_irr.assign(ph->indexlist_irred, ph->indexlist_irred + ph->nwv_irred);
@@ -5891,6 +5914,11 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
 }
 
 int64_t elph_ibzq_plan_stride(const elph_ibzq_plan *p) { return p ? p->stride : -1; }
+
+int elph_ibzq_plan_form(elph_ibzq_plan *p, int32_t want, int32_t *form) {
+    if (!p) return ELPH_EINVAL;
+    return axis_choice(want, p->ax.on, p->rcells.on, p->axis, p->axis_pts, form);
+}
 
 int elph_ibzq_plan_destroy(elph_ibzq_plan *p) {
     delete p;
@@ -5911,7 +5939,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
         HCHECK(hipEventRecord(c->ev_c, s));
         const int64_t gblk = nb2 * nbr * c->nwsk;
         // IBZ q per pass over gwann
-        const int64_t QB = p->rcells.on && p->ax.on && on_device ? axis_pts_max(gblk * (int64_t)sizeof(double2)) : 16 * kGReqNCB;
+        const int64_t QB = p->axis_pts && p->axis && on_device ? axis_pts_max(gblk * (int64_t)sizeof(double2)) : 16 * kGReqNCB;
         int64_t istate = first;
         while (istate <= last) {
             // states of up to QB distinct IBZ q
@@ -5956,11 +5984,11 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 sslot[t] = on_device ? (sts[t] - first) : t;
             }
             qst.push_back((int)nst);
-            if (p->ax.on)
+            if (p->axis)
                 for (int64_t b = 0; b < nqb; ++b)  // one row set per q
                     for (int d = 0; d < 3; ++d) sqe[3 * b + d] = sqe[3 * qst[b] + d];
             AxisPtsHost ph;
-            if (p->rcells.on) {
+            if (p->axis_pts) {
                 std::vector<int> qint(3 * nqb);
                 for (int64_t b = 0; b < nqb; ++b) {
                     int64_t v[3];
@@ -5972,7 +6000,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             TablePack &tp = p->tables;
             tp.clear();
             tp.add(qv, p->qv);
-            if (p->rcells.on) p->pts.pack(ph, tp);
+            if (p->axis_pts) p->pts.pack(ph, tp);
             tp.add(qst, p->qst);
             tp.add(sqb, p->st_qb);
             tp.add(sqe, p->st_qe);
@@ -5981,7 +6009,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             tp.add(sslot, p->st_slot);
             tp.upload(s, &p->tables_host);
             p->gq.alloc(nqb * gblk);
-            if (p->rcells.on) {
+            if (p->axis_pts) {
                 AxisPtsArgs pa{};
                 pa.g = c->gwann.p;
                 pa.cstride = nb2 * c->nwsk * nbr;
@@ -6004,13 +6032,13 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                 hipLaunchKernelGGL(k_polar_lp, dim3((unsigned)((nst + 255) / 256)), dim3(256), 0, s, (int)nst,
                                    (int)nbr, 1, p->st_qb.p, p->Lq.p, p->st_u.p, p->st_lp.p);
             }
-            if (!p->ax.on) p->h.alloc(nst * p->Kp * p->CP);
+            if (!p->axis) p->h.alloc(nst * p->Kp * p->CP);
             const int64_t tot = nst * p->Kp * p->CP;
-            if (!p->ax.on) hipLaunchKernelGGL(k_rotate_hq, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, (int)nst, (int)nb,
+            if (!p->axis) hipLaunchKernelGGL(k_rotate_hq, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, (int)nst, (int)nb,
                                (int)nbr, (int)c->npairk, (int)p->Kp, (int)p->CP, p->gq.p, gblk, p->st_qb.p, p->st_u.p,
                                c->gpair.p, c->ginvdeg.p, p->h.p);
             // rows of the states (axis form: of the q, which its states share)
-            const int64_t nrm = p->ax.on ? nqb : nst;
+            const int64_t nrm = p->axis ? nqb : nst;
             p->rowmap.alloc(nrm * p->nwv);
             p->rowoff.alloc(nrm * p->nwv);
             p->st_tot.alloc(nrm);
@@ -6126,7 +6154,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                     default: throw Error{ELPH_EINVAL, "unsupported column count"};
                 }
             };
-            if (p->ax.on) axis();
+            if (p->axis) axis();
             else if (packed) launch(std::true_type{});
             else launch(std::false_type{});
             HCHECK(hipGetLastError());
@@ -6138,7 +6166,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             HCHECK(hipEventElapsedTime(&ms, c->ev_a, c->ev_b));
             c->t_dominant_ms += ms;
             c->n_dominant += 1;
-            if (p->ax.on) {
+            if (p->axis) {
                 std::vector<int64_t> per_state(nst);
                 for (int64_t t = 0; t < nst; ++t) per_state[t] = tot_h[sqb[t]];
                 tot_h.swap(per_state);

@@ -59,8 +59,28 @@ def _dev_ptr(out):
     return out.ctypes.data_as(ct.c_void_p), 0
 
 
-class IbzkPlan:
+class _Form:
+    """How a plan sums over the Wannier cells (elph_ibzk_plan_form, elph_ibzq_plan_form)."""
+
+    _form = None  # name of the entry point
+
+    def form(self, pair=None, points=None):
+        """(pair stage axis by axis, sum at the IBZ points axis by axis), as runs take them; True or False
+        changes one of them for the runs that follow (ElphError if the plan does not have the form)."""
+        f, now = getattr(self.lib, self._form), ct.c_int32(0)
+        self.wann._check(f(self.plan, -1, ct.byref(now)), "plan form")
+        if pair is not None or points is not None:
+            want = (now.value & 1 if pair is None else int(pair)) | (now.value & 2 if points is None else 2 * int(points))
+            st = f(self.plan, want, ct.byref(now))
+            if st != 0:
+                raise ElphError(st, "plan form: the plan does not have it")
+        return bool(now.value & 1), bool(now.value & 2)
+
+
+class IbzkPlan(_Form):
     """calculate_eph_interaction_ibzk('g') with HBM-resident inputs."""
+
+    _form = "elph_ibzk_plan_form"
 
     def __init__(self, wann: Wannier, el, ph, mesh_ref: int = 1, precision: str = "fp64"):
         self.wann, self.lib = wann, wann.lib
@@ -271,8 +291,10 @@ class Batch:
             pass
 
 
-class IbzqPlan:
+class IbzqPlan(_Form):
     """calculate_eph_interaction_ibzq('g') with HBM-resident inputs."""
+
+    _form = "elph_ibzq_plan_form"
 
     def __init__(self, wann: Wannier, el, ph, precision: str = "fp64"):
         self.wann, self.lib = wann, wann.lib

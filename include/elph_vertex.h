@@ -166,6 +166,15 @@ int64_t elph_ibzk_plan_nprocs(const elph_ibzk_plan *plan);
  * the plan (which allocates) beforehand. */
 int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *plan, int64_t istate_first, int64_t istate_last, int64_t *counts,
                                double *g2_device);
+/* No counterpart in the reference.  How the plan sums over the Wannier cells: axis by
+ * axis of the mesh or as one product over all of them, for the pair stage
+ * (ELPH_FORM_AXIS_PAIR) and for the sum over Re at the IBZ k (ELPH_FORM_AXIS_POINTS;
+ * FP64 plans).  The plan chooses by its sizes when it is created; want >= 0 (the sum of
+ * the forms to take) changes that for the runs that follow, ELPH_EINVAL if the plan
+ * does not have the form.  form (may be NULL): what runs take now. */
+#define ELPH_FORM_AXIS_PAIR 1
+#define ELPH_FORM_AXIS_POINTS 2
+int elph_ibzk_plan_form(elph_ibzk_plan *plan, int32_t want, int32_t *form);
 int elph_ibzk_plan_destroy(elph_ibzk_plan *plan);
 /* One-shot form (plan + run + destroy). */
 int elph_ibzk_g2(elph_ctx *ctx, const elph_electrons *el, const elph_phonons *ph, int64_t mesh_ref,
@@ -181,6 +190,8 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
 int elph_ibzq_plan_run(elph_ibzq_plan *plan, int64_t istate_first, int64_t istate_last, int64_t *counts,
                        double *g2, int32_t g2_on_device);
 int64_t elph_ibzq_plan_stride(const elph_ibzq_plan *plan);
+/* elph_ibzk_plan_form for an ibzq plan (ELPH_FORM_AXIS_POINTS: the sum over Rp at the IBZ q). */
+int elph_ibzq_plan_form(elph_ibzq_plan *plan, int32_t want, int32_t *form);
 int elph_ibzq_plan_destroy(elph_ibzq_plan *plan);
 
 /* ---- Consumers of the g2 rows ----

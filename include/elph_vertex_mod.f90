@@ -194,6 +194,13 @@ module elph_vertex_mod
        type(c_ptr), value :: plan
      end function elph_ibzk_plan_nprocs
 
+     integer(c_int) function elph_ibzk_plan_form(plan, want, form) bind(C, name="elph_ibzk_plan_form")
+       import
+       type(c_ptr), value :: plan
+       integer(c_int32_t), value :: want
+       integer(c_int32_t) :: form
+     end function elph_ibzk_plan_form
+
      integer(c_int) function elph_ibzk_plan_destroy(plan) bind(C, name="elph_ibzk_plan_destroy")
        import
        type(c_ptr), value :: plan
@@ -233,6 +240,13 @@ module elph_vertex_mod
        import
        type(c_ptr), value :: plan
      end function elph_ibzq_plan_stride
+
+     integer(c_int) function elph_ibzq_plan_form(plan, want, form) bind(C, name="elph_ibzq_plan_form")
+       import
+       type(c_ptr), value :: plan
+       integer(c_int32_t), value :: want
+       integer(c_int32_t) :: form
+     end function elph_ibzq_plan_form
 
      integer(c_int) function elph_ibzq_plan_destroy(plan) bind(C, name="elph_ibzq_plan_destroy")
        import

@@ -3,7 +3,9 @@ k_axis_pair, k_axis_pair_q) against the oracle where its tiles and rules can go
 wrong: every kernel variant (bands, branches), meshes with three different
 lengths, odd ones and ones beyond 31 points (two row tiles), cells beyond 7 along an
 axis (four K steps), windows that leave lines short or empty, more than one round of
-work items, polar terms, mesh_ref 2, states of a k split over calls.  Counts exact, exact zeros
+work items, polar terms, mesh_ref 2, states of a k split over calls.  Every case runs in the
+form that the plan chose, which has to be this one (plan.form()), and as one product over all
+cells.  Counts exact, exact zeros
 equal, |g|^2 relative above 1e-6 * max within 1e-12 (FP64: sums of at most 1e3
 terms of one sign pattern, a few hundred units of 1.1e-16 after the cancellation
 the floor allows) and 1e-5 (mixed)."""
@@ -13,6 +15,7 @@ import numpy as np
 import pytest
 
 from elphbolt_amd import interactions, synth
+from elphbolt_amd._lib import ElphError
 from elphbolt_amd.wannier import Wannier
 from oracle import oracle as O
 
@@ -40,27 +43,6 @@ def _state(mat):
     el = O.Electrons(o, eye, 1, mat.wvmesh, mat.enref, mat.fsthick)
     ph = O.Phonons(o, eye, 1, mat.phmesh)
     return o, el, ph
-
-
-def _rows(el):
-    m = np.asarray(el.wvmesh)
-    i = np.asarray(el.indexlist) - 1
-    return np.stack([i % m[0], (i // m[0]) % m[1], i // (m[0] * m[1])], 1)
-
-
-def _takes_axis(cells, el, mixed):
-    """The dispatch's rule (axis_cost, axis_direct_cost) for these sizes."""
-    m, k = np.asarray(el.wvmesh), _rows(el)
-    npl, nl = len(set(k[:, 2])), len({(a, b) for a, b in k[:, 1:]})
-    c = np.asarray(cells)
-    rm, r1m = np.abs(c[:, 0]).max(), np.abs(c[:, 1]).max()
-    npair = (len(c) + 1) // 2  # symmetric sets pair up except R = 0
-    kp = -(-2 * npair // 64) * 64
-
-    def prod(n, r):
-        return 16.0 * ((n // 2 + 16) // 16) * (16.0 if r > 7 else 8.0) * 4.0
-    cost = 4.0 * npl * len(c) + npl * (2 * rm + 1) * prod(m[1], r1m) + nl * prod(m[0], rm)
-    return cost * (6.0 if mixed else 2.0) <= 2.0 * len(k) * kp
 
 
 # name, nb, nat, ws, mesh, bands in window, polar, precision
@@ -91,30 +73,33 @@ CASES = [
 def test_ibzk_axis(name, nb, nat, ws, mesh, biw, polar, precision):
     mat = _material(nb, nat, ws, mesh, biw, polar)
     o, el, ph = _state(mat)
-    assert _takes_axis(mat.rcells_q, el, precision == "mixed")
     plan = interactions.IbzkPlan(Wannier(mat), el, ph, precision=precision)
+    chosen = plan.form()
+    assert chosen == (True, precision == "fp64")
     # the in-window states of the first, a middle and the last k, over the first and last rows
     act = np.abs(el.ens_irred - el.enref) <= el.fsthick
     ks = np.nonzero(act.any(1))[0]
     nwin = (np.abs(el.ens - el.enref) <= el.fsthick).sum(1)
     offs = np.concatenate([[0], np.cumsum(nwin)]) * mat.nbr
     span = min(el.nwv, 48 if nb <= 8 else 20)
-    err = 0.0
+    err = {}
     for ik in sorted({int(ks[0]), int(ks[len(ks) // 2]), int(ks[-1])}):
         first, last = ik * nb + 1, (ik + 1) * nb
-        print(f"axis ibzk {name} {precision}: k {ik + 1}, {el.nwv} rows", flush=True)
-        c_g, g_g = plan.run(first, last)
-        for r0 in (0, el.nwv - span):
-            c_o, g_o, _ = O.ibzk_g2_window(o, el, ph, first, last, r0 + 1, span)
-            got = g_g[:, offs[r0]:offs[r0 + span]]
-            sel = c_o >= 0
-            assert np.array_equal(sel, c_g >= 0) and sel.any()
-            assert np.all(c_g[sel] == plan.nprocs)
-            ref = g_o[sel][:, :got.shape[1]]
-            assert np.array_equal(ref == 0.0, got[sel] == 0.0)
-            err = max(err, _rel(got[sel], ref))
-    print(f"  max rel {err:.2e}", flush=True)
-    assert err < (1e-12 if precision == "fp64" else 1e-5)
+        refs = [(r0, O.ibzk_g2_window(o, el, ph, first, last, r0 + 1, span)) for r0 in (0, el.nwv - span)]
+        for form in ((False, False), chosen):
+            print(f"axis ibzk {name} {precision}: k {ik + 1}, {el.nwv} rows, form {form}", flush=True)
+            assert plan.form(*form) == form
+            c_g, g_g = plan.run(first, last)
+            for r0, (c_o, g_o, _) in refs:
+                got = g_g[:, offs[r0]:offs[r0 + span]]
+                sel = c_o >= 0
+                assert np.array_equal(sel, c_g >= 0) and sel.any()
+                assert np.all(c_g[sel] == plan.nprocs)
+                ref = g_o[sel][:, :got.shape[1]]
+                assert np.array_equal(ref == 0.0, got[sel] == 0.0)
+                err[form] = max(err.get(form, 0.0), _rel(got[sel], ref))
+    print(f"  max rel {err}", flush=True)
+    assert max(err.values()) < (1e-12 if precision == "fp64" else 1e-5)
     # the same bits whatever states share a call
     one = plan.run(int(ks[0]) * nb + 1, int(ks[-1]) * nb + nb) if len(ks) < 40 else None
     if one is not None:
@@ -127,7 +112,6 @@ def test_ibzk_axis_mesh_ref2():
     interpolates), so both sides rotate with the same eigenvectors."""
     mat = _material(4, 2, [4, 4, 4], [14, 12, 10], 2.0, mesh_ref=2)
     o, el, ph = _state(mat)
-    assert _takes_axis(mat.rcells_q, el, False)
     w = Wannier(mat)
     mesh = np.asarray(mat.wvmesh)
     i = np.arange(int(np.prod(mesh)))
@@ -141,11 +125,15 @@ def test_ibzk_axis_mesh_ref2():
                                  indexlist_irred=np.arange(1, len(pts) + 1))
     last = 8
     c_o, g_o = O.ibzk_g2(o, el, fine, 1, 1, last)
-    c_g, g_g = interactions.IbzkPlan(w, el, ph, mesh_ref=2, precision="fp64").run(1, last)
-    assert np.array_equal(c_o, c_g) and (c_o >= 0).any()
+    plan = interactions.IbzkPlan(w, el, ph, mesh_ref=2, precision="fp64")
+    assert plan.form() == (True, True)
     act = c_o >= 0
-    assert np.array_equal(g_o[act] == 0.0, g_g[act] == 0.0)
-    assert _rel(g_g[act], g_o[act]) < 1e-12
+    for form in ((True, True), (False, False)):
+        assert plan.form(*form) == form
+        c_g, g_g = plan.run(1, last)
+        assert np.array_equal(c_o, c_g) and act.any()
+        assert np.array_equal(g_o[act] == 0.0, g_g[act] == 0.0)
+        assert _rel(g_g[act], g_o[act]) < 1e-12
 
 
 # name, nb, nat, ws, mesh, bands in window, polar
@@ -165,19 +153,22 @@ CASES_Q = [
 def test_ibzq_axis(name, nb, nat, ws, mesh, biw, polar):
     mat = _material(nb, nat, ws, mesh, biw, polar, seed=6)
     o, el, ph = _state(mat)
-    assert _takes_axis(mat.rcells_k, el, False)
     first = 3 * mat.nbr + 1  # past q = 0
     last = first + (mat.nbr if nb > 8 else 2 * mat.nbr) - 1
     print(f"axis ibzq {name}: states {first}..{last}, {el.nwv} rows", flush=True)
     c_o, g_o = O.ibzq_g2(o, el, ph, first, last)
-    c_g, g_g = interactions.IbzqPlan(Wannier(mat), el, ph).run(first, last)
-    assert np.array_equal(c_o, c_g) and c_o.max() > 0
-    err = 0.0
-    for t, n in enumerate(c_o):
-        assert np.array_equal(g_o[t, :n] == 0.0, g_g[t, :n] == 0.0)
-        err = max(err, _rel(g_g[t, :n], g_o[t, :n]))
-    print(f"  max rel {err:.2e}", flush=True)
-    assert err < 1e-12
+    plan = interactions.IbzqPlan(Wannier(mat), el, ph)
+    assert plan.form() == (True, True)
+    for form in ((True, True), (False, False)):
+        assert plan.form(*form) == form
+        c_g, g_g = plan.run(first, last)
+        assert np.array_equal(c_o, c_g) and c_o.max() > 0
+        err = 0.0
+        for t, n in enumerate(c_o):
+            assert np.array_equal(g_o[t, :n] == 0.0, g_g[t, :n] == 0.0)
+            err = max(err, _rel(g_g[t, :n], g_o[t, :n]))
+        print(f"  form {form}: max rel {err:.2e}", flush=True)
+        assert err < 1e-12
 
 
 @pytest.mark.parametrize("kind", ["ibzk", "ibzq"])
@@ -189,6 +180,7 @@ def test_many_points_per_pass(kind):
     _, el, ph = _state(mat)
     w = Wannier(mat)
     plan = (interactions.IbzkPlan if kind == "ibzk" else interactions.IbzqPlan)(w, el, ph)
+    assert plan.form() == (True, True)
     assert (el.nwv_irred if kind == "ibzk" else ph.nwv_irred) > 1024
     nst = (el if kind == "ibzk" else ph).nwv_irred * 3
     width = plan.nprocs if kind == "ibzk" else plan.stride
@@ -205,3 +197,16 @@ def test_many_points_per_pass(kind):
         else:
             for t, n in enumerate(c):
                 assert np.array_equal(got[t, :n], g[t, :n])
+
+
+def test_form_of_a_plan():
+    """A plan that does not have a form refuses it and keeps the one it has."""
+    mat = synth.tiny(nb=4, natoms=2, ws=3, wv=4, seed=12)  # the sums cost as much as the product
+    _, el, ph = _state(mat)
+    w = Wannier(mat)
+    plan = interactions.IbzkPlan(w, el, ph, precision="mixed")
+    assert plan.form() == (False, False)
+    for kw in (dict(pair=True), dict(points=True)):
+        with pytest.raises(ElphError):
+            plan.form(**kw)
+    assert plan.form(pair=False) == (False, False)
