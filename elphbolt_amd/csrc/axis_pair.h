@@ -8,7 +8,7 @@
 //   A  F1(q2; R0, R1) = sum_R2 e^{i 2 pi q2 R2 / N2} h(R)
 //   B  F2(q2, q1; R0) = sum_R1 e^{i 2 pi q1 R1 / N1} F1(q2; R0, R1)
 //   C  Y(q)           = sum_R0 e^{i 2 pi q0 R0 / N0} F2(q2, q1; R0)
-// (axis_cost counts the multiply-adds).  Axis 0 is the fastest index of the mesh,
+// (axis_time weighs them against the product).  Axis 0 is the fastest index of the mesh,
 // so the rows of one line (q1, q2) are consecutive rows of the driver's list and
 // their results one contiguous range of the output.  Three kernels:
 //   k_axis_rot   the band or branch rotation: h of the cells, in the order of the sums

@@ -3742,24 +3742,27 @@ int elph_selftest_mfma(int device, double *max_err) {
 namespace {
 
 // Kernel variant of the axis-by-axis form: bounds on nb and nbr (registers of an
-// item's U_k' row and g), in-window ranks per item.
+// item's U_k' row and g), in-window ranks per item, time of a round's band products
+// (ps each, axis_time) and how many times the later stages take at N0 > 31, whose second tile
+// of 16 q makes every variant spill.
 struct AxisTier {
     int id = -1, nbm = 0, ranks = 1;
+    double ps = 0, wide = 1;
 };
 AxisTier axis_tier(int64_t nb, int64_t nbr) {
-    if (nb <= 8 && nbr <= 6) return {0, 8, 2};
-    if (nb <= 8 && nbr <= 24) return {1, 8, 1};
-    if (nb <= 12 && nbr <= 12) return {2, 12, 1};
-    if (nb <= 16 && nbr <= 12) return {3, 16, 1};
-    if (nb <= 16 && nbr <= 24) return {4, 16, 1};
-    if (nb <= 32 && nbr <= 24) return {5, 32, 1};
+    if (nb <= 8 && nbr <= 6) return {0, 8, 2, 22.0, 4.0};
+    if (nb <= 8 && nbr <= 24) return {1, 8, 1, 47.0, 4.0};
+    if (nb <= 12 && nbr <= 12) return {2, 12, 1, 51.0, 4.0};
+    if (nb <= 16 && nbr <= 12) return {3, 16, 1, 70.0, 4.0};
+    if (nb <= 16 && nbr <= 24) return {4, 16, 1, 67.0, 4.0};
+    if (nb <= 32 && nbr <= 24) return {5, 32, 1, 85.0, 4.0};
     return {};
 }
 AxisTier axis_tier_q(int64_t nb) {
-    if (nb <= 8) return {0, 8, 2};
-    if (nb <= 12) return {1, 12, 1};
-    if (nb <= 16) return {2, 16, 1};
-    return nb <= 32 ? AxisTier{3, 32, 1} : AxisTier{};
+    if (nb <= 8) return {0, 8, 2, 33.0, 2.5};
+    if (nb <= 12) return {1, 12, 1, 75.0, 2.5};
+    if (nb <= 16) return {2, 16, 1, 60.0, 2.5};
+    return nb <= 32 ? AxisTier{3, 32, 1, 85.0, 2.5} : AxisTier{};
 }
 
 // The axis-by-axis form (axis_pair.h) of one driver: its tables on the device,
@@ -3781,30 +3784,61 @@ struct AxisPlan {
     }
 };
 
-// How many times cheaper (in multiply-adds) the axis sums must be than the direct
-// product: the axis kernels run at a smaller share of the FP64 rate than the fused FP64
-// product, and the int8 digit product does its multiply-adds several times faster than it.
-constexpr double kAxisMarginFp64 = 2.0, kAxisMarginMixed = 6.0;
+// The form of the pair stage is chosen by predicted time (ps per state, for a call of many),
+// fitted to both forms of 1588 plans on one card: meshes of 6 to 60 points along an axis, 93 to 617
+// cells, 4 to 26 bands, 3 to 24 branches, 0.3 to 5 bands in the window, both precisions.
+// Multiply-adds alone do not tell: where the axis form has a ninth of the int8 product's, it took twice
+// its time at N0 > 31 (40^3, 279 cells, 50 states: 0.63 against 1.26 ms); with many branches or bands
+// the epilogue outweighs the sums (17 bands, 9 branches, 14^3, 93 cells, mixed, 159 states: 1.71
+// against 2.11 ms); short lines leave lanes idle; and at 8 bands, 6 branches, 24^3 and 617 cells it takes
+// a sixth of the FP64 product's time.  The predicted ratio is off by 1.3 (one deviation, calls of 30
+// states and more), so the axis form has to promise 1.2: of the 1588, 7 are then more than 5% slower
+// than with the products alone (worst 0.81, a call of 2 states), 105 (worst 0.51) when it was
+// taken at 1/2 (FP64) and 1/6 (mixed) of the multiply-adds, and the mean gain is 1.50 against 1.47.
+constexpr double kAxisMargin = 1.2;
+// Stage A, then B and C by the elements of F2 and the epilogue by its products: `rounds` rounds of
+// 64 items with `work` band products per rank.
+double axis_time(const AxisTab &t, const AxisTier &k, int64_t n, int64_t rounds, double work) {
+    return 2.4 * (double)t.npl * n * t.CPs +
+           (t.N0 > 31 ? k.wide : 1.0) * (3.5 * (double)t.nl * (2 * t.rm + 1) * t.CPs + k.ps * (double)rounds * k.ranks * work);
+}
+// The direct product's constants: per row, cell-pair row and column, per row and column (Y through
+// memory on the column-tiled paths), and per multiply-add of the epilogue.
+struct DirectTime {
+    double product, column, epilogue;
+};
+double direct_time(const DirectTime &k, int64_t rows, int64_t Kp, int64_t CP, double epilogue) {
+    return (double)rows * CP * (k.product * Kp + k.column) + 30.0 * (double)Kp * CP + k.epilogue * epilogue;  // (30: folded operand)
+}
+// (shape: epilogue_class)
+DirectTime direct_ibzk(bool mixed, bool general, int shape) {
+    if (mixed) {
+        if (general) return {0.013, 14.5, 0.2};
+        return shape == 1 ? DirectTime{0.010, 4.8, 0.9} : (shape == 2 ? DirectTime{0.012, 0.0, 1.9} : DirectTime{0.018, 0.0, 5.1});
+    }
+    if (general) return {0.084, 14.0, 0.0};
+    return shape == 1 ? DirectTime{0.071, 5.0, 0.85} : (shape == 2 ? DirectTime{0.078, 8.2, 2.6} : DirectTime{0.05, 0.0, 6.0});
+}
+DirectTime direct_ibzq(bool general) { return {0.065, general ? 7.3 : 2.4, 2.5}; }
 
-// Real multiply-adds per column and state: the direct product over `rows` rows
-// and Kp cell-pair rows against the three axis sums (B and C in tiles of 16 q
-// and 4 R on the matrix cores).
-double axis_direct_cost(int64_t rows, int64_t Kp) { return 2.0 * (double)rows * (double)Kp; }
-double axis_cost(int64_t npl, int64_t nl, int64_t ncell, int64_t rm, int64_t r1m, int64_t N0, int64_t N1) {
-    auto prod = [](int64_t N, int64_t r) { return 16.0 * (double)((N / 2 + 16) / 16) * (r > 7 ? 16.0 : 8.0) * 4.0; };
-    return 4.0 * npl * ncell + (double)(npl * (2 * rm + 1)) * prod(N1, r1m) + (double)nl * prod(N0, rm);
+// Epilogue variant of the fused kernels: 1 for nb <= 8 and nbr <= 6, 2 for
+// nb <= 16 and nbr <= 12 (loops unrolled to those bounds), 0 otherwise.
+int epilogue_class(int64_t nb, int64_t nbr) {
+    if (nb <= 8 && nbr <= 6) return 1;
+    if (nb <= 16 && nbr <= 12) return 2;
+    return 0;
 }
 
 // Tables of the axis-by-axis form for `n` cells (column-major, leading dimension
 // ld) on the mesh N and the driver's rows (integer triplets).  nin / nout: inner and
-// outer column index counts; vals: results per in-window rank.  nwin, wband, offs
-// (ibzk): the rows' in-window bands and output offsets, for the list of work items; null
-// where the items depend on the state.  The form is taken (x.on) when its sums cost less
-// than 1 / `margin` of the direct product's, the rows are whole mesh lines in ascending
-// order and the sizes fit its kernels.
+// outer column index counts; vals: results per in-window rank.  nwin: the rows' in-window band
+// counts; wband, offs (ibzk): these bands and the rows' output offsets, for the list of work items;
+// null where the items depend on the state.  The form is taken (x.on) when its predicted time is
+// below the direct product's (`direct`, ps per state) by kAxisMargin, the rows ascend in mesh
+// order and the sizes fit its kernels.  work: axis_time.
 void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const int64_t *N, const std::vector<int> &rows,
-                int64_t nin, int64_t nout, int64_t nrot, int nb, int vals, AxisTier tier, const std::vector<int> *nwin,
-                const std::vector<int> *wband, const std::vector<int64_t> *offs, int64_t Kp, double margin, int64_t lds_max,
+                int64_t nin, int64_t nout, int64_t nrot, int nb, int vals, AxisTier tier, const std::vector<int> &nwin,
+                const std::vector<int> *wband, const std::vector<int64_t> *offs, double work, double direct, int64_t lds_max,
                 hipStream_t s) {
     x.on = false;
     const int64_t nwv = (int64_t)rows.size() / 3;
@@ -3858,7 +3892,6 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     }
     line_row.push_back((int)nwv);
     const int64_t npl = (int64_t)pl_k2.size(), nl = (int64_t)line_k.size();
-    if (axis_cost(npl, nl, n, rm, r1m, N[0], N[1]) * margin > axis_direct_cost(nwv, Kp)) return;
     std::vector<int> line_of(npl * N[1], -1);
     for (int64_t l = 0; l < nl; ++l) line_of[(line_k[l] >> 16) * N[1] + (line_k[l] & 0xffff)] = (int)l;
     // column tiles: whole inner ranges, as many per 16 columns as fit
@@ -3876,16 +3909,23 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     x.nbm = tier.nbm;
     x.vals = vals;
     x.nb = nb;
-    if (lds_max > 0 && (int64_t)std::max(x.lds_ab(), x.lds_c(nwin == nullptr)) > lds_max) return;
+    int64_t rounds = 0;
+    for (int64_t l = 0; l < nl; ++l) {
+        int64_t items = 0;
+        for (int r = line_row[l]; r < line_row[l + 1]; ++r) items += (nwin[r] + x.ranks - 1) / x.ranks;
+        rounds += (items + 63) / 64;
+    }
+    if (axis_time(t, tier, n, rounds, work) * kAxisMargin > direct) return;
+    if (lds_max > 0 && (int64_t)std::max(x.lds_ab(), x.lds_c(wband == nullptr)) > lds_max) return;
     std::vector<int> line_item;
     std::vector<int4> items;
-    if (nwin) {
+    if (wband) {
         if (!offs->empty() && offs->back() + (int64_t)nb * vals > 0x7fffffff) return;
         for (int64_t l = 0; l < nl; ++l) {
             line_item.push_back((int)items.size());
             for (int r = line_row[l]; r < line_row[l + 1]; ++r)
-                for (int j = 0; j < (*nwin)[r]; j += x.ranks) {
-                    const int nr = std::min(x.ranks, (*nwin)[r] - j), b0 = (*wband)[(int64_t)r * nb + j];
+                for (int j = 0; j < nwin[r]; j += x.ranks) {
+                    const int nr = std::min(x.ranks, nwin[r] - j), b0 = (*wband)[(int64_t)r * nb + j];
                     const int b1 = nr > 1 ? (*wband)[(int64_t)r * nb + j + 1] : b0;
                     items.push_back(make_int4(r, rows[3 * r] | nr << 8, b0 | b1 << 16, (int)((*offs)[r] + (int64_t)j * vals)));
                 }
@@ -3910,7 +3950,7 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     x.line_of.upload(line_of, s);
     x.line_k.upload(line_k, s);
     x.line_row.upload(line_row, s);
-    if (nwin) {
+    if (wband) {
         x.line_item.upload(line_item, s);
         x.items.upload(items, s);
     }
@@ -4541,14 +4581,6 @@ void pair_launch(elph_ibzk_plan *p, const IbzkGroup &gr, IbzkScratch &sc, hipStr
     if (timed) timed_end(c, s);
 }
 
-// Epilogue variant of the fused kernels: 1 for nb <= 8 and nbr <= 6, 2 for
-// nb <= 16 and nbr <= 12 (loops unrolled to those bounds), 0 otherwise.
-int epilogue_class(int64_t nb, int64_t nbr) {
-    if (nb <= 8 && nbr <= 6) return 1;
-    if (nb <= 16 && nbr <= 12) return 2;
-    return 0;
-}
-
 // Kernel shape of the fused pair stage of a plan: precision, column blocks,
 // epilogue class (FP64: the unrolled nb <= 16 form only where it keeps two
 // waves per SIMD, CB <= 2) and byte-packed phase indices (FP64).
@@ -5073,9 +5105,11 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         // context data
         if (precision == ELPH_MIXED) ensure_gwann_digits(ctx);
         {
-            axis_build(p->ax, ctx->rcells_q.data(), ctx->nwsq, ctx->nwsg, p->Nel, kpi, nb, nbr, nb, (int)nb, (int)nbr,
-                       axis_tier(nb, nbr), &nw, &wb, &offs, p->Kp, precision == ELPH_MIXED ? kAxisMarginMixed : kAxisMarginFp64,
-                       ctx->lds_max, s);
+            const double direct = direct_time(direct_ibzk(precision == ELPH_MIXED, p->general, epilogue_class(nb, nbr)), nwv, p->Kp,
+                                              p->CP, (double)total_win * nbr * (nb + nbr));
+            const AxisTier tier = axis_tier(nb, nbr);
+            axis_build(p->ax, ctx->rcells_q.data(), ctx->nwsq, ctx->nwsg, p->Nel, kpi, nb, nbr, nb, (int)nb, (int)nbr, tier, nw,
+                       &wb, &offs, (double)nbr * (tier.nbm + nbr), direct, ctx->lds_max, s);
             p->axis = p->ax.on;
             if (precision != ELPH_MIXED)
                 axis_cells_build(p->kcells, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, ctx->elwsdeg, p->Nel, s);
@@ -5893,8 +5927,11 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
             T[j] = make_double2(std::cos(x), std::sin(x));
         }
         p->T.upload(T, s);
-        axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb,
-                   axis_tier_q(nb), nullptr, nullptr, nullptr, p->Kp, kAxisMarginFp64, ctx->lds_max, s);
+        const double m = (double)total_win / (double)nwv;  // in-window bands per k
+        const AxisTier tier = axis_tier_q(nb);
+        axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb, tier, nw, nullptr,
+                   nullptr, tier.nbm * (nb + m), direct_time(direct_ibzq(p->general), nwv, p->Kp, p->CP, (double)total_win * nb * (nb + m)),
+                   ctx->lds_max, s);
         axis_cells_build(p->rcells, ctx->rcells_g.data(), ctx->nwsg, ctx->nwsg, ctx->gwsdeg, p->Nel, s);
         if (p->rcells.on && ctx->lds_max > 0 && (int64_t)axis_pts_lds(p->rcells, kPtsPlanes, 1024) > ctx->lds_max)
             p->rcells.on = false;

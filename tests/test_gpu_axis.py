@@ -50,17 +50,17 @@ CASES = [
     ("nb8_na2", 8, 2, [5, 5, 5], [14, 16, 9], 3.0, None, "fp64"),
     ("nb8_na2_mixed", 8, 2, [5, 5, 5], [14, 16, 8], 3.0, None, "mixed"),
     ("nb8_na2_wide", 8, 2, [4, 4, 4], [24, 7, 8], 7.5, None, "fp64"),    # more than 64 items on a line
-    ("nb7_na2_narrow", 7, 2, [5, 5, 5], [14, 16, 9], 0.4, None, "fp64"),  # short and missing lines
+    ("nb7_na2_narrow", 7, 2, [6, 6, 6], [14, 16, 9], 0.4, None, "fp64"),  # short and missing lines
     ("nb3_na1", 3, 1, [4, 4, 4], [11, 13, 10], 1.5, None, "fp64"),
     ("nb8_na2_polar", 8, 2, [5, 5, 5], [13, 12, 9], 3.0, "sic", "fp64"),
     ("nb5_na3", 5, 3, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
-    ("nb5_na3_polar_mixed", 5, 3, [5, 5, 5], [15, 20, 12], 2.0, "random", "mixed"),
+    ("nb5_na3_polar_mixed", 5, 3, [7, 7, 7], [24, 20, 12], 2.0, "random", "mixed"),
     ("nb11_na3", 11, 3, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
     ("nb13_na4", 13, 4, [4, 4, 4], [12, 11, 9], 2.0, None, "fp64"),
     ("nb16_na5_polar", 16, 5, [4, 4, 4], [12, 11, 8], 2.0, "random", "fp64"),
     ("nb19_na2", 19, 2, [4, 4, 4], [12, 11, 8], 2.0, None, "fp64"),
-    ("nb26_na8", 26, 8, [4, 4, 4], [12, 11, 8], 1.0, None, "fp64"),
-    ("n0_34", 4, 2, [4, 4, 4], [34, 6, 6], 2.0, None, "fp64"),
+    ("nb26_na8", 26, 8, [4, 4, 4], [24, 11, 8], 1.0, None, "fp64"),
+    ("n0_34", 4, 2, [5, 5, 5], [34, 6, 6], 2.0, None, "fp64"),
     ("n1_33", 4, 2, [4, 4, 4], [12, 33, 4], 2.0, None, "fp64"),
     ("n0_62_n1_61", 2, 1, [5, 5, 5], [62, 61, 2], 1.0, None, "fp64"),
     ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None, "fp64"),
@@ -143,8 +143,8 @@ CASES_Q = [
     ("nb8_na1_wide", 8, 1, [4, 4, 4], [24, 7, 8], 7.5, None),
     ("nb11_na2_polar", 11, 2, [4, 4, 4], [12, 11, 9], 2.0, "sic"),
     ("nb14_na1", 14, 1, [4, 4, 4], [12, 11, 9], 2.0, None),
-    ("nb19_na1", 19, 1, [4, 4, 4], [12, 11, 8], 2.0, None),
-    ("n0_35_n1_33", 4, 1, [4, 4, 4], [35, 33, 2], 1.5, None),
+    ("nb19_na1", 19, 1, [4, 4, 4], [24, 11, 8], 2.0, None),
+    ("n0_35_n1_33", 4, 1, [5, 5, 5], [35, 33, 2], 1.5, None),
     ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None),
 ]
 
@@ -176,7 +176,7 @@ def test_many_points_per_pass(kind):
     """More IBZ points than one pass of the mesh-point sum takes (1024), more than its
     8 planes and 64 lines at a time: a run into device rows, which takes the large
     groups, gives the bits of runs into host rows, which take groups of 64."""
-    mat = _material(3, 1, [4, 4, 4], [14, 16, 9], 1.5)
+    mat = _material(3, 1, [5, 5, 5], [14, 16, 9], 1.5)
     _, el, ph = _state(mat)
     w = Wannier(mat)
     plan = (interactions.IbzkPlan if kind == "ibzk" else interactions.IbzqPlan)(w, el, ph)
@@ -197,6 +197,24 @@ def test_many_points_per_pass(kind):
         else:
             for t, n in enumerate(c):
                 assert np.array_equal(got[t, :n], g[t, :n])
+
+
+# kind, nb, nat, ws, mesh, bands in window, precision: the axis sums have 1/10, 1/2.2, 1/2.8 of the
+# product's multiply-adds, and took longer on plans of these shapes (second tile of q; branches; short lines)
+SLOWER = [
+    ("ibzk", 15, 1, [4, 4, 4], [60, 8, 8], 4.0, "mixed"),
+    ("ibzk", 17, 5, [4, 4, 4], [6, 21, 15], 2.2, "fp64"),
+    ("ibzk", 8, 1, [5, 5, 5], [35, 12, 10], 0.3, "fp64"),
+    ("ibzq", 20, 2, [4, 4, 4], [7, 18, 8], 3.3, "fp64"),
+]
+
+
+@pytest.mark.parametrize("kind,nb,nat,ws,mesh,biw,precision", SLOWER, ids=[f"{c[0]}_nb{c[1]}_n0_{c[4][0]}" for c in SLOWER])
+def test_product_kept_where_it_is_faster(kind, nb, nat, ws, mesh, biw, precision):
+    mat = _material(nb, nat, ws, mesh, biw)
+    _, el, ph = _state(mat)
+    plan = (interactions.IbzkPlan if kind == "ibzk" else interactions.IbzqPlan)(Wannier(mat), el, ph, precision=precision)
+    assert not plan.form()[0]
 
 
 def test_form_of_a_plan():
