@@ -4057,10 +4057,17 @@ double2 axis_root(int64_t j, int64_t n) {
     const double a = kTwoPi * (double)fmodulo(j, n) / (double)n;
     return make_double2(std::cos(a), std::sin(a));
 }
+// Cells from which the mesh-point sum goes axis by axis.  Its cost per column tile (two barriers,
+// the line sums of few lines) does not shrink with the cells, and with 93 cells 37 of its 64 pair slots
+// work, while the product's one pass serves up to 64 k or 128 q: at 93 cells and up to 64 points the axis
+// sum takes 1.2 to 1.4 times the product's time (22 bands, 18 branches, 18 k: 0.79 against 1.34 ms), at
+// 165 cells 0.9, at 279 0.7 and at 617 0.6 (medians over 24 to 74 plans each, 1 to 64 points).
+// It is a rule on the plan, not on a call's points: rows keep their bits however states share calls.
+constexpr int64_t kAxisPtsCells = 150;
 void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n, const std::vector<int64_t> &deg,
                       const int64_t *N, hipStream_t s) {
     x.on = false;
-    if (n == 0 || n > 0x7fff || N[0] > 255 || N[1] > 0x7fff || N[2] > 0x7fff) return;
+    if (n < kAxisPtsCells || n > 0x7fff || N[0] > 255 || N[1] > 0x7fff || N[2] > 0x7fff) return;
     std::vector<int> order(n);
     std::iota(order.begin(), order.end(), 0);
     auto R = [&](int i, int d) { return cells[i + ld * d]; };
