@@ -3936,6 +3936,7 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
         const double a = kTwoPi * (double)fmodulo(j, m) / (double)m;
         return make_double2(std::cos(a), std::sin(a));
     };
+    if (N[2] * ne > (int64_t)1 << 24) return;  // 256 MiB of phases
     std::vector<double2> phA(N[2] * ne, make_double2(0.0, 0.0)), T0(N[0]), T1(N[1]), T2(N[2]);
     for (int64_t j = 0; j < N[0]; ++j) T0[j] = root(j, N[0]);
     for (int64_t j = 0; j < N[1]; ++j) T1[j] = root(j, N[1]);
@@ -3977,15 +3978,33 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
 // workgroups share it (24^3, 6 branches: 79.5 KB, 6.08 -> 5.21 ms; one workgroup per CU would halve the
 // waves that hide each other's latency).
 constexpr size_t kAxisUldsMax = 80 << 10;
-// The forms that a plan has (pair, pts) and takes (axis, axis_pts): elph_ibzk_plan_form.
-int axis_choice(int32_t want, bool pair, bool pts, bool &axis, bool &axis_pts, int32_t *form) {
+// The forms that a plan has (pair, pts) and takes (axis, axis_pts, small): elph_ibzk_plan_form.
+int axis_choice(int32_t want, bool pair, bool pts, bool &axis, bool &axis_pts, bool &small, int32_t *form) {
     if (want >= 0) {
-        if (want > 3 || ((want & ELPH_FORM_AXIS_PAIR) && !pair) || ((want & ELPH_FORM_AXIS_POINTS) && !pts)) return ELPH_EINVAL;
+        if (want > 7 || ((want & ELPH_FORM_AXIS_PAIR) && !pair) || ((want & ELPH_FORM_AXIS_POINTS) && !pts)) return ELPH_EINVAL;
         axis = (want & ELPH_FORM_AXIS_PAIR) != 0;
         axis_pts = (want & ELPH_FORM_AXIS_POINTS) != 0;
+        small = (want & ELPH_FORM_SMALL) != 0;
     }
-    if (form) *form = (axis ? ELPH_FORM_AXIS_PAIR : 0) | (axis_pts ? ELPH_FORM_AXIS_POINTS : 0);
+    if (form) *form = (axis ? ELPH_FORM_AXIS_PAIR : 0) | (axis_pts ? ELPH_FORM_AXIS_POINTS : 0) | (small ? ELPH_FORM_SMALL : 0);
     return ELPH_OK;
+}
+
+// Runs `go`, and where the device has no room for its buffers, again with less (the plan keeps the
+// choice): small groups and chunks, then the direct product (F2 of a single state may be the larger).
+template <typename Go, typename Free>
+void with_room(bool &axis, bool &small, Go &&go, Free &&free_buffers) {
+    while (true) {
+        try {
+            go();
+            return;
+        } catch (const Error &e) {
+            if (e.code != ELPH_ENOMEM || (small && !axis)) throw;
+            if (small) axis = false;
+            else small = true;
+        }
+        free_buffers();
+    }
 }
 
 // States per chunk of the axis path for nst states: h and F2 of a chunk within `cap`
@@ -4304,6 +4323,7 @@ struct IbzkGroup {
     DBuf<int> kst;              // [nkb + 1] first state of each k
     std::vector<int> kst_host;
     AxisPts pts;                // the k by planes and lines (axis form of the Re sum)
+    bool axis_pts = false;      // (which the group takes)
     DBuf<int64_t> st_slot;
 };
 
@@ -4312,6 +4332,17 @@ struct IbzkScratch {
     DBuf<double2> gk, h, phiT, Y, F2;
     DBuf<v4i> bphi, bsl;
     DBuf<double> bscale, hmax;
+    void release() {
+        gk.release();
+        h.release();
+        phiT.release();
+        Y.release();
+        F2.release();
+        bphi.release();
+        bsl.release();
+        bscale.release();
+        hmax.release();
+    }
 };
 
 }  // namespace
@@ -4354,6 +4385,7 @@ struct elph_ibzk_plan {
     DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
     AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 plans) where kcells.on; `axis_pts`
     bool axis_pts = false;  // says whether runs take it
+    bool small = false;     // groups of one launch of the direct Re contraction, chunks of its operand's size
     TablePack tables;       // the groups' tables of the running call
     HostBuf tables_host;
     DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
@@ -4391,7 +4423,8 @@ int64_t general_chunk(const elph_ibzk_plan *p, int64_t nst) {
 }
 
 int64_t axis_chunk(const elph_ibzk_plan *p, int64_t nst) {
-    return axis_chunk(p->ax, nst, p->y_bytes_cap > 0 ? p->y_bytes_cap : kAxisChunkBytes);
+    const int64_t most = p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes;
+    return axis_chunk(p->ax, nst, p->y_bytes_cap > 0 ? p->y_bytes_cap : most);
 }
 
 // Axis-by-axis path, a chunk of states at a time.
@@ -4792,7 +4825,8 @@ void ibzk_group_pack(const elph_ibzk_plan *p, GroupHost &h, IbzkGroup &g, TableP
     t.add(h.ski, g.st_kint);
     t.add(h.kst, g.kst);
     g.kst_host = h.kst;
-    if (p->axis_pts) {
+    g.axis_pts = p->axis_pts;
+    if (g.axis_pts) {
         h.pts = axis_pts_host(p->kcells, h.kint);
         g.pts.pack(h.pts, t);
     }
@@ -4814,7 +4848,7 @@ void ibzk_groups(elph_ibzk_plan *p, int64_t first, int64_t last, bool on_device,
                  std::vector<std::unique_ptr<IbzkGroup>> &groups, TablePack &tables, HostBuf *pinned, bool compact = false) {
     // IBZ k per group: the k of one launch of the Re contraction
     // (rows staged for the host, and the direct product's operand, bound a group at the smaller size)
-    const int64_t KB = p->axis_pts && p->axis && on_device
+    const int64_t KB = p->axis_pts && p->axis && on_device && !p->small
                            ? axis_pts_max(p->nb * p->nb * p->nbr * p->ctx->nwsg * (int64_t)sizeof(double2))
                            : (p->precision == ELPH_MIXED ? kGkKTMixed : kGkKT);
     std::vector<GroupHost> hosts = ibzk_group_hosts(p, first, last, on_device, counts, compact, KB);
@@ -4833,7 +4867,7 @@ void ibzk_scratch(const elph_ibzk_plan *p, IbzkScratch &sc, int64_t nkb, int64_t
     elph_ctx *c = p->ctx;
     const int64_t nb2 = p->nb * p->nb, nslices = p->nbr * c->nwsg;
     get(sc.gk, nkb * nb2 * nslices);
-    get(sc.phiT, gk_phi_count(c));
+    if (!p->axis_pts) get(sc.phiT, gk_phi_count(c));
     if (p->precision == ELPH_MIXED) get(sc.bphi, gk_bphi_count(c));
     if (p->axis) {
         get(sc.h, axis_chunk(p, nst) * p->ax.h_state());
@@ -4874,7 +4908,7 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
 void ibzk_prep(elph_ibzk_plan *p, const IbzkGroup &g, IbzkScratch &sc, hipStream_t s) {
     elph_ctx *c = p->ctx;
     const int64_t nb = p->nb, nbr = p->nbr, nb2 = nb * nb, nslices = nbr * c->nwsg;
-    if (p->axis_pts) {
+    if (g.axis_pts) {
         AxisPtsArgs a{};
         a.g = c->gwann.p;
         a.cstride = nb2;
@@ -5111,19 +5145,17 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         // the int8 digits of gwann, once per context, so that runs allocate no
         // context data
         if (precision == ELPH_MIXED) ensure_gwann_digits(ctx);
-        {
+        try {
             const double direct = direct_time(direct_ibzk(precision == ELPH_MIXED, p->general, epilogue_class(nb, nbr)), nwv, p->Kp,
                                               p->CP, (double)total_win * nbr * (nb + nbr));
             const AxisTier tier = axis_tier(nb, nbr);
             axis_build(p->ax, ctx->rcells_q.data(), ctx->nwsq, ctx->nwsg, p->Nel, kpi, nb, nbr, nb, (int)nb, (int)nbr, tier, nw,
                        &wb, &offs, (double)nbr * (tier.nbm + nbr), direct, ctx->lds_max, s);
-            p->axis = p->ax.on;
             if (precision != ELPH_MIXED)
                 axis_cells_build(p->kcells, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, ctx->elwsdeg, p->Nel, s);
             if (p->kcells.on && ctx->lds_max > 0 &&
                 (int64_t)axis_pts_lds(p->kcells, kPtsPlanes, 1024) > ctx->lds_max)
                 p->kcells.on = false;
-            p->axis_pts = p->kcells.on;
             if (p->ax.on) {
                 auto transposed = [&](const std::vector<double2> &v, DBuf<double2> &dst) {
                     std::vector<double2> w(v.size());
@@ -5147,7 +5179,12 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
                     weights(omf_host, p->wfT);
                 }
             }
+        } catch (const Error &e) {
+            if (e.code != ELPH_ENOMEM) throw;
+            p->ax.on = p->kcells.on = false;  // no room for the tables: the products do without
         }
+        p->axis = p->ax.on;
+        p->axis_pts = p->kcells.on;
         // IBZ data
         p->kint_irr.resize(3 * p->nirr);
         p->ens_irred.assign(el->ens_irred, el->ens_irred + p->nirr * nb);
@@ -5174,7 +5211,7 @@ int64_t elph_ibzk_plan_nprocs(const elph_ibzk_plan *p) { return p ? p->nprocs : 
 
 int elph_ibzk_plan_form(elph_ibzk_plan *p, int32_t want, int32_t *form) {
     if (!p) return ELPH_EINVAL;
-    return axis_choice(want, p->ax.on, p->kcells.on, p->axis, p->axis_pts, form);
+    return axis_choice(want, p->ax.on, p->kcells.on, p->axis, p->axis_pts, p->small, form);
 }
 
 int elph_ibzk_plan_destroy(elph_ibzk_plan *p) {
@@ -5193,16 +5230,25 @@ int elph_ibzk_plan_run(elph_ibzk_plan *p, int64_t first, int64_t last, int64_t *
         c->t_dominant_ms = 0;
         c->n_dominant = 0;
         c->tev_used = 0;
-        std::vector<std::unique_ptr<IbzkGroup>> groups;
-        ibzk_groups(p, first, last, on_device != 0, counts, s, groups, p->tables, &p->tables_host);
-        int64_t nkb = 1, nst = 1;
-        for (auto &g : groups) {
-            nkb = std::max(nkb, g->nkb);
-            nst = std::max(nst, g->nst);
-        }
         if (p->precision == ELPH_MIXED) ensure_gwann_digits(c);
-        ibzk_reserve(p, p->scr, nkb, nst);
-        if (!on_device) p->g2stage.alloc(nst * p->nprocs);
+        std::vector<std::unique_ptr<IbzkGroup>> groups;
+        with_room(
+            p->axis, p->small,
+            [&] {
+                groups.clear();
+                ibzk_groups(p, first, last, on_device != 0, counts, s, groups, p->tables, &p->tables_host);
+                int64_t nkb = 1, nst = 1;
+                for (auto &g : groups) {
+                    nkb = std::max(nkb, g->nkb);
+                    nst = std::max(nst, g->nst);
+                }
+                ibzk_reserve(p, p->scr, nkb, nst);
+                if (!on_device) p->g2stage.alloc(nst * p->nprocs);
+            },
+            [&] {
+                HCHECK(hipStreamSynchronize(s));  // (the tables' copy)
+                p->scr.release();
+            });
         HCHECK(hipEventRecord(c->ev_c, s));
         for (auto &g : groups) {
             ibzk_enqueue(p, *g, p->scr, s, on_device ? g2 : p->g2stage.p, true);
@@ -5493,6 +5539,103 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
     return r;
 }
 
+// The groups of an item's plan as its form now has them (again after a change of the form).
+void batch_groups(elph_batch *b, elph_batch::Item &it, int64_t *counts) {
+    it.groups.clear();
+    ibzk_groups(it.p, it.first, it.last, true, counts, b->streams[0], it.groups, *it.tables, nullptr, true);
+}
+
+// Size classes, streams and buffers of the batch's plans; allocates all that its graph needs.
+void batch_plan(elph_batch *b, bool autotune_tiles) {
+    b->classes.clear();
+    // size classes: (precision, bucket of nb*nbr, bucket of Kp)
+    std::map<std::tuple<int, int, int>, int> key2cls;
+    for (auto &it : b->items) {
+        if (it.groups.empty()) continue;
+        const auto key = std::make_tuple((int)it.p->precision, col_bucket(it.p->CPf), kp_bucket(it.p->Kp));
+        auto f = key2cls.find(key);
+        if (f == key2cls.end()) {
+            elph_batch::Class c;
+            c.precision = it.p->precision;
+            c.cb = std::get<1>(key);
+            c.kb = std::get<2>(key);
+            c.rep = autotune(b, it, b->streams[0], autotune_tiles != 0);
+            c.axis = it.p->axis;
+            key2cls[key] = (int)b->classes.size();
+            b->classes.push_back(c);
+            f = key2cls.find(key);
+        } else {
+            // plans of the axis-by-axis form keep it; the others take the class's
+            // tile shape where one was timed, else the plan's own
+            const elph_batch_class_t &r = b->classes[f->second].rep;
+            if (!it.p->axis && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
+        }
+        it.cls = f->second;
+        b->classes[f->second].members += 1;
+        b->classes[f->second].rep.members = b->classes[f->second].members;
+    }
+    // longest work first onto the least-loaded stream
+    std::vector<size_t> order(b->items.size());
+    std::iota(order.begin(), order.end(), 0);
+    std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return b->items[x].work > b->items[y].work; });
+    std::vector<double> load(b->streams.size(), 0.0);
+    for (size_t i : order) {
+        const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        b->items[i].stream = s;
+        load[s] += b->items[i].work;
+    }
+    for (auto &it : b->items)
+        for (auto &g : it.groups) ibzk_reserve(it.p, *b->scr[it.stream], g->nkb, g->nst);
+    // fused path: per-group operand buffers and the work lists of the
+    // multi-material launches (one per kernel shape)
+    std::map<FusedShape, size_t> shape2list;
+    b->lists.clear();
+    for (auto &it : b->items) {
+        it.ops.clear();
+        if (it.p->general || it.p->axis) continue;
+        elph_ibzk_plan *p = it.p;
+        const FusedShape f = fused_shape(p);
+        auto fl = shape2list.find(f);
+        if (fl == shape2list.end()) {
+            auto jl = std::make_unique<elph_batch::JobList>();
+            jl->shape = f;
+            jl->ncu = (int)p->ctx->ncu;
+            fl = shape2list.emplace(f, b->lists.size()).first;
+            b->lists.push_back(std::move(jl));
+        }
+        elph_batch::JobList &jl = *b->lists[fl->second];
+        jl.lds = std::max(jl.lds, fused_lds(p));
+        const int nrb = (int)((p->nwv + fused_rows(p->precision) - 1) / fused_rows(p->precision));
+        for (auto &g : it.groups) {
+            auto o = std::make_unique<elph_batch::Item::Ops>();
+            IbzkScratch view;
+            if (p->precision == ELPH_MIXED) {
+                o->bsl.alloc((size_t)g->nst * p->nkc * (p->CP / 16) * 2 * kNS * 64);
+                o->bscale.alloc((size_t)g->nst * p->CP);
+                view.bsl.borrow(o->bsl.p, o->bsl.n);
+                view.bscale.borrow(o->bscale.p, o->bscale.n);
+            } else {
+                o->h.alloc((size_t)g->nst * p->Kp * p->CP);
+                view.h.borrow(o->h.p, o->h.n);
+            }
+            PairJob j{};
+            j.a = pair_args(p, *g, view, it.out);
+            j.Tdig = p->Tdig.p;
+            j.Rpk = p->Rpk.p;
+            j.bsl = view.bsl.p;
+            j.bscale = view.bscale.p;
+            j.nkc = (int)p->nkc;
+            j.nrb = nrb;
+            j.tile0 = jl.ntiles;
+            jl.ntiles += g->nst * nrb;
+            if (g->nst > 0) jl.host.push_back(j);
+            it.ops.push_back(std::move(o));
+        }
+    }
+    for (auto &jl : b->lists) jl->dev.upload(jl->host, b->streams[0]);
+    HCHECK(hipDeviceSynchronize());
+}
+
 }  // namespace
 
 extern "C" {
@@ -5544,7 +5687,7 @@ int elph_batch_add(elph_batch *b, elph_ibzk_plan *plan, int64_t first, int64_t l
         it.last = last;
         it.out = g2_device;
         it.tables = std::make_unique<TablePack>();
-        ibzk_groups(plan, first, last, true, counts, b->streams[0], it.groups, *it.tables, nullptr, true);
+        batch_groups(b, it, counts);
         int64_t nst = 0;
         for (auto &g : it.groups) nst += g->nst;
         it.work = (double)nst * plan->nwv * plan->Kp * plan->nb * plan->nbr;
@@ -5561,92 +5704,29 @@ int elph_batch_prepare(elph_batch *b, int32_t autotune_tiles) {
     if (!b) return ELPH_EINVAL;
     try {
         HCHECK(hipSetDevice(b->device));
-        // size classes: (precision, bucket of nb*nbr, bucket of Kp)
-        std::map<std::tuple<int, int, int>, int> key2cls;
+        bool axis = false, small = true;
+        std::vector<int64_t> counts;  // (the caller has them from elph_batch_add)
+        auto regroup = [&](elph_batch::Item &it) {
+            counts.resize(it.last - it.first + 1);
+            batch_groups(b, it, counts.data());
+        };
         for (auto &it : b->items) {
-            if (it.groups.empty()) continue;
-            const auto key = std::make_tuple((int)it.p->precision, col_bucket(it.p->CPf), kp_bucket(it.p->Kp));
-            auto f = key2cls.find(key);
-            if (f == key2cls.end()) {
-                elph_batch::Class c;
-                c.precision = it.p->precision;
-                c.cb = std::get<1>(key);
-                c.kb = std::get<2>(key);
-                c.rep = autotune(b, it, b->streams[0], autotune_tiles != 0);
-                c.axis = it.p->axis;
-                key2cls[key] = (int)b->classes.size();
-                b->classes.push_back(c);
-                f = key2cls.find(key);
-            } else {
-                // plans of the axis-by-axis form keep it; the others take the class's
-                // tile shape where one was timed, else the plan's own
-                const elph_batch_class_t &r = b->classes[f->second].rep;
-                if (!it.p->axis && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
-            }
-            it.cls = f->second;
-            b->classes[f->second].members += 1;
-            b->classes[f->second].rep.members = b->classes[f->second].members;
+            if (!it.groups.empty() && it.groups[0]->axis_pts != it.p->axis_pts) regroup(it);
+            axis = axis || it.p->axis;
+            small = small && it.p->small;
         }
-        // longest work first onto the least-loaded stream
-        std::vector<size_t> order(b->items.size());
-        std::iota(order.begin(), order.end(), 0);
-        std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return b->items[x].work > b->items[y].work; });
-        std::vector<double> load(b->streams.size(), 0.0);
-        for (size_t i : order) {
-            const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-            b->items[i].stream = s;
-            load[s] += b->items[i].work;
-        }
-        for (auto &it : b->items)
-            for (auto &g : it.groups) ibzk_reserve(it.p, *b->scr[it.stream], g->nkb, g->nst);
-        // fused path: per-group operand buffers and the work lists of the
-        // multi-material launches (one per kernel shape)
-        std::map<FusedShape, size_t> shape2list;
-        b->lists.clear();
-        for (auto &it : b->items) {
-            it.ops.clear();
-            if (it.p->general || it.p->axis) continue;
-            elph_ibzk_plan *p = it.p;
-            const FusedShape f = fused_shape(p);
-            auto fl = shape2list.find(f);
-            if (fl == shape2list.end()) {
-                auto jl = std::make_unique<elph_batch::JobList>();
-                jl->shape = f;
-                jl->ncu = (int)p->ctx->ncu;
-                fl = shape2list.emplace(f, b->lists.size()).first;
-                b->lists.push_back(std::move(jl));
-            }
-            elph_batch::JobList &jl = *b->lists[fl->second];
-            jl.lds = std::max(jl.lds, fused_lds(p));
-            const int nrb = (int)((p->nwv + fused_rows(p->precision) - 1) / fused_rows(p->precision));
-            for (auto &g : it.groups) {
-                auto o = std::make_unique<elph_batch::Item::Ops>();
-                IbzkScratch view;
-                if (p->precision == ELPH_MIXED) {
-                    o->bsl.alloc((size_t)g->nst * p->nkc * (p->CP / 16) * 2 * kNS * 64);
-                    o->bscale.alloc((size_t)g->nst * p->CP);
-                    view.bsl.borrow(o->bsl.p, o->bsl.n);
-                    view.bscale.borrow(o->bscale.p, o->bscale.n);
-                } else {
-                    o->h.alloc((size_t)g->nst * p->Kp * p->CP);
-                    view.h.borrow(o->h.p, o->h.n);
-                }
-                PairJob j{};
-                j.a = pair_args(p, *g, view, it.out);
-                j.Tdig = p->Tdig.p;
-                j.Rpk = p->Rpk.p;
-                j.bsl = view.bsl.p;
-                j.bscale = view.bscale.p;
-                j.nkc = (int)p->nkc;
-                j.nrb = nrb;
-                j.tile0 = jl.ntiles;
-                jl.ntiles += g->nst * nrb;
-                if (g->nst > 0) jl.host.push_back(j);
-                it.ops.push_back(std::move(o));
-            }
-        }
-        for (auto &jl : b->lists) jl->dev.upload(jl->host, b->streams[0]);
-        HCHECK(hipDeviceSynchronize());
+        with_room(axis, small, [&] { batch_plan(b, autotune_tiles != 0); },
+                  [&] {
+                      HCHECK(hipDeviceSynchronize());
+                      for (auto &sc : b->scr) sc->release();
+                      b->lists.clear();
+                      for (auto &it : b->items) {
+                          it.ops.clear();
+                          it.p->small = true;
+                          it.p->axis = it.p->axis && axis;
+                          regroup(it);
+                      }
+                  });
         // capture: fork from stream 0; every stream first prepares its fused
         // items' groups (event `prepped`), then runs its column-tiled items;
         // the multi-material pair launches run on lstream once every stream's
@@ -5831,7 +5911,7 @@ struct elph_ibzq_plan {
     AxisPlan ax;
     DBuf<double2> F2;
     AxisCells rcells;
-    bool axis = false, axis_pts = false;
+    bool axis = false, axis_pts = false, small = false;
     AxisPts pts;
     TablePack tables;      // the tables of the running batch of q
     HostBuf tables_host;
@@ -5936,12 +6016,17 @@ int elph_ibzq_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
         p->T.upload(T, s);
         const double m = (double)total_win / (double)nwv;  // in-window bands per k
         const AxisTier tier = axis_tier_q(nb);
-        axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb, tier, nw, nullptr,
-                   nullptr, tier.nbm * (nb + m), direct_time(direct_ibzq(p->general), nwv, p->Kp, p->CP, (double)total_win * nb * (nb + m)),
-                   ctx->lds_max, s);
-        axis_cells_build(p->rcells, ctx->rcells_g.data(), ctx->nwsg, ctx->nwsg, ctx->gwsdeg, p->Nel, s);
-        if (p->rcells.on && ctx->lds_max > 0 && (int64_t)axis_pts_lds(p->rcells, kPtsPlanes, 1024) > ctx->lds_max)
-            p->rcells.on = false;
+        try {
+            axis_build(p->ax, ctx->rcells_k.data(), ctx->nwsk, ctx->nwsk, p->Nel, ki, nb, nb, nbr, (int)nb, (int)nb, tier, nw, nullptr,
+                       nullptr, tier.nbm * (nb + m), direct_time(direct_ibzq(p->general), nwv, p->Kp, p->CP, (double)total_win * nb * (nb + m)),
+                       ctx->lds_max, s);
+            axis_cells_build(p->rcells, ctx->rcells_g.data(), ctx->nwsg, ctx->nwsg, ctx->gwsdeg, p->Nel, s);
+            if (p->rcells.on && ctx->lds_max > 0 && (int64_t)axis_pts_lds(p->rcells, kPtsPlanes, 1024) > ctx->lds_max)
+                p->rcells.on = false;
+        } catch (const Error &e) {
+            if (e.code != ELPH_ENOMEM) throw;
+            p->ax.on = p->rcells.on = false;
+        }
         p->axis = p->ax.on;
         p->axis_pts = p->rcells.on;
         p->nirr_q = ph->nwv_irred;
@@ -5961,7 +6046,7 @@ int64_t elph_ibzq_plan_stride(const elph_ibzq_plan *p) { return p ? p->stride : 
 
 int elph_ibzq_plan_form(elph_ibzq_plan *p, int32_t want, int32_t *form) {
     if (!p) return ELPH_EINVAL;
-    return axis_choice(want, p->ax.on, p->rcells.on, p->axis, p->axis_pts, form);
+    return axis_choice(want, p->ax.on, p->rcells.on, p->axis, p->axis_pts, p->small, form);
 }
 
 int elph_ibzq_plan_destroy(elph_ibzq_plan *p) {
@@ -5982,11 +6067,11 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
         c->n_dominant = 0;
         HCHECK(hipEventRecord(c->ev_c, s));
         const int64_t gblk = nb2 * nbr * c->nwsk;
-        // IBZ q per pass over gwann
-        const int64_t QB = p->axis_pts && p->axis && on_device ? axis_pts_max(gblk * (int64_t)sizeof(double2)) : 16 * kGReqNCB;
-        int64_t istate = first;
-        while (istate <= last) {
-            // states of up to QB distinct IBZ q
+        // the states of up to QB distinct IBZ q from istate on; returns the next one
+        auto batch = [&](const int64_t istate) {
+            // IBZ q per pass over gwann
+            const int64_t QB =
+                p->axis_pts && p->axis && on_device && !p->small ? axis_pts_max(gblk * (int64_t)sizeof(double2)) : 16 * kGReqNCB;
             std::vector<int64_t> qs, sts;
             int64_t j = istate;
             for (; j <= last; ++j) {
@@ -6131,7 +6216,8 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             const bool packed = p->L <= 255 && p->Nel[0] <= 255 && p->Nel[1] <= 255 && p->Nel[2] <= 255;
             auto axis = [&]() {
                 const AxisTab &t = p->ax.t;
-                const int64_t chunk = axis_chunk(p->ax, nst, kAxisChunkBytes);
+                const int64_t chunk =
+                    axis_chunk(p->ax, nst, p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes);
                 p->h.alloc(chunk * p->ax.h_state());
                 p->F2.alloc(chunk * p->ax.f2_state());
                 AxisRotArgs r{};
@@ -6225,8 +6311,19 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                                           tot_h[t] * sizeof(double), hipMemcpyDeviceToHost, s));
                 HCHECK(hipStreamSynchronize(s));
             }
-            istate = j;
-        }
+            return j;
+        };
+        for (int64_t istate = first; istate <= last;)
+            with_room(p->axis, p->small, [&] { istate = batch(istate); },
+                      [&] {
+                          HCHECK(hipStreamSynchronize(s));
+                          p->gq.release();
+                          p->h.release();
+                          p->F2.release();
+                          p->Y.release();
+                          p->rowmap.release();
+                          p->rowoff.release();
+                      });
         HCHECK(hipEventRecord(c->ev_d, s));
         HCHECK(hipEventSynchronize(c->ev_d));
         float ms = 0;

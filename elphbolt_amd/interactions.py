@@ -64,17 +64,27 @@ class _Form:
 
     _form = None  # name of the entry point
 
-    def form(self, pair=None, points=None):
-        """(pair stage axis by axis, sum at the IBZ points axis by axis), as runs take them; True or False
-        changes one of them for the runs that follow (ElphError if the plan does not have the form)."""
+    def _set_form(self, bits, on):
         f, now = getattr(self.lib, self._form), ct.c_int32(0)
         self.wann._check(f(self.plan, -1, ct.byref(now)), "plan form")
-        if pair is not None or points is not None:
-            want = (now.value & 1 if pair is None else int(pair)) | (now.value & 2 if points is None else 2 * int(points))
+        want = now.value
+        for bit, v in zip(bits, on):
+            if v is not None:
+                want = want | bit if v else want & ~bit
+        if want != now.value:
             st = f(self.plan, want, ct.byref(now))
             if st != 0:
                 raise ElphError(st, "plan form: the plan does not have it")
-        return bool(now.value & 1), bool(now.value & 2)
+        return tuple(bool(now.value & bit) for bit in bits)
+
+    def form(self, pair=None, points=None):
+        """(pair stage axis by axis, sum at the IBZ points axis by axis), as runs take them; True or False
+        changes one of them for the runs that follow (ElphError if the plan does not have the form)."""
+        return self._set_form((1, 2), (pair, points))
+
+    def small(self, on=None):
+        """Whether runs take small groups of IBZ points and little scratch; True or False changes it."""
+        return self._set_form((4,), (on,))[0]
 
 
 class IbzkPlan(_Form):

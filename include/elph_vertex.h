@@ -169,11 +169,14 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *plan, int64_t istate_first, int64
 /* No counterpart in the reference.  How the plan sums over the Wannier cells: axis by
  * axis of the mesh or as one product over all of them, for the pair stage
  * (ELPH_FORM_AXIS_PAIR) and for the sum over Re at the IBZ k (ELPH_FORM_AXIS_POINTS;
- * FP64 plans).  The plan chooses by its sizes when it is created; want >= 0 (the sum of
- * the forms to take) changes that for the runs that follow, ELPH_EINVAL if the plan
- * does not have the form.  form (may be NULL): what runs take now. */
+ * FP64 plans).  ELPH_FORM_SMALL: groups of 64 (FP64) or 128 IBZ points and little scratch
+ * instead of up to 3 GiB.  The plan chooses the first two by its sizes when it is created; want >= 0 (the
+ * sum of the forms to take) changes that for the runs that follow, ELPH_EINVAL if the plan
+ * does not have the form.  A run that finds no room on the device takes ELPH_FORM_SMALL, then
+ * the product, from then on.  form (may be NULL): what runs take now. */
 #define ELPH_FORM_AXIS_PAIR 1
 #define ELPH_FORM_AXIS_POINTS 2
+#define ELPH_FORM_SMALL 4
 int elph_ibzk_plan_form(elph_ibzk_plan *plan, int32_t want, int32_t *form);
 int elph_ibzk_plan_destroy(elph_ibzk_plan *plan);
 /* One-shot form (plan + run + destroy). */

@@ -198,6 +198,15 @@ def test_many_points_per_pass(kind):
         else:
             for t, n in enumerate(c):
                 assert np.array_equal(got[t, :n], g[t, :n])
+    # the form that a run takes when the device has no room for the large groups
+    assert plan.small(True) and plan.form() == (True, True)
+    few = w.device_buffer((nst, width))
+    c, _ = plan.run(1, nst, out=few)
+    assert np.array_equal(c, counts)
+    part = few.numpy()
+    for t in np.flatnonzero(c > 0):
+        assert np.array_equal(part[t, :c[t]], rows[t, :c[t]])
+    assert not plan.small(False)
 
 
 # kind, nb, nat, ws, mesh, bands in window, precision: the axis sums have 1/10, 1/2.2, 1/2.8 of the
