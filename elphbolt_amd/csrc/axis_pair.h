@@ -44,7 +44,9 @@ struct AxisTab {
     const unsigned short *pidx = nullptr;  // [2 rm + 1][2 r1m + 1] pair of (R0, R1), np if there is none
     const double2 *phA = nullptr;      // [N2][ncell] e^{i 2 pi q2 R2 / N2}
     const double2 *T0 = nullptr, *T1 = nullptr;  // e^{i 2 pi j / N0}, e^{i 2 pi j / N1}
-    int npl = 0, nl = 0;               // planes (one k2) and lines (one k1, k2) that hold rows
+    // planes (one k2) and lines (one k1, k2) that hold rows; a launch takes npl planes from pl0 on and
+    // their nl lines from l0 on, whose F2 it indexes from 0
+    int npl = 0, nl = 0, pl0 = 0, l0 = 0;
     const int *pl_k2 = nullptr;        // [npl]
     const int *line_of = nullptr;      // [npl][N1] line of k1, -1 if it holds no row
     const int *line_k = nullptr;       // [nl] k1 | plane << 16
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(256, MT * KS > 2 ? 1 : 3) void k_axis_ab(AxisTab x,
     const int nct = x.CPs >> 4, per = x.npl * nct;
     const int id = blockIdx.x, r8 = id >> 3, stl = r8 / per * 8 + (id & 7), sub = r8 % per;
     if (stl >= ns) return;
-    const int pl = sub / nct, ct = sub - pl * nct, st = st0 + stl;
+    const int pl = x.pl0 + sub / nct, ct = sub % nct, st = st0 + stl;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
     double2 *F1 = smem, *ph = smem + (x.np + 1) * 16;
@@ -225,8 +227,8 @@ __global__ __launch_bounds__(256, MT * KS > 2 ? 1 : 3) void k_axis_ab(AxisTab x,
         }
     }
     __syncthreads();
-    double2 *F2s = F2 + (size_t)stl * x.nl * (2 * x.rm + 1) * x.CPs + ct * 16 + li;
     const size_t lstride = (size_t)(2 * x.rm + 1) * x.CPs;
+    double2 *F2s = F2 + (size_t)stl * x.nl * lstride + ct * 16 + li;
     auto put = [](double2 *o, dv2 v) { __builtin_nontemporal_store(v, reinterpret_cast<dv2 *>(o)); };
     for (int R = wave; R <= x.rm; R += 4) {
         d4 ecr[MT], eci[MT], esr[MT], esi[MT], dcr[MT], dci[MT], dsr[MT], dsi[MT];
@@ -277,12 +279,12 @@ __global__ __launch_bounds__(256, MT * KS > 2 ? 1 : 3) void k_axis_ab(AxisTab x,
                 if (2 * q > x.N1) continue;
                 const int la = lineq[q], lb = q > 0 && 2 * q < x.N1 ? lineq[x.N1 - q] : -1;
                 if (la >= 0) {
-                    double2 *o = F2s + la * lstride;
+                    double2 *o = F2s + (la - x.l0) * lstride;
                     put(o + R * x.CPs, dv2{ecr[mt][r] + esr[mt][r], eci[mt][r] + esi[mt][r]});
                     if (R > 0) put(o + (x.rm + R) * x.CPs, dv2{dcr[mt][r] + dsr[mt][r], dci[mt][r] + dsi[mt][r]});
                 }
                 if (lb >= 0) {
-                    double2 *o = F2s + lb * lstride;
+                    double2 *o = F2s + (lb - x.l0) * lstride;
                     put(o + R * x.CPs, dv2{ecr[mt][r] - esr[mt][r], eci[mt][r] - esi[mt][r]});
                     if (R > 0) put(o + (x.rm + R) * x.CPs, dv2{dcr[mt][r] - dsr[mt][r], dci[mt][r] - dsi[mt][r]});
                 }
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
     if (s_lo >= s_hi) return;
     const int nb = a.nb, nbr = ULDS ? NBRM : a.nbr, N0 = x.N0;
     const int k0 = a.st_kint[3 * s_lo];
-    const int lk12 = x.line_k[line];
+    const int lk12 = x.line_k[x.l0 + line];
     int q1 = (lk12 & 0xffff) - a.st_kint[3 * s_lo + 1], q2 = x.pl_k2[lk12 >> 16] - a.st_kint[3 * s_lo + 2];
     q1 += q1 < 0 ? x.N1 : 0;
     q2 += q2 < 0 ? x.N2 : 0;
@@ -435,7 +437,7 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair(AxisTab x, AxisKArgs a, co
     }
     AxisC<MT, KS> sc;
     sc.init(x, lane);
-    const int it0 = x.line_item[line], nit = x.line_item[line + 1] - it0;
+    const int it0 = x.line_item[x.l0 + line], nit = x.line_item[x.l0 + line + 1] - it0;
     const size_t lsz = (size_t)(2 * x.rm + 1) * x.CPs, ssz = (size_t)x.nl * lsz;
     const double2 *F2l = F2 + (size_t)line * lsz;
     constexpr bool PF = !ULDS && NBRM <= 12;  // u of the next sp loaded ahead
@@ -637,7 +639,7 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
     sc.init(x, lane);
     const int *rowmap = a.rowmap + (size_t)qb * a.nwv;  // (one row set per q)
     const int64_t *rowoff = a.rowoff + (size_t)qb * a.nwv;
-    const int row0 = x.line_row[line], nrow = x.line_row[line + 1] - row0;
+    const int row0 = x.line_row[x.l0 + line], nrow = x.line_row[x.l0 + line + 1] - row0;
     int mine = 0;
     if (lane < nrow) {
         const int kp = rowmap[row0 + lane];

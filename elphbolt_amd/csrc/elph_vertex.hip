@@ -3771,12 +3771,23 @@ struct AxisPlan {
     bool on = false;
     AxisTab t;
     int tier = 0, ranks = 1, nbm = 8, vals = 0, nb = 0;  // kernel variant; results per rank
+    std::vector<int> pl_line;  // [planes + 1] first line of a plane
+    int most = 0;              // most lines of a plane
     DBuf<int> pe, ecell, pl_k2, line_of, line_k, line_row, line_item;
     DBuf<unsigned short> pidx;
     DBuf<int4> items;
     DBuf<double2> phA, T0, T1;
     int64_t h_state() const { return (int64_t)t.ncell * t.CPs; }                   // elements of h per state
-    int64_t f2_state() const { return (int64_t)t.nl * (2 * t.rm + 1) * t.CPs; }    // elements of F2 per state
+    int64_t f2_lines(int64_t n) const { return n * (2 * t.rm + 1) * t.CPs; }        // elements of F2 per state
+    // The launch over `n` planes from p0 on.
+    AxisTab planes(int p0, int n) const {
+        AxisTab c = t;
+        c.npl = std::min(n, t.npl - p0);
+        c.pl0 = p0;
+        c.l0 = pl_line[p0];
+        c.nl = pl_line[p0 + c.npl] - c.l0;
+        return c;
+    }
     size_t lds_ab() const { return axis_ab_lds(t.np, t.ncell, t.rm, t.r1m, t.N1); }
     size_t lds_c(bool items) const {  // 4 waves
         return 4 * (axis_wave_bytes(t.N0, axis_ystride(t.CT, nbm, nb), 64 * ranks * vals) +
@@ -3878,6 +3889,8 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
     const int64_t ne = (int64_t)order.size();
     // lines and planes of the rows; ascending mesh order is what makes a line's rows consecutive
     std::vector<int> pl_k2, line_k, line_row;
+    x.pl_line.clear();
+    x.most = 0;
     for (int64_t r = 0; r < nwv; ++r) {
         const int *k = &rows[3 * r];
         if (r > 0) {
@@ -3886,12 +3899,15 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
         }
         if (r == 0 || k[2] != k[-1]) pl_k2.push_back(k[2]);
         if (r == 0 || k[2] != k[-1] || k[1] != k[-2]) {
+            if (pl_k2.size() > x.pl_line.size()) x.pl_line.push_back((int)line_k.size());
             line_k.push_back(k[1] | (int)(pl_k2.size() - 1) << 16);
             line_row.push_back((int)r);
         }
     }
     line_row.push_back((int)nwv);
     const int64_t npl = (int64_t)pl_k2.size(), nl = (int64_t)line_k.size();
+    x.pl_line.push_back((int)nl);
+    for (int64_t p = 0; p < npl; ++p) x.most = std::max(x.most, x.pl_line[p + 1] - x.pl_line[p]);
     std::vector<int> line_of(npl * N[1], -1);
     for (int64_t l = 0; l < nl; ++l) line_of[(line_k[l] >> 16) * N[1] + (line_k[l] & 0xffff)] = (int)l;
     // column tiles: whole inner ranges, as many per 16 columns as fit
@@ -4007,28 +4023,51 @@ void with_room(bool &axis, bool &small, Go &&go, Free &&free_buffers) {
     }
 }
 
-// States per chunk of the axis path for nst states: h and F2 of a chunk within `cap`
-// bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
+// Chunks of the axis path for nst states: h of `states` states and F2 of `planes` planes of them within
+// `cap` bytes.  1 GiB: a launch over few states ends in a mostly empty last round of waves (pair stage
 // of 1786 states at 617 cells, 24^3: 15.0 / 10.6 / 10.2 / 10.1 / 9.9 ms at 64 MiB / 128 MiB /
 // 512 MiB / 1 GiB / 3 GB; 251 states of 16 bands, 15 branches on 20^3: 14.4 / 9.3 / 7.8 / 7.2 / 7.1).
+// `tight`, where the cap is a fraction of that: as many states as h has room for and the planes
+// that are left for F2, whose lines are many more than the states' cells.
 constexpr int64_t kAxisChunkBytes = (int64_t)1 << 30;
-int64_t axis_chunk(const AxisPlan &x, int64_t nst, int64_t cap) {
-    const int64_t per_state = (x.h_state() + x.f2_state()) * (int64_t)sizeof(double2);
-    return std::max<int64_t>(1, std::min<int64_t>(nst, cap / per_state));
+struct AxisSplit {
+    int64_t states;
+    int planes;
+};
+AxisSplit axis_split(const AxisPlan &x, int64_t nst, int64_t cap, bool tight) {
+    const int64_t el = cap / (int64_t)sizeof(double2), h = x.h_state(), full = h + x.f2_lines(x.t.nl), plane = x.f2_lines(x.most);
+    if (!tight || nst * full <= el) return {std::max<int64_t>(1, std::min(nst, el / full)), x.t.npl};
+    const int64_t states = std::max<int64_t>(1, std::min(nst, el / (h + plane)));
+    return {states, (int)std::max<int64_t>(1, std::min<int64_t>(x.t.npl, (el / states - h) / plane))};
+}
+// The chunks of nst states that buffers of h_n and f2_n elements hold (at least those that
+// axis_split gave when they were sized, for these or more states).
+AxisSplit axis_fit(const AxisPlan &x, int64_t nst, int64_t h_n, int64_t f2_n, bool tight) {
+    const int64_t all = std::min(h_n / x.h_state(), f2_n / x.f2_lines(x.t.nl)), plane = x.f2_lines(x.most);
+    if (all >= nst || (!tight && all > 0)) return {std::min(nst, all), x.t.npl};
+    const int64_t states = std::min({nst, h_n / x.h_state(), f2_n / plane});
+    if (states < 1) throw Error{ELPH_ENOMEM, "the axis sums' buffers hold no state"};
+    return {states, (int)std::min<int64_t>(x.t.npl, f2_n / (states * plane))};
+}
+int64_t axis_h_count(const AxisPlan &x, const AxisSplit &c) { return c.states * x.h_state(); }
+int64_t axis_f2_count(const AxisPlan &x, const AxisSplit &c) {
+    return c.states * x.f2_lines(c.planes < x.t.npl ? (int64_t)c.planes * x.most : x.t.nl);
 }
 
-// Rotation and stages A and B of the states s0 .. s0 + ns - 1, of the k (or q) kb0 .. kb1 - 1.
-void axis_front(const AxisPlan &x, const AxisRotArgs &r, const int *st_shift, int s0, int ns, int kb0, int kb1, double2 *F2,
-                hipStream_t s) {
-    const AxisTab &t = x.t;
-    const dim3 rg((unsigned)((t.ncell + 3) / 4), (unsigned)(kb1 - kb0));
-    auto rot = [&](auto kern) { hipLaunchKernelGGL(kern, rg, dim3(256), 0, s, t, r, s0, ns, kb0); };
+// Rotation of the states s0 .. s0 + ns - 1, of the k (or q) kb0 .. kb1 - 1.
+void axis_rot(const AxisPlan &x, const AxisRotArgs &r, int s0, int ns, int kb0, int kb1, hipStream_t s) {
+    const dim3 rg((unsigned)((x.t.ncell + 3) / 4), (unsigned)(kb1 - kb0));
+    auto rot = [&](auto kern) { hipLaunchKernelGGL(kern, rg, dim3(256), 0, s, x.t, r, s0, ns, kb0); };
     if (r.nrot <= 8) rot(k_axis_rot<8>);
     else if (r.nrot <= 16) rot(k_axis_rot<16>);
     else rot(k_axis_rot<32>);
+    HCHECK(hipGetLastError());
+}
+// Stages A and B of these states on the planes of t.
+void axis_ab(const AxisPlan &x, const AxisTab &t, const double2 *h, const int *st_shift, int s0, int ns, double2 *F2, hipStream_t s) {
     const int64_t per = (int64_t)t.npl * (t.CPs / 16);
     const dim3 ag((unsigned)((ns + 7) / 8 * 8 * per));
-    auto ab = [&](auto kern) { hipLaunchKernelGGL(kern, ag, dim3(256), x.lds_ab(), s, t, r.h, st_shift, s0, ns, F2); };
+    auto ab = [&](auto kern) { hipLaunchKernelGGL(kern, ag, dim3(256), x.lds_ab(), s, t, h, st_shift, s0, ns, F2); };
     if (t.N1 > 31) ab(k_axis_ab<2, 4>);
     else if (t.r1m > 7) ab(k_axis_ab<1, 4>);
     else ab(k_axis_ab<1, 2>);
@@ -4037,15 +4076,22 @@ void axis_front(const AxisPlan &x, const AxisRotArgs &r, const int *st_shift, in
 
 // Launch shape of the C kernels for nk k (or q) of up to nm states: workgroups of
 // four lines (a multiple of the XCDs, so that the same lines of every k share an L2),
-// times the ways a k's states are split where that leaves the device idle.
+// times the ways a k's states are split where that leaves the device idle: up to eight rounds of two
+// workgroups per CU, and where one round holds all lines, the split with the shortest sum of
+// rounds, a wave taking the time of about two states before its first (11 k of 4.3 states on 5
+// planes of 24^3: 62 us split by 5, 49 us not split).
 struct AxisGrid {
     int nblk, msplit;
 };
 AxisGrid axis_grid(const AxisTab &t, int64_t nk, int64_t nm, int64_t ncu) {
     AxisGrid g;
     g.nblk = (t.nl + 31) / 32 * 8;
-    const int64_t have = nk * ((t.nl + 3) / 4), want = 16 * std::max<int64_t>(ncu, 1);
-    g.msplit = (int)std::max<int64_t>(1, std::min<int64_t>(nm, want / have));
+    const int64_t have = nk * ((t.nl + 3) / 4), slots = 2 * std::max<int64_t>(ncu, 1);
+    g.msplit = (int)std::max<int64_t>(1, std::min<int64_t>(nm, 8 * slots / have));
+    if (have > slots) return g;
+    auto time = [&](int64_t m) { return (have * m + slots - 1) / slots * (2 + (nm + m - 1) / m); };
+    for (int m = g.msplit - 1; m > 0; --m)
+        if (time(m) <= time(g.msplit)) g.msplit = m;
     return g;
 }
 // Calls f(tiles of 16 q, K steps of 4 R0) with the forms of stage C the kernels have.
@@ -4389,7 +4435,7 @@ struct elph_ibzk_plan {
     TablePack tables;       // the groups' tables of the running call
     HostBuf tables_host;
     DBuf<double> wT, wfT;   // [q][s] 1 / (2 omega) in the units of |g|^2, 0 where omega is 0
-    int64_t y_bytes_cap = 0;  // general and axis paths: bytes of Y (or h and F2) per chunk of states (0: 512 MiB, axis kAxisChunkBytes)
+    int64_t y_bytes_cap = 0;  // general and axis paths: bytes of Y, or of h and F2, per chunk (0: 512 MiB, kAxisChunkBytes)
     int64_t CPf = 0;  // column count of the fused layout (16-rounded nb*nbr)
     ConsumerScratch cons;
 };
@@ -4422,16 +4468,16 @@ int64_t general_chunk(const elph_ibzk_plan *p, int64_t nst) {
     return std::max<int64_t>(1, std::min<int64_t>(nst, cap / per_state));
 }
 
-int64_t axis_chunk(const elph_ibzk_plan *p, int64_t nst) {
-    const int64_t most = p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes;
-    return axis_chunk(p->ax, nst, p->y_bytes_cap > 0 ? p->y_bytes_cap : most);
+AxisSplit axis_split(const elph_ibzk_plan *p, int64_t nst) {
+    if (p->y_bytes_cap > 0) return axis_split(p->ax, nst, p->y_bytes_cap, true);
+    return axis_split(p->ax, nst, p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes, p->small);
 }
 
-// Axis-by-axis path, a chunk of states at a time.
+// Axis-by-axis path, a chunk of states (and of planes, where scratch is tight) at a time.
 void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, IbzkScratch &sc, hipStream_t s) {
     const elph_ctx *c = p->ctx;
-    const int64_t chunk = axis_chunk(p, gr.nst);
-    const AxisTab &t = p->ax.t;
+    const AxisSplit split = axis_fit(p->ax, gr.nst, (int64_t)sc.h.n, (int64_t)sc.F2.n, p->y_bytes_cap > 0 || p->small);
+    const int64_t chunk = split.states;
     AxisRotArgs r{};
     r.g = sc.gk.p;
     r.g_kstride = p->nb * p->nb * p->nbr * c->nwsg;
@@ -4466,7 +4512,7 @@ void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, Ibzk
     K.out = a.out;
     K.nprocs = a.nprocs;
     // u_q in LDS where that leaves room for two workgroups per CU
-    const size_t lds_u = p->ax.lds_c(false) + 4 * axis_u_bytes(t.N0, (int)p->nbr);
+    const size_t lds_u = p->ax.lds_c(false) + 4 * axis_u_bytes(p->ax.t.N0, (int)p->nbr);
     const bool ulds = p->ax.tier == 0 && (p->nbr == 3 || p->nbr == 6) &&
                       lds_u <= std::min<size_t>(kAxisUldsMax, c->lds_max > 0 ? (size_t)c->lds_max : kAxisUldsMax);
     const size_t lds = ulds ? lds_u : p->ax.lds_c(false);
@@ -4474,29 +4520,33 @@ void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, Ibzk
         const int ns = (int)std::min(chunk, gr.nst - s0);
         int kb0, kb1;
         axis_range(gr.kst_host, s0, ns, kb0, kb1);
-        axis_front(p->ax, r, gr.st_kint.p, (int)s0, ns, kb0, kb1, sc.F2.p, s);
-        const AxisGrid g = axis_grid(t, kb1 - kb0, (ns + kb1 - kb0 - 1) / (kb1 - kb0), c->ncu);
-        const dim3 grid((unsigned)(g.nblk * g.msplit), (unsigned)(kb1 - kb0));
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, t, K, sc.F2.p, (int)s0, ns, kb0, g.nblk, g.msplit);
-        };
-        axis_form(t, [&](auto mt, auto ks) {
-            constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
-            if (ulds) {
-                if (p->nbr == 3) go(k_axis_pair<8, 3, 2, MT, KS, true, true>);
-                else go(k_axis_pair<8, 6, 2, MT, KS, true, true>);
-                return;
-            }
-            switch (p->ax.tier) {
-                case 0: go(k_axis_pair<8, 6, 2, MT, KS, true, false>); break;
-                case 1: go(k_axis_pair<8, 24, 1, MT, KS, true, false>); break;
-                case 2: go(k_axis_pair<12, 12, 1, MT, KS, true, false>); break;
-                case 3: go(k_axis_pair<16, 12, 1, MT, KS, true, false>); break;
-                case 4: go(k_axis_pair<16, 24, 1, MT, KS, true, false>); break;
-                default: go(k_axis_pair<32, 24, 1, MT, KS, false, false>); break;
-            }
-        });
-        HCHECK(hipGetLastError());
+        axis_rot(p->ax, r, (int)s0, ns, kb0, kb1, s);
+        for (int p0 = 0; p0 < p->ax.t.npl; p0 += split.planes) {
+            const AxisTab t = p->ax.planes(p0, split.planes);
+            axis_ab(p->ax, t, sc.h.p, gr.st_kint.p, (int)s0, ns, sc.F2.p, s);
+            const AxisGrid g = axis_grid(t, kb1 - kb0, (ns + kb1 - kb0 - 1) / (kb1 - kb0), c->ncu);
+            const dim3 grid((unsigned)(g.nblk * g.msplit), (unsigned)(kb1 - kb0));
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, t, K, sc.F2.p, (int)s0, ns, kb0, g.nblk, g.msplit);
+            };
+            axis_form(t, [&](auto mt, auto ks) {
+                constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+                if (ulds) {
+                    if (p->nbr == 3) go(k_axis_pair<8, 3, 2, MT, KS, true, true>);
+                    else go(k_axis_pair<8, 6, 2, MT, KS, true, true>);
+                    return;
+                }
+                switch (p->ax.tier) {
+                    case 0: go(k_axis_pair<8, 6, 2, MT, KS, true, false>); break;
+                    case 1: go(k_axis_pair<8, 24, 1, MT, KS, true, false>); break;
+                    case 2: go(k_axis_pair<12, 12, 1, MT, KS, true, false>); break;
+                    case 3: go(k_axis_pair<16, 12, 1, MT, KS, true, false>); break;
+                    case 4: go(k_axis_pair<16, 24, 1, MT, KS, true, false>); break;
+                    default: go(k_axis_pair<32, 24, 1, MT, KS, false, false>); break;
+                }
+            });
+            HCHECK(hipGetLastError());
+        }
     }
 }
 
@@ -4870,8 +4920,9 @@ void ibzk_scratch(const elph_ibzk_plan *p, IbzkScratch &sc, int64_t nkb, int64_t
     if (!p->axis_pts) get(sc.phiT, gk_phi_count(c));
     if (p->precision == ELPH_MIXED) get(sc.bphi, gk_bphi_count(c));
     if (p->axis) {
-        get(sc.h, axis_chunk(p, nst) * p->ax.h_state());
-        get(sc.F2, axis_chunk(p, nst) * p->ax.f2_state());
+        const AxisSplit c = axis_split(p, nst);
+        get(sc.h, axis_h_count(p->ax, c));
+        get(sc.F2, axis_f2_count(p->ax, c));
         return;
     }
     if (p->precision != ELPH_MIXED) get(sc.h, nst * p->Kp * p->CP);  // mixed: digits straight from gk
@@ -4887,10 +4938,9 @@ void ibzk_reserve(const elph_ibzk_plan *p, IbzkScratch &sc, int64_t nkb, int64_t
     ibzk_scratch(p, sc, nkb, nst, [](auto &buf, int64_t n) { buf.alloc((size_t)n); });
 }
 
-// Bytes of scratch and group tables for groups of up to nkb IBZ k and nst
-// states (each buffer rounded up to 256 bytes, as Carve places them).
-size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, bool with_y) {
-    size_t total = 0;
+// Bytes of scratch for groups of up to nkb IBZ k and nst states (each buffer rounded up
+// to 256 bytes, as Carve places them), on top of `total`.
+size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, bool with_y, size_t total) {
     auto add = [&total](auto &buf, int64_t n) {
         using T = std::remove_pointer_t<decltype(buf.p)>;
         total += ((std::max<int64_t>(n, 1) * sizeof(T)) + 255) & ~(size_t)255;
@@ -4900,7 +4950,6 @@ size_t ibzk_noalloc_bytes(const elph_ibzk_plan *p, int64_t nkb, int64_t nst, boo
         const void *b = &buf;
         if (with_y || (b != &probe.Y && !(p->axis && (b == &probe.h || b == &probe.F2)))) add(buf, n);
     });
-    total += ibzk_group_bytes(p, nkb, nst);
     return total;
 }
 
@@ -5277,7 +5326,6 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
     if (!p || !g2_device || !counts) return ELPH_EINVAL;
     elph_ctx *c = p->ctx;
     const int64_t y_cap = p->y_bytes_cap;
-    const bool axis = p->axis;
     try {
         HCHECK(hipSetDevice(c->device));
         if (first < 1 || last > p->nirr * p->nb || last < first - 1)
@@ -5285,25 +5333,27 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         if (!c->noalloc_scratch) throw Error{ELPH_EDEVICE, "no scratch array address for this device"};
         if (p->precision == ELPH_MIXED && !c->gdig.p) throw Error{ELPH_EINVAL, "gwann digits missing"};
         const size_t cap = kNoAllocScratchBytes;
-        // the largest group of IBZ k whose tables and scratch fit the array
-        // (a general-path plan also bounds its chunk of Y by what is left)
-        const int64_t nb = p->nb;
+        // the largest group of IBZ k whose tables and scratch fit the array (a general-path plan also
+        // bounds its chunk of Y by what is left; the axis form leaves three fifths of it for h and F2)
+        const int64_t nb = p->nb, nk = (last - first) / nb + 2;
+        // tables of all groups where they are small: one copy, and no wait between groups
+        auto tables_bytes = [&](int64_t nkb) {
+            const size_t one = ibzk_group_bytes(p, nkb, nkb * nb), all = one * ((nk + nkb - 1) / nkb);
+            return all <= (size_t)4 << 20 ? all : one;
+        };
         auto need = [&](int64_t nkb) {
+            const size_t tab = tables_bytes(nkb);
             if (p->general || p->axis) {
-                const size_t fixed = ibzk_noalloc_bytes(p, nkb, nkb * nb, false);
-                const int64_t per = (p->axis ? p->ax.h_state() + p->ax.f2_state() : p->nwv * p->CP) * (int64_t)sizeof(double2);
-                if (fixed + per + 512 > cap) return cap + 1;
-                p->y_bytes_cap = ((int64_t)(cap - fixed) - 512) / per * per;
+                const size_t fixed = ibzk_noalloc_bytes(p, nkb, nkb * nb, false, tab);
+                const int64_t per = (p->axis ? p->ax.h_state() + p->ax.f2_lines(p->ax.most) : p->nwv * p->CP) * (int64_t)sizeof(double2);
+                if (fixed + per + 512 > cap || (p->axis && nkb > 1 && fixed > cap / 5 * 2)) return cap + 1;
+                p->y_bytes_cap = (int64_t)(cap - fixed) - 512;
+                if (!p->axis) p->y_bytes_cap = p->y_bytes_cap / per * per;
             }
-            return ibzk_noalloc_bytes(p, nkb, nkb * nb, true);
+            return ibzk_noalloc_bytes(p, nkb, nkb * nb, true, tab);
         };
         int64_t KB = 64;
-        while (KB > 1 && need(KB) > cap) KB = (KB + 1) / 2;
-        if (need(KB) > cap && p->axis) {  // h and F2 of one state do not fit: the direct product
-            p->axis = false;
-            KB = 64;
-            while (KB > 1 && need(KB) > cap) KB = (KB + 1) / 2;
-        }
+        while (KB > 1 && need(KB) > cap) KB = p->axis && KB > 3 ? KB * 3 / 4 : (KB + 1) / 2;
         if (need(KB) > cap)
             throw Error{ELPH_ENOMEM, "one IBZ k of this material needs more than the " + std::to_string(cap >> 20) +
                                          " MiB scratch of the allocation-free entry point"};
@@ -5320,14 +5370,20 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         Carve cv{c->noalloc_scratch, cap};
         IbzkScratch sc;
         ibzk_scratch(p, sc, nkb, nst, [&cv](auto &buf, int64_t n) { cv.take(buf, (size_t)n); });
-        IbzkGroup g;
+        std::vector<IbzkGroup> groups(hosts.size());
         TablePack tables;
-        cv.take(tables.dev, ibzk_group_bytes(p, nkb, nst));
+        for (size_t i = 0; i < hosts.size(); ++i) ibzk_group_pack(p, hosts[i], groups[i], tables);
+        const bool once = ((cv.used + 255) & ~(size_t)255) + tables.used <= cap;
+        cv.take(tables.dev, once ? tables.used : ibzk_group_bytes(p, nkb, nst));
+        if (once && !hosts.empty()) tables.upload(s, nullptr);
+        else tables.clear();
         HCHECK(hipEventRecord(c->ev_c, s));
-        for (GroupHost &h : hosts) {
-            ibzk_group_pack(p, h, g, tables);
-            tables.upload(s, nullptr);  // stream-ordered after the previous group's kernels
-            ibzk_enqueue(p, g, sc, s, g2_device, true);
+        for (size_t i = 0; i < hosts.size(); ++i) {
+            if (!once) {
+                ibzk_group_pack(p, hosts[i], groups[i], tables);
+                tables.upload(s, nullptr);  // stream-ordered after the previous group's kernels
+            }
+            ibzk_enqueue(p, groups[i], sc, s, g2_device, true);
         }
         HCHECK(hipEventRecord(c->ev_d, s));
         HCHECK(hipEventSynchronize(c->ev_d));
@@ -5337,12 +5393,10 @@ int elph_ibzk_plan_run_noalloc(elph_ibzk_plan *p, int64_t first, int64_t last, i
         timing_flush(c);
     } catch (const Error &e) {
         p->y_bytes_cap = y_cap;
-        p->axis = axis;
         c->tev_used = 0;
         return ret_error(c, e);
     }
     p->y_bytes_cap = y_cap;
-    p->axis = axis;
     return ELPH_OK;
 }
 
@@ -6215,11 +6269,11 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
             a.Lmul = phase_lmul(p->L);
             const bool packed = p->L <= 255 && p->Nel[0] <= 255 && p->Nel[1] <= 255 && p->Nel[2] <= 255;
             auto axis = [&]() {
-                const AxisTab &t = p->ax.t;
-                const int64_t chunk =
-                    axis_chunk(p->ax, nst, p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes);
-                p->h.alloc(chunk * p->ax.h_state());
-                p->F2.alloc(chunk * p->ax.f2_state());
+                const AxisSplit split =
+                    axis_split(p->ax, nst, p->small ? std::min(kAxisChunkBytes, nst * p->Kp * p->CP * 8) : kAxisChunkBytes, p->small);
+                const int64_t chunk = split.states;
+                p->h.alloc(axis_h_count(p->ax, split));
+                p->F2.alloc(axis_f2_count(p->ax, split));  // (one split for all states of the call's batch)
                 AxisRotArgs r{};
                 r.g = p->gq.p;
                 r.g_kstride = gblk;
@@ -6236,23 +6290,27 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                     const int nc = (int)std::min(chunk, nst - t0);
                     int qb0, qb1;
                     axis_range(qst, t0, nc, qb0, qb1);
-                    axis_front(p->ax, r, nullptr, (int)t0, nc, qb0, qb1, p->F2.p, s);
-                    const AxisGrid ag = axis_grid(t, qb1 - qb0, (nc + qb1 - qb0 - 1) / (qb1 - qb0), c->ncu);
-                    const dim3 g((unsigned)(ag.nblk * ag.msplit), (unsigned)(qb1 - qb0));
-                    auto go = [&](auto kern) {
-                        hipLaunchKernelGGL(kern, g, dim3(256), p->ax.lds_c(true), s, t, a, p->F2.p, (int)t0, nc, qb0,
-                                           p->qst.p, ag.nblk, ag.msplit);
-                    };
-                    axis_form(t, [&](auto mt, auto ks) {
-                        constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
-                        switch (p->ax.tier) {
-                            case 0: go(k_axis_pair_q<8, 2, MT, KS>); break;
-                            case 1: go(k_axis_pair_q<12, 1, MT, KS>); break;
-                            case 2: go(k_axis_pair_q<16, 1, MT, KS>); break;
-                            default: go(k_axis_pair_q<32, 1, MT, KS>); break;
-                        }
-                    });
-                    HCHECK(hipGetLastError());
+                    axis_rot(p->ax, r, (int)t0, nc, qb0, qb1, s);
+                    for (int p0 = 0; p0 < p->ax.t.npl; p0 += split.planes) {
+                        const AxisTab t = p->ax.planes(p0, split.planes);
+                        axis_ab(p->ax, t, p->h.p, nullptr, (int)t0, nc, p->F2.p, s);
+                        const AxisGrid ag = axis_grid(t, qb1 - qb0, (nc + qb1 - qb0 - 1) / (qb1 - qb0), c->ncu);
+                        const dim3 g((unsigned)(ag.nblk * ag.msplit), (unsigned)(qb1 - qb0));
+                        auto go = [&](auto kern) {
+                            hipLaunchKernelGGL(kern, g, dim3(256), p->ax.lds_c(true), s, t, a, p->F2.p, (int)t0, nc, qb0,
+                                               p->qst.p, ag.nblk, ag.msplit);
+                        };
+                        axis_form(t, [&](auto mt, auto ks) {
+                            constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+                            switch (p->ax.tier) {
+                                case 0: go(k_axis_pair_q<8, 2, MT, KS>); break;
+                                case 1: go(k_axis_pair_q<12, 1, MT, KS>); break;
+                                case 2: go(k_axis_pair_q<16, 1, MT, KS>); break;
+                                default: go(k_axis_pair_q<32, 1, MT, KS>); break;
+                            }
+                        });
+                        HCHECK(hipGetLastError());
+                    }
                 }
             };
             auto launch = [&](auto pk) {
