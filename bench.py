@@ -478,7 +478,7 @@ def batched_bench(args, gen):
                      "vertices_per_s": vert / (np.mean(ms) * 1e-3), "wall_ms_one_replay": round(wall_ms, 2),
                      "prepare_s": round(t_prep, 2),
                      "tile_classes": [{"cols": c["cols"], "kp": c["kp"], "members": c["members"],
-                                       "path": "fused" if c["path"] == 0 else "column-tiled",
+                                       "path": ("fused", "column-tiled", "axis by axis")[c["path"]],
                                        "cb": c["cb"], "rb": c["rb"], "candidates": c["candidates"],
                                        "tuned_ms": round(c["ms"], 3)} for c in cls]}
         log(f"[bench] batched {prec}: {vert:.3e} vertices per step, {np.mean(ms):.1f} ms per graph replay, "

@@ -5488,7 +5488,6 @@ struct elph_batch {
         int cb = 0, kb = 0;  // size buckets of nb*nbr and Kp
         int64_t members = 0;
         elph_batch_class_t rep{};
-        bool axis = false;  // the first member takes the axis-by-axis form (no tile choice for the others)
     };
     int device = 0;
     std::vector<hipStream_t> streams;
@@ -5546,8 +5545,8 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
         for (int cb = 1; cb <= 4; ++cb)
             for (int rb = 1; rb <= 2; ++rb) cands.push_back({true, cb, rb});
     }
-    // the axis-by-axis form where the sizes take it: it is not timed against the
-    // direct product, whose operand preparation lies outside the pair stage
+    // the axis-by-axis form where the plan takes it: the plan's rule knows the operand's
+    // preparation, which lies outside the pair stage that is timed here
     if (p->axis) cands.assign(1, TileCand{false, 0, 0, true});
     if (!tune) cands.resize(1);
     const IbzkGroup &g = *it.groups.front();
@@ -5578,7 +5577,7 @@ elph_batch_class_t autotune(elph_batch *b, elph_batch::Item &it, hipStream_t st,
     elph_batch_class_t r{};
     r.precision = p->precision;
     if (bc.axis) {
-        r.path = p->general ? 1 : 0;
+        r.path = 2;
         r.cb = p->ax.t.CPs / 16;
         r.rb = 1;
     } else {
@@ -5602,11 +5601,12 @@ void batch_groups(elph_batch *b, elph_batch::Item &it, int64_t *counts) {
 // Size classes, streams and buffers of the batch's plans; allocates all that its graph needs.
 void batch_plan(elph_batch *b, bool autotune_tiles) {
     b->classes.clear();
-    // size classes: (precision, bucket of nb*nbr, bucket of Kp)
-    std::map<std::tuple<int, int, int>, int> key2cls;
+    // size classes: (precision, bucket of nb*nbr, bucket of Kp), the plans of the axis-by-axis form
+    // apart: they have no tile shape to choose
+    std::map<std::tuple<int, int, int, bool>, int> key2cls;
     for (auto &it : b->items) {
         if (it.groups.empty()) continue;
-        const auto key = std::make_tuple((int)it.p->precision, col_bucket(it.p->CPf), kp_bucket(it.p->Kp));
+        const auto key = std::make_tuple((int)it.p->precision, col_bucket(it.p->CPf), kp_bucket(it.p->Kp), it.p->axis);
         auto f = key2cls.find(key);
         if (f == key2cls.end()) {
             elph_batch::Class c;
@@ -5614,15 +5614,12 @@ void batch_plan(elph_batch *b, bool autotune_tiles) {
             c.cb = std::get<1>(key);
             c.kb = std::get<2>(key);
             c.rep = autotune(b, it, b->streams[0], autotune_tiles != 0);
-            c.axis = it.p->axis;
             key2cls[key] = (int)b->classes.size();
             b->classes.push_back(c);
             f = key2cls.find(key);
         } else {
-            // plans of the axis-by-axis form keep it; the others take the class's
-            // tile shape where one was timed, else the plan's own
             const elph_batch_class_t &r = b->classes[f->second].rep;
-            if (!it.p->axis && !b->classes[f->second].axis) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
+            if (r.path != 2) apply_cand(it.p, {r.path == 1, r.cb, r.rb});
         }
         it.cls = f->second;
         b->classes[f->second].members += 1;

@@ -385,8 +385,8 @@ int elph_last_timing(const elph_ctx *ctx, double out[3]);
  * ------------------------------------------------------------------------ */
 typedef struct elph_batch elph_batch;
 typedef struct {
-    int32_t precision, path;  /* path 0: up to the columns of the fused kernels, 1: beyond (column tiles) */
-    int32_t cb, rb;           /* column blocks of 16, row blocks of 16 per wave */
+    int32_t precision, path;  /* path 0: fused kernel, 1: general column-tiled, 2: axis by axis */
+    int32_t cb, rb;           /* column blocks of 16, row blocks of 16 per wave (path 2: 1) */
     int32_t candidates;       /* shapes timed */
     int64_t cols, kp;         /* nb*nbr and Kp of the class's tuning material */
     int64_t members;

@@ -209,6 +209,37 @@ def test_many_points_per_pass(kind):
     assert not plan.small(False)
 
 
+def test_batch_of_both_forms():
+    """Two plans of one size class, the first in this form: the other still has its tile shape timed, a
+    change of the point sum after a plan was added takes effect, and the replayed rows are the plans' own."""
+    mat = _material(4, 2, [5, 5, 5], [14, 12, 10], 2.0)
+    _, el, ph = _state(mat)
+    w = Wannier(mat)
+    plans = [interactions.IbzkPlan(w, el, ph) for _ in range(2)]
+    assert plans[0].form() == (True, True) and plans[1].form(pair=False) == (False, True)
+    b = interactions.Batch(nstreams=2)
+    last = 40 * mat.nb
+    outs = [b.add(p, 1, last) for p in plans]
+    plans[0].form(points=False)
+    b.prepare(autotune=True)
+    cls = {c["path"]: c for c in b.classes()}
+    print("batch of both forms", cls, flush=True)
+    assert len(cls) == 2 and cls[2]["members"] == 1 and cls[2]["candidates"] == 1
+    tiles = cls[0] if 0 in cls else cls[1]
+    assert tiles["members"] == 1 and tiles["candidates"] > 1
+    eager = []
+    for p, form in zip(plans, ((True, False), (False, True))):
+        assert p.form() == form
+        c, g = p.run(1, last)
+        eager.append(g[c >= 0])
+    for _ in range(2):
+        assert b.run() > 0
+        for (c, out), g in zip(outs, eager):
+            assert np.array_equal(out.numpy(), g)
+        w.synchronize()
+    b.close()
+
+
 # kind, nb, nat, ws, mesh, bands in window, precision: the axis sums have 1/10, 1/2.2, 1/2.8 of the
 # product's multiply-adds, and took longer on plans of these shapes (second tile of q; branches; short lines)
 SLOWER = [

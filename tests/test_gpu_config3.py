@@ -1,10 +1,11 @@
 """The batched workload's materials under oracle parity: draws of the
 multi-material generator at the benchmark's vertex cap (2 GB) and window
 (~4 bands), spanning its size range -- 16 bands x 15 branches (the most
-columns), 24 branches, 26 bands (column-tiled general path) and 857 WS cells
-(fused path).  Each plan runs first on its own (its default path), then all
-run together through one captured batch graph (elph_batch_*) with the tile
-shapes the autotuner picks.  The first two IBZ k of each material are
+columns), 24 branches, 26 bands and 857 WS cells with few columns.  Each
+plan runs first on its own, then all run together through one captured batch
+graph (elph_batch_*): in the form the plans choose (axis by axis or product), and
+as one product over all cells, where the autotuner picks the tile shapes (the
+first, second and fourth column-tiled, the third also fused).  The first two IBZ k of each material are
 checked against the oracle's calculate_eph_interaction_ibzk('g')
 (src/interactions.f90:2095-2400) over two k' windows of the row (its start
 and its middle): FP64 within 1e-12, mixed within 1e-5 relative above 1e-6 *
@@ -69,14 +70,17 @@ def _worst(rows, counts, refs, plan):
     return worst, len(pairs)
 
 
+@pytest.mark.parametrize("form", ["chosen", "product"])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_config3_batch_vs_oracle(batch_mats, precision):
+def test_config3_batch_vs_oracle(batch_mats, precision, form):
     tol = 1e-12 if precision == "fp64" else 1e-5
     b = interactions.Batch(nstreams=4)
     runs = []
     for m in batch_mats:
         plan = interactions.IbzkPlan(m["w"], m["el"], m["ph"], precision=precision)
-        # the plan on its own, default path (fused where nb*nbr fits)
+        if form == "product":
+            assert plan.form(False, False) == (False, False)
+        # the plan on its own (product: fused where nb*nbr fits)
         c1, g1 = plan.run(1, m["last"])
         worst, nblk = _worst(g1[c1 >= 0], c1, m["ref"], plan)
         print(f"  {m['mat'].name} alone: {nblk} blocks, max rel {worst:.2e}", flush=True)
@@ -88,7 +92,13 @@ def test_config3_batch_vs_oracle(batch_mats, precision):
     paths = {c["path"] for c in cls}
     print(f"config 3 {precision}: {len(cls)} size classes, paths {sorted(paths)}", flush=True)
     assert sum(c["members"] for c in cls) == len(batch_mats)
-    assert 1 in paths                # the column-tiled path is exercised
+    axis = [plan.form()[0] for _, plan, _, _ in runs]
+    assert sum(c["members"] for c in cls if c["path"] == 2) == sum(axis)
+    if form == "product":
+        assert 1 in paths            # the column-tiled path is exercised
+        assert not any(axis)
+    else:
+        assert precision == "mixed" or any(axis)  # the axis-by-axis form is exercised
     for rep in range(2):
         assert b.run() > 0
         for m, plan, counts, out in runs:
