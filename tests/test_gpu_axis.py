@@ -63,8 +63,10 @@ CASES = [
     ("n0_34", 4, 2, [5, 5, 5], [34, 6, 6], 2.0, None, "fp64"),
     ("n1_33", 4, 2, [4, 4, 4], [12, 33, 4], 2.0, None, "fp64"),
     ("n0_62_n1_61", 2, 1, [5, 5, 5], [62, 61, 2], 1.0, None, "fp64"),
-    ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None, "fp64"),
-    ("r1_beyond_7", 4, 1, [3, 15, 3], [13, 24, 8], 2.0, None, "fp64"),
+    ("r0_beyond_7", 4, 1, [24, 3, 3], [24, 10, 8], 2.0, None, "fp64"),
+    ("r1_beyond_7", 4, 1, [3, 24, 3], [13, 24, 8], 2.0, None, "fp64"),
+    ("n0_40_r0_beyond_7", 4, 1, [24, 3, 3], [40, 10, 8], 2.0, None, "fp64"),
+    ("n1_40_r1_beyond_7", 4, 1, [3, 24, 3], [13, 40, 8], 2.0, None, "fp64"),
     ("r2_long", 4, 1, [3, 3, 15], [12, 13, 24], 2.0, None, "fp64"),
 ]
 
@@ -72,6 +74,7 @@ CASES = [
 @pytest.mark.parametrize("name,nb,nat,ws,mesh,biw,polar,precision", CASES, ids=[c[0] for c in CASES])
 def test_ibzk_axis(name, nb, nat, ws, mesh, biw, polar, precision):
     mat = _material(nb, nat, ws, mesh, biw, polar)
+    _reaches(name, mat.rcells_q)
     o, el, ph = _state(mat)
     plan = interactions.IbzkPlan(Wannier(mat), el, ph, precision=precision)
     chosen = plan.form()
@@ -145,13 +148,21 @@ CASES_Q = [
     ("nb14_na1", 14, 1, [4, 4, 4], [12, 11, 9], 2.0, None),
     ("nb19_na1", 19, 1, [4, 4, 4], [24, 11, 8], 2.0, None),
     ("n0_35_n1_33", 4, 1, [5, 5, 5], [35, 33, 2], 1.5, None),
-    ("r0_beyond_7", 4, 1, [15, 3, 3], [24, 10, 8], 2.0, None),
+    ("r0_beyond_7", 4, 1, [24, 3, 3], [24, 10, 8], 2.0, None),
 ]
+
+
+def _reaches(name, cells):
+    """Cases named for cells beyond 7 along an axis have them (four K steps; k_axis_pts beyond 7 along R0)."""
+    for axis in (0, 1):
+        if f"r{axis}_beyond_7" in name:
+            assert np.abs(np.asarray(cells)[:, axis]).max() > 7
 
 
 @pytest.mark.parametrize("name,nb,nat,ws,mesh,biw,polar", CASES_Q, ids=[c[0] for c in CASES_Q])
 def test_ibzq_axis(name, nb, nat, ws, mesh, biw, polar):
     mat = _material(nb, nat, ws, mesh, biw, polar, seed=6)
+    _reaches(name, mat.rcells_k)
     o, el, ph = _state(mat)
     first = 3 * mat.nbr + 1  # past q = 0
     last = first + (mat.nbr if nb > 8 else 2 * mat.nbr) - 1
