@@ -1,6 +1,7 @@
 """The reference's own CPU-sized case (config 0: Si-like, 6^3 WS cells, 12^3
 mesh, window +-0.5 eV) as a parity case: every IBZ state's |g|^2 against the
-oracle (FP64 1e-12, mixed 1e-5, relative above 1e-6 * max; counts exact), and
+oracle (FP64 1e-12, mixed 1e-5, relative above 1e-6 * max; counts exact; in the form the
+plan chooses and, where that is axis by axis, as one product over all cells), and
 the transport-delta proxy over the whole chain -- g2 -> X+/- (tetrahedra) ->
 RTA rates -> field terms multiplied by the symmetrizers -> sigma, sigma*S and
 S symmetrized over the Cartesian operations -- against the oracle's chain
@@ -68,12 +69,16 @@ def cfg0():
     return dict(mat=mat, el=el, ph=ph, nst=nst, c_o=c_o, g_o=g_o, mu=mu, neq=neq, m=m, vels=vels, vol=vol, ref=ref)
 
 
-@pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_config0_g2_and_transport(cfg0, precision):
+# (mixed: the chosen form is the product)
+@pytest.mark.parametrize("precision,form", [("fp64", "chosen"), ("fp64", "product"), ("mixed", "chosen")])
+def test_config0_g2_and_transport(cfg0, precision, form):
     mat, el, ph, nst = cfg0["mat"], cfg0["el"], cfg0["ph"], cfg0["nst"]
-    print(f"config 0 {precision}", flush=True)
     w = Wannier(mat)
     plan = interactions.IbzkPlan(w, el, ph, precision=precision)
+    assert any(plan.form()) == (precision == "fp64")
+    if form == "product":
+        assert plan.form(False, False) == (False, False)
+    print(f"config 0 {precision}, form {plan.form()}", flush=True)
     g2d = DeviceBuffer(w, (nst, plan.nprocs))
     counts, _ = plan.run(1, nst, out=g2d)
     c_o, g_o = cfg0["c_o"], cfg0["g_o"]

@@ -8,7 +8,8 @@ calculate_eph_interaction_ibzk('g') (src/interactions.f90:2095-2400) runs it.
 * sampled states against the oracle: every in-window band of the first, a
   middle and the last IBZ k, over three k' windows of the 13824-long row
   (its start, middle and end), so the phase tables of every q = k' - k region
-  and the tail of the row are covered; FP64 within 1e-12 and mixed within
+  and the tail of the row are covered, in the form that the plan chooses (axis
+  by axis) and as one product over all cells; FP64 within 1e-12 and mixed within
   1e-5 relative on entries above 1e-6 * max|g|^2, counts and zeros exact;
 * the whole job (all 3304 IBZ states, 1786 in the window, 13824 k' each):
   mixed against FP64 within 1e-5 above 1e-6 * the global max, counts, row
@@ -75,11 +76,15 @@ def test_config1_setup_matches_oracle(cfg1):
     assert np.max(np.abs(ph.ens - ph_o.ens)) < 1e-10
 
 
+@pytest.mark.parametrize("form", ["chosen", "product"])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_config1_sampled_states_vs_oracle(cfg1, precision):
+def test_config1_sampled_states_vs_oracle(cfg1, precision, form):
     mat, el, ph, w = cfg1["mat"], cfg1["el"], cfg1["ph"], cfg1["w"]
     tol = 1e-12 if precision == "fp64" else 1e-5
     plan = interactions.IbzkPlan(w, el, ph, precision=precision)
+    assert plan.form() == (True, precision == "fp64")
+    if form == "product":
+        assert plan.form(False, False) == (False, False)
     nprocs = el.nstates_inwindow * mat.nbr
     assert plan.nprocs == nprocs
     pairs = []
@@ -102,16 +107,19 @@ def test_config1_sampled_states_vs_oracle(cfg1, precision):
         n += int(sel.sum())
         if sel.any():
             worst = max(worst, float(np.max(np.abs(got[sel] - r[sel]) / np.abs(r[sel]))))
-    _flush(f"config 1 {precision}: {len(pairs)} (state, k' window) blocks, {n} entries, max rel {worst:.2e}")
+    _flush(f"config 1 {precision} {form}: {len(pairs)} (state, k' window) blocks, {n} entries, max rel {worst:.2e}")
     assert worst < tol
 
 
-def test_config1_whole_job_mixed_vs_fp64(cfg1):
+@pytest.mark.parametrize("form", ["chosen", "product"])
+def test_config1_whole_job_mixed_vs_fp64(cfg1, form):
     """All IBZ states of the benchmark step, mixed against FP64 (both on the
-    device), in chunks of 64 IBZ k."""
+    device), in chunks of 64 IBZ k; `product`: mixed as the int8 product."""
     mat, el, ph, w = cfg1["mat"], cfg1["el"], cfg1["ph"], cfg1["w"]
     nb = mat.nb
     plans = {p: interactions.IbzkPlan(w, el, ph, precision=p) for p in ("fp64", "mixed")}
+    if form == "product":
+        assert plans["mixed"].form(pair=False) == (False, False)
     nprocs = plans["fp64"].nprocs
     nst = el.nwv_irred * nb
     chunk = 64 * nb
@@ -149,7 +157,7 @@ def test_config1_whole_job_mixed_vs_fp64(cfg1):
     for p in plans:
         bufs[p].free()
         plans[p].close()
-    _flush(f"config 1 whole job: {nact} in-window states, {nsel} entries above the floor, mixed vs FP64 max rel "
+    _flush(f"config 1 whole job {form}: {nact} in-window states, {nsel} entries above the floor, mixed vs FP64 max rel "
            f"{worst:.2e} (chunk medians <= {max(med):.2e})")
     assert nact == int(act_ref.sum()) == 1786
     assert worst < 1e-5
