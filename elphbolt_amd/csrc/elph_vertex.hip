@@ -4205,10 +4205,12 @@ void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n,
     x.on = true;
 }
 
-// Pinned host memory that a plan keeps for its calls.
+// Pinned host memory that a plan keeps for its calls, from the second one on: its allocation
+// takes longer than the first call saves by it.
 struct HostBuf {
     char *p = nullptr;
     size_t n = 0;
+    bool used = false;
     HostBuf() = default;
     HostBuf(const HostBuf &) = delete;
     HostBuf &operator=(const HostBuf &) = delete;
@@ -4256,6 +4258,10 @@ struct TablePack {
     // the copy may be in flight on return: the memory is the plan's, whose calls
     // all end with the stream drained.
     void upload(hipStream_t s, HostBuf *pinned) {
+        if (pinned && !pinned->used) {
+            pinned->used = true;
+            pinned = nullptr;
+        }
         std::vector<char> pageable(pinned ? 0 : used);
         char *h = pinned ? pinned->get(used) : pageable.data();
         for (const Part &x : parts)
