@@ -59,7 +59,7 @@ struct AxisTab {
     int CT = 16, spt = 1, CPs = 16;
 };
 
-constexpr int kAxisMaxCnt = 32;  // cells of one (R0, R1)
+constexpr int kAxisMaxCnt = 32;  // cells of one (R0, R1): one thread's chain in stage A (longer ones would run, not measured)
 constexpr int kAxisMaxR = 15;    // |R0|, |R1|
 constexpr int kAxisMaxN = 62;    // N0, N1
 
@@ -716,7 +716,8 @@ __global__ __launch_bounds__(256, 2) void k_axis_pair_q(AxisTab x, PairQArgs a, 
                     ++mp;
                     Yr += nb;
                 };
-                for (const int m1 = min(mp + x.spt, nb); mp < m1;) {
+                const int m1 = min(mp + x.spt, nb);
+                while (mp < m1) {
                     mac(0);
                     if (mp < m1) mac(1);
                     if (mp < m1) load_u(mp);

@@ -3741,6 +3741,75 @@ int elph_selftest_mfma(int device, double *max_err) {
 // ===========================================================================
 namespace {
 
+// Pinned host memory that a plan keeps for its calls, from the second one on: its allocation
+// takes longer than the first call saves by it.
+struct HostBuf {
+    char *p = nullptr;
+    size_t n = 0;
+    bool used = false;
+    HostBuf() = default;
+    HostBuf(const HostBuf &) = delete;
+    HostBuf &operator=(const HostBuf &) = delete;
+    ~HostBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    char *get(size_t count) {
+        if (count > n) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+            n = 0;
+            if (hipHostMalloc((void **)&p, count, hipHostMallocDefault) != hipSuccess) {
+                p = nullptr;
+                throw Error{ELPH_ENOMEM, "hipHostMalloc of " + std::to_string(count) + " bytes failed"};
+            }
+            n = count;
+        }
+        return p;
+    }
+};
+
+// The small host tables of a call, packed so that one buffer and one copy carry them
+// all: a buffer and a copy of its own for each of a dozen tables took 0.08 ms of a call
+// (one k, 24^3 mesh, mixed: 0.39 -> 0.32 ms; 48 k, 12^3 mesh: 0.53 -> 0.41).  The parts become
+// views of `dev` at 256-byte offsets.
+struct TablePack {
+    DBuf<char> dev;
+    struct Part { const void *src; size_t off, bytes; };
+    std::vector<Part> parts;
+    std::vector<std::function<void(char *)>> bind;
+    size_t used = 0;
+    static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 255) & ~(size_t)255; }
+    void clear() {
+        parts.clear();
+        bind.clear();
+        used = 0;
+    }
+    template <typename T> void add(const std::vector<T> &v, DBuf<T> &dst) {
+        const size_t off = used, n = v.size();
+        parts.push_back({v.data(), off, n * sizeof(T)});
+        bind.push_back([&dst, off, n](char *p) { dst.borrow((T *)(p + off), n); });
+        used += round(n * sizeof(T));
+    }
+    // Copies the parts, whose vectors are still there, and empties the list.  With `pinned`
+    // the copy may be in flight on return: the memory is the plan's, whose calls
+    // all end with the stream drained.
+    void upload(hipStream_t s, HostBuf *pinned) {
+        if (pinned && !pinned->used) {
+            pinned->used = true;
+            pinned = nullptr;
+        }
+        std::vector<char> pageable(pinned ? 0 : used);
+        char *h = pinned ? pinned->get(used) : pageable.data();
+        for (const Part &x : parts)
+            if (x.bytes) std::memcpy(h + x.off, x.src, x.bytes);
+        dev.alloc(used);
+        HCHECK(hipMemcpyAsync(dev.p, h, used, hipMemcpyHostToDevice, s));
+        if (!pinned) HCHECK(hipStreamSynchronize(s));
+        for (auto &b : bind) b(dev.p);
+        clear();
+    }
+};
+
 // Kernel variant of the axis-by-axis form: bounds on nb and nbr (registers of an
 // item's U_k' row and g), in-window ranks per item, time of a round's band products
 // (ps each, axis_time) and how many times the later stages take at N0 > 31, whose second tile
@@ -3773,6 +3842,7 @@ struct AxisPlan {
     int tier = 0, ranks = 1, nbm = 8, vals = 0, nb = 0;  // kernel variant; results per rank
     std::vector<int> pl_line;  // [planes + 1] first line of a plane
     int most = 0;              // most lines of a plane
+    TablePack tables;          // one buffer and copy for all of these
     DBuf<int> pe, ecell, pl_k2, line_of, line_k, line_row, line_item;
     DBuf<unsigned short> pidx;
     DBuf<int4> items;
@@ -3838,6 +3908,12 @@ int epilogue_class(int64_t nb, int64_t nbr) {
     if (nb <= 8 && nbr <= 6) return 1;
     if (nb <= 16 && nbr <= 12) return 2;
     return 0;
+}
+
+// e^{i 2 pi j / n}
+double2 axis_root(int64_t j, int64_t n) {
+    const double a = kTwoPi * (double)fmodulo(j, n) / (double)n;
+    return make_double2(std::cos(a), std::sin(a));
 }
 
 // Tables of the axis-by-axis form for `n` cells (column-major, leading dimension
@@ -3948,33 +4024,29 @@ void axis_build(AxisPlan &x, const int64_t *cells, int64_t ld, int64_t n, const 
         }
         line_item.push_back((int)items.size());
     }
-    auto root = [](int64_t j, int64_t m) {
-        const double a = kTwoPi * (double)fmodulo(j, m) / (double)m;
-        return make_double2(std::cos(a), std::sin(a));
-    };
     if (N[2] * ne > (int64_t)1 << 24) return;  // 256 MiB of phases
     std::vector<double2> phA(N[2] * ne, make_double2(0.0, 0.0)), T0(N[0]), T1(N[1]), T2(N[2]);
-    for (int64_t j = 0; j < N[0]; ++j) T0[j] = root(j, N[0]);
-    for (int64_t j = 0; j < N[1]; ++j) T1[j] = root(j, N[1]);
-    for (int64_t j = 0; j < N[2]; ++j) T2[j] = root(j, N[2]);
+    for (int64_t j = 0; j < N[0]; ++j) T0[j] = axis_root(j, N[0]);
+    for (int64_t j = 0; j < N[1]; ++j) T1[j] = axis_root(j, N[1]);
+    for (int64_t j = 0; j < N[2]; ++j) T2[j] = axis_root(j, N[2]);
     for (int64_t q = 0; q < N[2]; ++q)
         for (int64_t e = 0; e < ne; ++e)
             if (order[e] >= 0) phA[q * ne + e] = T2[fmodulo(q * R(order[e], 2), N[2])];
-    x.pe.upload(pe, s);
-    x.ecell.upload(order, s);
-    x.pidx.upload(pidx, s);
-    x.pl_k2.upload(pl_k2, s);
-    x.line_of.upload(line_of, s);
-    x.line_k.upload(line_k, s);
-    x.line_row.upload(line_row, s);
-    if (wband) {
-        x.line_item.upload(line_item, s);
-        x.items.upload(items, s);
-    }
-    x.phA.upload(phA, s);
-    x.T0.upload(T0, s);
-    x.T1.upload(T1, s);
-    HCHECK(hipStreamSynchronize(s));  // the host vectors may go out of scope
+    TablePack &tp = x.tables;
+    tp.clear();
+    tp.add(pe, x.pe);
+    tp.add(order, x.ecell);
+    tp.add(pidx, x.pidx);
+    tp.add(pl_k2, x.pl_k2);
+    tp.add(line_of, x.line_of);
+    tp.add(line_k, x.line_k);
+    tp.add(line_row, x.line_row);
+    tp.add(line_item, x.line_item);
+    tp.add(items, x.items);
+    tp.add(phA, x.phA);
+    tp.add(T0, x.T0);
+    tp.add(T1, x.T1);
+    tp.upload(s, nullptr);
     t.pe = x.pe.p;
     t.ecell = x.ecell.p;
     t.pidx = x.pidx.p;
@@ -4114,14 +4186,11 @@ struct AxisCells {
     int RM = 15;
     AxisCellTab t;
     std::vector<int> r2;  // the R2
+    TablePack tables;     // of these
     DBuf<int> pe, ent, poff;
     DBuf<double> dinv;
     DBuf<double2> T0, T1;
 };
-double2 axis_root(int64_t j, int64_t n) {
-    const double a = kTwoPi * (double)fmodulo(j, n) / (double)n;
-    return make_double2(std::cos(a), std::sin(a));
-}
 // Cells from which the mesh-point sum goes axis by axis.  Its cost per column tile (two barriers,
 // the line sums of few lines) does not shrink with the cells, and with 93 cells 37 of its 64 pair slots
 // work, while the product's one pass serves up to 64 k or 128 q: at 93 cells and up to 64 points the axis
@@ -4183,18 +4252,18 @@ void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n,
     t.rm = (int)rm;
     t.r1m = (int)r1m;
     t.r2n = (int)r2n;
-    DBuf<double2> *T[2] = {&x.T0, &x.T1};
-    for (int d = 0; d < 2; ++d) {
-        std::vector<double2> v(N[d]);
-        for (int64_t j = 0; j < N[d]; ++j) v[j] = axis_root(j, N[d]);
-        T[d]->upload(v, s);
-        HCHECK(hipStreamSynchronize(s));
-    }
-    x.pe.upload(pe, s);
-    x.ent.upload(ent, s);
-    x.dinv.upload(dinv, s);
-    x.poff.upload(poff, s);
-    HCHECK(hipStreamSynchronize(s));
+    std::vector<double2> T[2];
+    for (int d = 0; d < 2; ++d)
+        for (int64_t j = 0; j < N[d]; ++j) T[d].push_back(axis_root(j, N[d]));
+    TablePack &tp = x.tables;
+    tp.clear();
+    tp.add(T[0], x.T0);
+    tp.add(T[1], x.T1);
+    tp.add(pe, x.pe);
+    tp.add(ent, x.ent);
+    tp.add(dinv, x.dinv);
+    tp.add(poff, x.poff);
+    tp.upload(s, nullptr);
     t.pe = x.pe.p;
     t.ent = x.ent.p;
     t.dinv = x.dinv.p;
@@ -4204,75 +4273,6 @@ void axis_cells_build(AxisCells &x, const int64_t *cells, int64_t ld, int64_t n,
     x.r2 = r2;
     x.on = true;
 }
-
-// Pinned host memory that a plan keeps for its calls, from the second one on: its allocation
-// takes longer than the first call saves by it.
-struct HostBuf {
-    char *p = nullptr;
-    size_t n = 0;
-    bool used = false;
-    HostBuf() = default;
-    HostBuf(const HostBuf &) = delete;
-    HostBuf &operator=(const HostBuf &) = delete;
-    ~HostBuf() {
-        if (p) (void)hipHostFree(p);
-    }
-    char *get(size_t count) {
-        if (count > n) {
-            if (p) (void)hipHostFree(p);
-            p = nullptr;
-            n = 0;
-            if (hipHostMalloc((void **)&p, count, hipHostMallocDefault) != hipSuccess) {
-                p = nullptr;
-                throw Error{ELPH_ENOMEM, "hipHostMalloc of " + std::to_string(count) + " bytes failed"};
-            }
-            n = count;
-        }
-        return p;
-    }
-};
-
-// The small host tables of a call, packed so that one buffer and one copy carry them
-// all: a buffer and a copy of its own for each of a dozen tables took 0.08 ms of a call
-// (one k, 24^3 mesh, mixed: 0.39 -> 0.32 ms; 48 k, 12^3 mesh: 0.53 -> 0.41).  The parts become
-// views of `dev` at 256-byte offsets.
-struct TablePack {
-    DBuf<char> dev;
-    struct Part { const void *src; size_t off, bytes; };
-    std::vector<Part> parts;
-    std::vector<std::function<void(char *)>> bind;
-    size_t used = 0;
-    static size_t round(size_t n) { return (std::max<size_t>(n, 1) + 255) & ~(size_t)255; }
-    void clear() {
-        parts.clear();
-        bind.clear();
-        used = 0;
-    }
-    template <typename T> void add(const std::vector<T> &v, DBuf<T> &dst) {
-        const size_t off = used, n = v.size();
-        parts.push_back({v.data(), off, n * sizeof(T)});
-        bind.push_back([&dst, off, n](char *p) { dst.borrow((T *)(p + off), n); });
-        used += round(n * sizeof(T));
-    }
-    // Copies the parts, whose vectors are still there, and empties the list.  With `pinned`
-    // the copy may be in flight on return: the memory is the plan's, whose calls
-    // all end with the stream drained.
-    void upload(hipStream_t s, HostBuf *pinned) {
-        if (pinned && !pinned->used) {
-            pinned->used = true;
-            pinned = nullptr;
-        }
-        std::vector<char> pageable(pinned ? 0 : used);
-        char *h = pinned ? pinned->get(used) : pageable.data();
-        for (const Part &x : parts)
-            if (x.bytes) std::memcpy(h + x.off, x.src, x.bytes);
-        dev.alloc(used);
-        HCHECK(hipMemcpyAsync(dev.p, h, used, hipMemcpyHostToDevice, s));
-        if (!pinned) HCHECK(hipStreamSynchronize(s));
-        for (auto &b : bind) b(dev.p);
-        clear();
-    }
-};
 
 // A list of mesh points (integer triplets) by planes and lines, for k_axis_pts.
 struct AxisPtsHost {
@@ -4434,6 +4434,7 @@ struct elph_ibzk_plan {
     // says whether runs take it
     AxisPlan ax;
     bool axis = false;
+    TablePack utables;      // uT .. wfT
     DBuf<double2> uT, ufT;  // u, uf transposed: [q][sp][s]
     AxisCells kcells;       // axis-by-axis form of the Re sum (FP64 plans) where kcells.on; `axis_pts`
     bool axis_pts = false;  // says whether runs take it
@@ -5212,27 +5213,29 @@ int elph_ibzk_plan_create(elph_ctx *ctx, const elph_electrons *el, const elph_ph
                 (int64_t)axis_pts_lds(p->kcells, kPtsPlanes, 1024) > ctx->lds_max)
                 p->kcells.on = false;
             if (p->ax.on) {
-                auto transposed = [&](const std::vector<double2> &v, DBuf<double2> &dst) {
+                auto transposed = [&](const std::vector<double2> &v) {
                     std::vector<double2> w(v.size());
                     const int64_t b2 = nbr * nbr;
                     for (size_t q = 0; q < v.size() / b2; ++q)
                         for (int64_t sb = 0; sb < nbr; ++sb)
                             for (int64_t sp = 0; sp < nbr; ++sp) w[q * b2 + sp * nbr + sb] = v[q * b2 + sb * nbr + sp];
-                    dst.upload(w, s);
-                    HCHECK(hipStreamSynchronize(s));
+                    return w;
                 };
-                auto weights = [&](const std::vector<double> &v, DBuf<double> &dst) {
+                auto weights = [&](const std::vector<double> &v) {
                     std::vector<double> w(v.size());
                     for (size_t i = 0; i < v.size(); ++i) w[i] = v[i] != 0.0 ? 0.5 * kG2Unit / v[i] : 0.0;
-                    dst.upload(w, s);
-                    HCHECK(hipStreamSynchronize(s));
+                    return w;
                 };
-                transposed(u, p->uT);
-                weights(om, p->wT);
+                const std::vector<double2> uT = transposed(u), ufT = transposed(uf_host);
+                const std::vector<double> wT = weights(om), wfT = weights(omf_host);
+                TablePack &tp = p->utables;
+                tp.add(uT, p->uT);
+                tp.add(wT, p->wT);
                 if (mesh_ref > 1) {
-                    transposed(uf_host, p->ufT);
-                    weights(omf_host, p->wfT);
+                    tp.add(ufT, p->ufT);
+                    tp.add(wfT, p->wfT);
                 }
+                tp.upload(s, nullptr);
             }
         } catch (const Error &e) {
             if (e.code != ELPH_ENOMEM) throw;
