@@ -31,6 +31,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "|g|² vertices/sec, 1 MI355X, mixed vs FP64 at ≤1e-5 rel err; p50/p99 latency"
+FP64_PEAK_TFLOPS = 78.6
+INT8_PEAK_TOPS = 5000.0
 HBM_PEAK_GBS = 8000.0
 
 
@@ -358,16 +360,51 @@ def ibzq_bench(args, w, el, ph, mat):
         log(f"[bench] ibzq step {i}: {walls[-1] * 1e3:.1f} ms wall, pair kernels {tm['dominant_ms']:.1f} ms "
             f"in {tm['launches']} launches")
     vertices = int(counts.sum())
-    nbytes = axis_pair_bytes(mat.rcells_k, el, mat.nb, mat.nb) * nst + 8.0 * vertices
-    ach = nbytes / (np.mean(dom) * 1e-3) / 1e9
+    dom_s = float(np.mean(dom)) * 1e-3
+    if plan.form()[0]:
+        nbytes = axis_pair_bytes(mat.rcells_k, el, mat.nb, mat.nb) * nst + 8.0 * vertices
+        roof = roofline_of("hbm", nbytes / dom_s / 1e9, HBM_PEAK_GBS, "GB/s", "k_axis_rot + k_axis_ab + k_axis_pair_q")
+        roof["bytes_per_step"] = nbytes
+    else:
+        k2 = -(-pair_rows(mat.rcells_k) // 32) * 32    # cos/sin rows of the Re cell pairs, padded
+        flops = 4.0 * k2 * mat.nb ** 2 * el.nwv * nst   # real phase x complex h, per (state, k row)
+        roof = roofline_of("mfma", flops / dom_s / 1e12, FP64_PEAK_TFLOPS, "TFLOP/s",
+                           "k_pair_q_fp64" if mat.nb ** 2 <= 96 else "k_ibzq_y + k_ibzq_epi")
+        roof["flops_per_step"] = flops
+    roof["pair_ms_per_step"] = round(dom_s * 1e3, 2)
     out.free()
     plan.close()
     return {"workload": f"all {nst} IBZ phonon states (q, s), {el.nwv} k rows each, FP64",
             "vertices_per_step": vertices, "value": vertices / float(np.mean(walls)), "unit": "vertices/s",
-            "ms_per_step": round(float(np.mean(walls)) * 1e3, 2),
-            "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(ach / HBM_PEAK_GBS, 4), "kernel": "k_axis_ab + k_axis_pair_q",
-                         "pair_ms_per_step": round(float(np.mean(dom)), 2), "bytes_per_step": nbytes}}
+            "ms_per_step": round(float(np.mean(walls)) * 1e3, 2), "roofline": roof}
+
+
+def roofline_of(bound, achieved, peak, unit, kernel):
+    return {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": unit, "frac": round(achieved / peak, 4),
+            "kernel": kernel}
+
+
+def pair_roofline(plan, mixed, mat, el, res):
+    """Roofline of the ibzk pair stage by the form the plan takes: axis by axis the HBM bytes of the sums and
+    rows, as a product its int8 operations or FP64 flops."""
+    n, t, cols = res["states_per_launch"], res["avg_launch_s"], mat.nb * mat.nbr
+    k2 = pair_rows(mat.rcells_q[:mat.nwsg])
+    fl64 = algorithmic_flops(n, el.nwv, el.nstates_inwindow, mat.nb, mat.nbr, k2)
+    if plan.form()[0]:
+        nbytes = n * (axis_pair_bytes(mat.rcells_q, el, mat.nb, mat.nbr) + 8.0 * plan.nprocs)
+        r = roofline_of("hbm", nbytes / t / 1e9, HBM_PEAK_GBS, "GB/s", "k_axis_rot + k_axis_ab + k_axis_pair")
+        r["bytes_per_launch"] = nbytes
+    elif mixed:
+        ops = n * el.nwv * 10 * 2 * 2.0 * k2 * cols    # 10 digit products x (Re, Im) columns
+        r = roofline_of("mfma", ops / t / 1e12, INT8_PEAK_TOPS, "TOP/s", "k_pair_i8" if cols <= 64 else "k_ibzk_y_i8 + epilogue")
+        r["ops_per_launch"] = ops
+    else:
+        r = roofline_of("mfma", fl64 / t / 1e12, FP64_PEAK_TFLOPS, "TFLOP/s",
+                        "k_pair_fp64" if cols <= 96 else "k_ibzk_y_fp64 + epilogue")
+        r["flops_per_launch"] = fl64
+    r["avg_launch_ms"] = round(t * 1e3, 3)
+    r["product_equivalent_tflops"] = round(fl64 / t / 1e12, 2)
+    return r
 
 
 def axis_pair_bytes(cells, el, inner, outer):
@@ -621,25 +658,9 @@ def main():
            "zeros_match": exact_zero_match, "bound_met": bool(rel.max() <= 1e-5)}
     log(f"[bench] mixed vs fp64: max rel {err['max_rel']:.2e} median {err['median_rel']:.2e}")
 
-    k2 = pair_rows(mat.rcells_q[:mat.nwsg])
-    spl = res_mx["states_per_launch"]
-    out_bytes = 8.0 * nprocs
-    bytes_mx = spl * (axis_pair_bytes(mat.rcells_q, el, nb, nbr) + out_bytes)
-    ach_mx = bytes_mx / res_mx["avg_launch_s"] / 1e9
-    f64eq_mx = algorithmic_flops(spl, el.nwv, el.nstates_inwindow, nb, nbr, k2) / res_mx["avg_launch_s"] / 1e12
-    spl64 = res_64["states_per_launch"]
-    fl64 = algorithmic_flops(spl64, el.nwv, el.nstates_inwindow, nb, nbr, k2)
-    bytes_64 = spl64 * (axis_pair_bytes(mat.rcells_q, el, nb, nbr) + out_bytes)
-    ach64 = bytes_64 / res_64["avg_launch_s"] / 1e9
-    roofline = {"bound": "hbm", "achieved": round(ach_mx, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach_mx / HBM_PEAK_GBS, 4), "kernel": "k_axis_rot + k_axis_ab + k_axis_pair",
-                "avg_launch_ms": round(res_mx["avg_launch_s"] * 1e3, 3),
-                "bytes_per_launch": bytes_mx, "direct_product_equivalent_tflops": round(f64eq_mx, 2)}
+    roofline = pair_roofline(plans["mixed"], True, mat, el, res_mx)
     fp64 = {"value": res_64["value"], "ms_per_step": res_64["elapsed"] / args.steps * 1e3,
-            "roofline": {"bound": "hbm", "achieved": round(ach64, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(ach64 / HBM_PEAK_GBS, 4), "kernel": "k_axis_rot + k_axis_ab + k_axis_pair",
-                         "avg_launch_ms": round(res_64["avg_launch_s"] * 1e3, 3), "bytes_per_launch": bytes_64,
-                         "direct_product_equivalent_tflops": round(fl64 / res_64["avg_launch_s"] / 1e12, 2)}}
+            "roofline": pair_roofline(plans["fp64"], False, mat, el, res_64)}
     res = {"metric": METRIC, "value": res_mx["value"], "unit": "vertices/s", "n_gpus": 1, "steps": args.steps,
            "warmup": args.warmup, "ms_per_step": res_mx["elapsed"] / args.steps * 1e3, "higher_is_better": True,
            "scaling": "weak", "vs_baseline": None, "dtype": "int8+f64", "data": "synthetic",
