@@ -3821,9 +3821,9 @@ struct AxisTier {
 AxisTier axis_tier(int64_t nb, int64_t nbr) {
     if (nb <= 8 && nbr <= 6) return {0, 8, 2, 22.0, 4.0};
     if (nb <= 8 && nbr <= 24) return {1, 8, 1, 47.0, 4.0};
-    if (nb <= 12 && nbr <= 12) return {2, 12, 1, 51.0, 4.0};
+    if (nb <= 12 && nbr <= 12) return {2, 12, 1, 55.0, 4.0};
     if (nb <= 16 && nbr <= 12) return {3, 16, 1, 70.0, 4.0};
-    if (nb <= 16 && nbr <= 24) return {4, 16, 1, 67.0, 4.0};
+    if (nb <= 16 && nbr <= 24) return {4, 16, 1, 60.0, 4.0};
     if (nb <= 32 && nbr <= 24) return {5, 32, 1, 85.0, 4.0};
     return {};
 }
@@ -3873,9 +3873,11 @@ struct AxisPlan {
 // the epilogue outweighs the sums (17 bands, 9 branches, 14^3, 93 cells, mixed, 159 states: 1.71
 // against 2.11 ms); short lines leave lanes idle; and at 8 bands, 6 branches, 24^3 and 617 cells it takes
 // a sixth of the FP64 product's time.  The predicted ratio is off by 1.3 (one deviation, calls of 30
-// states and more), so the axis form has to promise 1.2: of the 1588, 7 are then more than 5% slower
+// states and more), so the axis form has to promise 1.2: of the 1588, 11 are then more than 5% slower
 // than with the products alone (worst 0.81, a call of 2 states), 105 (worst 0.51) when it was
 // taken at 1/2 (FP64) and 1/6 (mixed) of the multiply-adds, and the mean gain is 1.50 against 1.47.
+// 64 materials of 0.5e6 k-q pairs each in mixed precision take 208 ms by this rule, 198 with the better
+// form of each.
 constexpr double kAxisMargin = 1.2;
 // Stage A, then B and C by the elements of F2 and the epilogue by its products: `rounds` rounds of
 // 64 items with `work` band products per rank.
@@ -3894,8 +3896,8 @@ double direct_time(const DirectTime &k, int64_t rows, int64_t Kp, int64_t CP, do
 // (shape: epilogue_class)
 DirectTime direct_ibzk(bool mixed, bool general, int shape) {
     if (mixed) {
-        if (general) return {0.013, 14.5, 0.2};
-        return shape == 1 ? DirectTime{0.010, 4.8, 0.9} : (shape == 2 ? DirectTime{0.012, 0.0, 1.9} : DirectTime{0.018, 0.0, 5.1});
+        if (general) return {0.015, 16.0, 0.2};
+        return shape == 1 ? DirectTime{0.009, 4.1, 0.8} : (shape == 2 ? DirectTime{0.0095, 0.0, 1.5} : DirectTime{0.015, 0.0, 4.5});
     }
     if (general) return {0.084, 14.0, 0.0};
     return shape == 1 ? DirectTime{0.071, 5.0, 0.85} : (shape == 2 ? DirectTime{0.078, 8.2, 2.6} : DirectTime{0.05, 0.0, 6.0});
