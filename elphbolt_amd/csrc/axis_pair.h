@@ -19,8 +19,8 @@
 // and at -q C - S: real coefficients and half the q.
 // Measured with 617 cells on 24^3, 8 bands, 6 branches (1786 states, 13824 rows): pair stage
 // 53.0 ms per pass as one FP64 product (k_pair_fp64), 15.1 ms in int8 digits (k_pair_i8),
-// 8.1 ms in this form (C and epilogue 5.4, A and B 2.15, rotation 0.6); ibzq (2478 states) 106 ms
-// (k_pair_q_fp64) against 15.6 ms.  FP64 vector and matrix instructions share one pipe on this
+// 7.9 ms in this form (C and epilogue 5.2, A and B 2.1, rotation 0.6); ibzq (2478 states) 106 ms
+// (k_pair_q_fp64) against 15.4 ms.  FP64 vector and matrix instructions share one pipe on this
 // chip (their times add), so what is left is the epilogue's multiply-adds and its latency.
 
 // Scalar (wave-uniform) loads.

@@ -4331,7 +4331,7 @@ struct AxisPts {
     }
 };
 // Points of one k_axis_pts launch: their results within 2 GiB (one pass over gwann
-// serves them all), at most what the LDS list holds.
+// serves those of 8 planes), at most what the LDS list holds.
 int64_t axis_pts_max(int64_t bytes_per_point) {
     return std::max<int64_t>(64, std::min<int64_t>(1024, ((int64_t)2 << 30) / std::max<int64_t>(1, bytes_per_point)));
 }

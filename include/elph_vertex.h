@@ -377,7 +377,8 @@ int elph_last_timing(const elph_ctx *ctx, double out[3]);
  * |g|^2 rows written to g2_device (device memory, row stride = the plan's
  * nprocs; one row per in-window state, in istate order) and counts filled as
  * elph_ibzk_plan_run does (-1 for out-of-window states).  prepare() picks the
- * pair-stage tile shape of each size class (nb*nbr and Kp buckets) by timing
+ * pair-stage tile shape of each size class (nb*nbr and Kp buckets; plans that sum
+ * axis by axis have none and are classes of their own) by timing
  * the candidates on the class's first group when autotune != 0, assigns
  * plans to streams and captures the whole step into one hipGraph; run()
  * replays it (ms = device time of the replay).  Plans are tuned in place:
