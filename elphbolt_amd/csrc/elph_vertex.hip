@@ -4151,18 +4151,19 @@ void axis_ab(const AxisPlan &x, const AxisTab &t, const double2 *h, const int *s
 // Launch shape of the C kernels for nk k (or q) of up to nm states: workgroups of
 // four lines (a multiple of the XCDs, so that the same lines of every k share an L2),
 // times the ways a k's states are split where that leaves the device idle: up to eight rounds of two
-// workgroups per CU, and where one round holds all lines, the split with the shortest sum of
-// rounds, a wave taking the time of about two states before its first (11 k of 4.3 states on 5
-// planes of 24^3: 62 us split by 5, 49 us not split).
+// workgroups per CU.  With u_q in LDS (`staged`) a wave takes the time of about two states before its
+// first: where one round holds all lines, the split with the shortest sum of rounds (11 k of 4.3
+// states on 5 planes of 24^3: 62 us split by 5, 49 us not split; the kernels without that copy
+// gain from every split: 10 k of 4.7 states, 6 bands, 18 branches, 126 lines: 437 us not split, 319).
 struct AxisGrid {
     int nblk, msplit;
 };
-AxisGrid axis_grid(const AxisTab &t, int64_t nk, int64_t nm, int64_t ncu) {
+AxisGrid axis_grid(const AxisTab &t, int64_t nk, int64_t nm, int64_t ncu, bool staged) {
     AxisGrid g;
     g.nblk = (t.nl + 31) / 32 * 8;
     const int64_t have = nk * ((t.nl + 3) / 4), slots = 2 * std::max<int64_t>(ncu, 1);
     g.msplit = (int)std::max<int64_t>(1, std::min<int64_t>(nm, 8 * slots / have));
-    if (have > slots) return g;
+    if (!staged || have > slots) return g;
     auto time = [&](int64_t m) { return (have * m + slots - 1) / slots * (2 + (nm + m - 1) / m); };
     for (int m = g.msplit - 1; m > 0; --m)
         if (time(m) <= time(g.msplit)) g.msplit = m;
@@ -4533,7 +4534,7 @@ void axis_launch(elph_ibzk_plan *p, const IbzkGroup &gr, const PairArgs &a, Ibzk
         for (int p0 = 0; p0 < p->ax.t.npl; p0 += split.planes) {
             const AxisTab t = p->ax.planes(p0, split.planes);
             axis_ab(p->ax, t, sc.h.p, gr.st_kint.p, (int)s0, ns, sc.F2.p, s);
-            const AxisGrid g = axis_grid(t, kb1 - kb0, (ns + kb1 - kb0 - 1) / (kb1 - kb0), c->ncu);
+            const AxisGrid g = axis_grid(t, kb1 - kb0, (ns + kb1 - kb0 - 1) / (kb1 - kb0), c->ncu, ulds);
             const dim3 grid((unsigned)(g.nblk * g.msplit), (unsigned)(kb1 - kb0));
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, t, K, sc.F2.p, (int)s0, ns, kb0, g.nblk, g.msplit);
@@ -6302,7 +6303,7 @@ int elph_ibzq_plan_run(elph_ibzq_plan *p, int64_t first, int64_t last, int64_t *
                     for (int p0 = 0; p0 < p->ax.t.npl; p0 += split.planes) {
                         const AxisTab t = p->ax.planes(p0, split.planes);
                         axis_ab(p->ax, t, p->h.p, nullptr, (int)t0, nc, p->F2.p, s);
-                        const AxisGrid ag = axis_grid(t, qb1 - qb0, (nc + qb1 - qb0 - 1) / (qb1 - qb0), c->ncu);
+                        const AxisGrid ag = axis_grid(t, qb1 - qb0, (nc + qb1 - qb0 - 1) / (qb1 - qb0), c->ncu, false);
                         const dim3 g((unsigned)(ag.nblk * ag.msplit), (unsigned)(qb1 - qb0));
                         auto go = [&](auto kern) {
                             hipLaunchKernelGGL(kern, g, dim3(256), p->ax.lds_c(true), s, t, a, p->F2.p, (int)t0, nc, qb0,
